@@ -71,10 +71,11 @@ def listed():
         _image("ragged_dirty2ms", "dirty2ms", 1000003, 2310, 3125, 4.0, 1.4e9, 1e-5, "tracks",
                extent=4000.0, uvw32=True, weights=False),
         # full W-stacking, the benchmark's default workload, both directions
+        # (|w| up to 5000 wavelengths)
         _image("full_ms2dirty", "ms2dirty", 1 << 27, 8192, 8192, 3.0, 1.4e9, 1e-6, "tracks",
-               weights=False, shuffled=True),
+               weights=False, shuffled=True, extent=7660.0),
         _image("full_dirty2ms", "dirty2ms", 1 << 27, 8192, 8192, 3.0, 1.4e9, 1e-6, "tracks",
-               weights=False, shuffled=True),
+               weights=False, shuffled=True, extent=7660.0),
         # complex128 at eps 1e-12 on a wide field, 1e6 rows over the whole uv
         # plane: the high-accuracy workload of the method
         _image("double_ms2dirty", "ms2dirty", 1000000, 2048, 2048, 10.0, 1e9, 1e-12, "uniform",
@@ -297,13 +298,13 @@ def prepare(case, seed):
     g = _gen(seed)
     items = []
     for rows, n, freq in _batch_shapes(c):
-        # the full configuration's pixel size; baselines up to 5000
+        # the full configuration's pixel size; baselines up to 7660
         # wavelengths at 1.4 GHz
         vis = _complex(g, (rows,), False)
         img = torch.zeros(n, n, device="cuda", dtype=torch.complex64)
         if c["direction"] == "dirty2ms":
             img.real = torch.randn(n, n, generator=g, device="cuda")
-        items.append(dict(uvw=_tracks(g, rows, False) * (5000.0 * C_LIGHT / 1.4e9), vis=vis, wgt=None,
+        items.append(dict(uvw=_tracks(g, rows, False) * (7660.0 * C_LIGHT / 1.4e9), vis=vis, wgt=None,
                           dirty=img, fov=3.0 / 8192 * n, freq=freq))
     out = [it["dirty" if c["direction"] == "ms2dirty" else "vis"] for it in items]
     return dict(case=c, batch=_context().batch(c["direction"], items, c["eps"]), out=out)
@@ -382,7 +383,7 @@ def work(case):
         return {k: v * times for k, v in one.items()}
     total = {"bytes": 0.0, "flops": 0.0}
     for rows, n, freq in _batch_shapes(c):
-        p = _planes(dict(coverage="tracks", extent=5000.0 * freq / 1.4e9, nx=n, ny=n, fov=3.0 / 8192 * n, eps=c["eps"]))
+        p = _planes(dict(coverage="tracks", extent=7660.0 * freq / 1.4e9, nx=n, ny=n, fov=3.0 / 8192 * n, eps=c["eps"]))
         for k, v in _work(rows, rows, n, n, p, c["eps"], False, 24, False, 3).items():
             total[k] += v
     return total
