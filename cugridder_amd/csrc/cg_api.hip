@@ -252,7 +252,9 @@ template <typename T>
 static int grid_masks(Ctx &C, GridArgs &g, const uint8_t *mask, int nf1, int nf2)
 {
     if (mask && C.stop_after != 1 && fft_rows_masked<T>(nf1) && fft_spectrum_pruned<T>(nf2)) {
-        CG_TRY(ensure(C.tlist, sizeof(int32_t) * ((size_t)g.ntx * g.nty + 1)));
+        // W-stacking grids are gridded in 8 x 8 blocks, 2-D ones in sort tiles
+        const int64_t n = g.nf3 > 1 ? sparse_blocks(nf1, nf2) : (int64_t)g.ntx * g.nty;
+        CG_TRY(ensure(C.tlist, sizeof(int32_t) * (size_t)(n + 1)));
         g.rowmask = mask;
         g.colmask = mask + nf2;
         g.tile_list = as<int32_t>(C.tlist);
@@ -636,8 +638,12 @@ static int exec_ms2dirty(Ctx &C, const CallPlan &cp, const TU *uvw, const cx_t<T
             g.zn = zn;
             g.nchunk = (zn + t.pc - 1) / t.pc;
         }
-        CG_TRY(launch_grid<T>(as<geo_t<T>>(C.geo), as<cx_t<T>>(C.val), as<int32_t>(C.tstart),
-                              as<cx_t<T>>(C.grid), g, P.conv.kw, C.stream));
+        if (P.wstack)
+            CG_TRY(launch_grid_sparse<T>(as<geo_t<T>>(C.geo), as<cx_t<T>>(C.val), as<int32_t>(C.tstart),
+                                         as<cx_t<T>>(C.grid), g, P.conv.kw, C.stream));
+        else
+            CG_TRY(launch_grid<T>(as<geo_t<T>>(C.geo), as<cx_t<T>>(C.val), as<int32_t>(C.tstart),
+                                  as<cx_t<T>>(C.grid), g, P.conv.kw, C.stream));
         if (cp.dense_min > 0) {
             CG_TRY(ensure(C.dlist, sizeof(int32_t) * dense_list_ints(t.ntiles(), g.m)));
             CG_TRY(clk.mark(ST_COUNT + 1));

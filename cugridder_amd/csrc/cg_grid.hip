@@ -6,8 +6,9 @@
 // input-driven conv.cu:166-244), psi(d) = exp(beta sqrt(1 - c d^2)) for
 // |d| < kw/2 (conv.cu:32-36, unnormalised as in the reference).
 //
-// MI355X design: one workgroup owns a tx*ty tile of grid cells for a chunk of
-// w-planes and accumulates it in LDS (real parts, then imaginary parts, so
+// W-stacking grids: cg_sparse.hip, and for dense bins k_grid_dense2 below.
+// 2-D grids (one plane): one workgroup owns a tx*ty tile of grid cells and
+// accumulates it in LDS (real parts, then imaginary parts, so
 // the lanes' random cells spread over twice as many banks as interleaved
 // pairs would) with FP64 ds_add atomics (on gfx950 the
 // FP32 LDS atomic add runs ~20x slower than the FP64 one, and FP64 also makes
@@ -25,137 +26,9 @@
 #include <cstdlib>
 #include <type_traits>
 
-#include "cg_internal.hpp"
+#include "cg_kernel.hpp"
 
 namespace cg {
-
-__device__ __forceinline__ uint32_t geo_bits(float w) { return __float_as_uint(w); }
-__device__ __forceinline__ uint32_t geo_bits(double w) { return (uint32_t)__double_as_longlong(w); }
-
-__device__ __forceinline__ double es_val(double d, double beta, double c, double hw)
-{
-    return fabs(d) < hw ? exp(beta * sqrt(1.0 - c * d * d)) : 0.0;
-}
-
-// FP32 kernel values divided by e^beta (the MFMA gridders scale their sums
-// back once, the other FP32 kernels every value):
-//   psi(d) / e^beta = exp(beta (sqrt(1 - u) - 1) + y) = 2^(-beta log2(e) u / (1 + sqrt(1 - u)) + log2(e) y),
-// u = c d^2, y the learned kernel's polynomial in s = 2 u - 1 (0 for the ES
-// kernel).  The rewritten exponent has no cancellation near the centre, so
-// the hardware square root, reciprocal and exp2 (about ten instructions
-// instead of the library's correctly rounded expf and sqrtf) keep the large
-// central taps within a few ulp; only the taps near the support edge, whose
-// values are ~e^-beta of the centre, see errors up to ~beta * 1e-7.
-struct KernelEvalN {
-    float nb, ec, hw;
-    int learned;
-    const float *q;  // the launch argument's polynomial coefficients
-    __device__ __forceinline__ explicit KernelEvalN(const GridArgs &g, int kw)
-        : nb(g.f_nb), ec(g.f_ec), hw(0.5f * (float)kw), learned(g.learned), q(g.kq)
-    {
-    }
-    // LEARNED: -1 follows the launch's flag, 0 / 1 fix the kernel at compile
-    // time (no learned-polynomial code in the ES instantiations)
-    template <int LEARNED = -1>
-    __device__ __forceinline__ float at(float off0, int t) const
-    {
-        const float d = off0 + (float)t;
-        const float u = ec * d * d;
-        float y = nb * u * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_sqrtf(1.0f - u));
-        if (LEARNED == 1 || (LEARNED < 0 && learned)) {
-            const float s = 2.0f * u - 1.0f;
-            float p = q[LEARN_MAXDEG];
-#pragma unroll
-            for (int k = LEARN_MAXDEG - 1; k >= 0; k--) p = p * s + q[k];
-            y += 1.4426950408889634f * p;
-        }
-        const float v = __builtin_amdgcn_exp2f(y);
-        return fabsf(d) < hw ? v : 0.0f;
-    }
-    __device__ __forceinline__ float operator()(float off0, int t) const { return at(off0, t); }
-};
-
-// Kernel-value source of the complex64 MFMA kernels, fixed per
-// instantiation: the ES exp2 form or the per-tap polynomials (tp_on; KernelEvalN
-// also takes kKerLearned for the exact learned form).
-enum : int { kKerES = 0, kKerLearned = 1, kKerPoly = 2 };
-// the MFMA kernels are instantiated for the ES form and the polynomials: a
-// learned kernel always comes with its polynomials (grid_args), so a
-// learned launch without them is refused
-inline int ker_mode(const GridArgs &g) { return g.tp_on ? kKerPoly : g.learned ? -1 : kKerES; }
-
-// FP32 kernel values psi(off0 + t) / e^beta (the normalisation of
-// KernelEvalN) from per-tap polynomials in x = 2 off0 + kw - 1 (host fit,
-// tap_polynomials), coefficients in LDS; zero outside the taps.  Eleven FMAs
-// instead of the square root, reciprocal and exp2 of KernelEvalN, and the
-// same cost for the ES and the learned kernel.
-struct TapPolyN {
-    const float *tab;  // kw rows of kTapStride coefficients
-    int kw;
-    __device__ __forceinline__ float operator()(float off0, int t) const
-    {
-        if (t < 0 || t >= kw) return 0.f;
-        const float x = 2.f * off0 + (float)(kw - 1);
-        const float4 *c = reinterpret_cast<const float4 *>(tab + t * kTapStride);
-        const float4 c0 = c[0], c1 = c[1], c2 = c[2];
-        float p = c2.z;
-        p = p * x + c2.y;
-        p = p * x + c2.x;
-        p = p * x + c1.w;
-        p = p * x + c1.z;
-        p = p * x + c1.y;
-        p = p * x + c1.x;
-        p = p * x + c0.w;
-        p = p * x + c0.z;
-        p = p * x + c0.y;
-        p = p * x + c0.x;
-        return p;
-    }
-};
-
-// Kernel values of a point: the ES kernel exp(beta sqrt(1 - c d^2)) at the
-// tap offsets d, or the learned kernel, whose exponent adds the network's
-// polynomial sum_k q_k s^k in s = 2 c d^2 - 1 (c = (2/kw)^2).  The choice is
-// uniform across a launch and the coefficients are launch arguments, so
-// they stay in scalar registers.  FP64 evaluates the formula directly; FP32
-// is KernelEvalN times e^beta.
-template <typename T>
-struct KernelEval {
-    T beta, ec, hw;
-    int learned;
-    T q[LEARN_MAXDEG + 1];
-    __device__ __forceinline__ explicit KernelEval(const GridArgs &g, int kw)
-        : beta((T)g.beta), ec((T)g.es_c), hw((T)(0.5 * kw)), learned(g.learned)
-    {
-#pragma unroll
-        for (int k = 0; k <= LEARN_MAXDEG; k++) q[k] = (T)g.kq[k];
-    }
-    // value of tap t of a point whose first tap sits at offset off0
-    __device__ __forceinline__ T operator()(T off0, int t) const
-    {
-        const T d = off0 + (T)t;
-        if (!learned) return es_val(d, beta, ec, hw);
-        if (!(fabs(d) < hw)) return (T)0;
-        const T r = (T)1 - ec * d * d;
-        const T s = (T)1 - (T)2 * r;
-        T y = q[LEARN_MAXDEG];
-#pragma unroll
-        for (int k = LEARN_MAXDEG - 1; k >= 0; k--) y = y * s + q[k];
-        return exp(beta * sqrt(r) + y);
-    }
-};
-template <>
-struct KernelEval<float> : KernelEvalN {
-    float eb;  // e^beta
-    __device__ __forceinline__ explicit KernelEval(const GridArgs &g, int kw)
-        : KernelEvalN(g, kw), eb(g.f_e1)
-    {
-    }
-    __device__ __forceinline__ float operator()(float off0, int t) const
-    {
-        return KernelEvalN::operator()(off0, t) * eb;
-    }
-};
 
 // gridding accumulates in FP64 whatever the grid precision: 16 bytes per cell
 int grid_lds_bytes(const GridArgs &g, int) { return g.pc * g.tx * g.ty * 16; }
@@ -167,7 +40,7 @@ int degrid_lds_bytes(const GridArgs &g, int kw, int elem)
 
 // ------------------------------------------------------------ gridding
 
-// Footprint of a point relative to a tile (or plane chunk) [0, t) of an axis
+// Footprint of a point relative to a tile [0, t) of an axis
 // of length n, given its start r relative to the tile origin (in [0, n)):
 // first tap position s (negative when the footprint starts in an earlier
 // tile) and the taps [lo, hi) that land inside the tile.  With one tile
@@ -200,24 +73,19 @@ template <typename T, int KW>
 __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
                                                const cx_t<T> *__restrict__ val,
                                                const int32_t *__restrict__ tile_start,
-                                               cx_t<T> *__restrict__ fw, GridArgs g, int is2d)
+                                               cx_t<T> *__restrict__ fw, GridArgs g)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     double *acc = reinterpret_cast<double *>(smem_raw);
     __shared__ int s_beg[kMaxBins], s_cnt[kMaxBins], s_ox[kMaxBins], s_oy[kMaxBins];
     __shared__ int s_total;
-    // work item = (tile, plane chunk): one per workgroup, or, with a tile
-    // list (the tiles some FFT pass reads), the workgroups walk the list
-    const int nwork = g.tile_list ? g.tile_list[0] * g.nchunk : (int)gridDim.x;
+    // work item = a tile: one per workgroup, or, with a tile list (the tiles
+    // some FFT pass reads), the workgroups walk the list
+    const int nwork = g.tile_list ? g.tile_list[0] : (int)gridDim.x;
     for (int wi = blockIdx.x; wi < nwork; wi += gridDim.x) {
-    const int chunk = wi % g.nchunk;
-    const int tile = g.tile_list ? g.tile_list[1 + wi / g.nchunk] : wi / g.nchunk;
+    const int tile = g.tile_list ? g.tile_list[1 + wi] : wi;
     const int bx = tile % g.ntx, by = tile / g.ntx;
-    // planes [p0, p0 + np) of the slab [zb, zb + zn) held by the buffer
-    const int zn = slab_planes(g);
-    const int p0 = g.zb + chunk * g.pc;
-    const int np = min(g.pc, g.zb + zn - p0);
-    const int cells = np * g.ty * g.tx;
+    const int cells = g.ty * g.tx;
     for (int k = threadIdx.x; k < 2 * cells; k += blockDim.x) acc[k] = 0.0;
     // source bins whose footprints can reach this tile: bin (bx - sx, by - sy)
     const int nbins = g.sbx * g.sby;
@@ -234,8 +102,6 @@ __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
             const int sidx = sby_ * g.ntx + sbx_;
             s_beg[b] = tile_start[sidx];
             s_cnt[b] = tile_start[sidx + 1] - s_beg[b];
-            // dense bins are added afterwards by k_grid_dense
-            if (g.dense_min > 0 && s_cnt[b] >= g.dense_min) s_cnt[b] = 0;
             s_ox[b] = ox;
             s_oy[b] = oy;
             tot += s_cnt[b];
@@ -265,13 +131,6 @@ __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
         const Span X = tile_span<KW>(rx, g.tx, g.nf1);
         const Span Y = tile_span<KW>(ry, g.ty, g.nf2);
         if (X.lo >= X.hi || Y.lo >= Y.hi) continue;
-        Span Z{0, 0, 1};
-        if (!is2d) {
-            int rz = (int)(pk >> 16) - p0;
-            if (rz < 0) rz += g.nf3;
-            Z = tile_span<KW>(rz, np, g.nf3);
-            if (Z.lo >= Z.hi) continue;
-        }
         const cx_t<T> v = val[idx];
         T kx[KW], ky[KW];
 #pragma unroll
@@ -279,36 +138,27 @@ __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
             kx[t] = ker(G.x, t);
             ky[t] = ker(G.y, t);
         }
-        for (int tz = Z.lo; tz < Z.hi; tz++) {
-            int zz = Z.s + tz;
-            if (zz >= np) zz -= np;  // wraps only when one chunk holds every plane
-            const T kz = is2d ? (T)1 : ker(G.z, tz);
-            const T vzr = v.x * kz, vzi = v.y * kz;
 #pragma unroll
-            for (int t2 = 0; t2 < KW; t2++) {
-                if (t2 < Y.lo || t2 >= Y.hi) continue;
-                int yy = Y.s + t2;
-                if (yy >= g.nf2) yy -= g.nf2;  // wraps only with one tile along nf2
-                const T vyr = vzr * ky[t2], vyi = vzi * ky[t2];
-                double *row = acc + (zz * g.ty + yy) * g.tx;
+        for (int t2 = 0; t2 < KW; t2++) {
+            if (t2 < Y.lo || t2 >= Y.hi) continue;
+            int yy = Y.s + t2;
+            if (yy >= g.nf2) yy -= g.nf2;  // wraps only with one tile along nf2
+            const T vyr = v.x * ky[t2], vyi = v.y * ky[t2];
+            double *row = acc + yy * g.tx;
 #pragma unroll
-                for (int t1 = 0; t1 < KW; t1++) {
-                    if (t1 < X.lo || t1 >= X.hi) continue;
-                    int xx = X.s + t1;
-                    if (xx >= g.nf1) xx -= g.nf1;
-                    atomicAdd(row + xx, (double)(vyr * kx[t1]));
-                    atomicAdd(row + cells + xx, (double)(vyi * kx[t1]));
-                }
+            for (int t1 = 0; t1 < KW; t1++) {
+                if (t1 < X.lo || t1 >= X.hi) continue;
+                int xx = X.s + t1;
+                if (xx >= g.nf1) xx -= g.nf1;
+                atomicAdd(row + xx, (double)(vyr * kx[t1]));
+                atomicAdd(row + cells + xx, (double)(vyi * kx[t1]));
             }
         }
     }
     __syncthreads();
-    const int plane_cells = g.ty * g.tx;
     for (int k = threadIdx.x; k < cells; k += blockDim.x) {
-        int lz = k / plane_cells;
-        int rem = k - lz * plane_cells;
-        int y = rem / g.tx, x = rem - y * g.tx;
-        size_t gi = ((size_t)(p0 - g.zb + lz) * g.nf2 + (size_t)(by * g.ty + y)) * g.nf1 + bx * g.tx + x;
+        const int y = k / g.tx, x = k - y * g.tx;
+        const size_t gi = (size_t)(by * g.ty + y) * g.nf1 + bx * g.tx + x;
         fw[gi] = mkc((T)acc[k], (T)acc[cells + k]);
     }
     __syncthreads();  // acc and the bin table are reused by the next item
@@ -346,13 +196,6 @@ struct Queue2d {
     float vr[kQueue], vi[kQueue];   // strength
     int beg[4], cnt[4], ox[4], oy[4];  // source bins
 };
-
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 template <int KW>
 __global__ __launch_bounds__(64 * kQWaves) void k_grid2d_mfma(const float4 *__restrict__ geo,
@@ -531,11 +374,10 @@ template <typename T, int KW>
 static int grid_kw(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *ts, cx_t<T> *fw,
                    const GridArgs &g, hipStream_t s)
 {
-    if (g.sbx * g.sby > kMaxBins) return CG_ERR_SIZE;
-    int is2d = g.nf3 == 1 ? 1 : 0;
+    if (g.sbx * g.sby > kMaxBins || g.nf3 != 1 || g.nchunk != 1) return CG_ERR_SIZE;
     size_t lds = (size_t)grid_lds_bytes(g, (int)sizeof(cx_t<T>));
     const int64_t ntiles = (int64_t)g.ntx * g.nty;
-    unsigned nblk = (unsigned)(ntiles * g.nchunk);
+    unsigned nblk = (unsigned)ntiles;
     if (g.tile_list) {
         // build the list of tiles to write; workgroups then walk it
         hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, const_cast<int32_t *>(g.tile_list),
@@ -546,7 +388,7 @@ static int grid_kw(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *ts, c
         const int threads = grid_threads(lds);
         const int per_cu = std::max(1, std::min((int)(163840 / std::max<size_t>(lds, 1)),
                                                 2048 / threads));
-        nblk = (unsigned)std::min<int64_t>(ntiles * g.nchunk, (int64_t)256 * per_cu);
+        nblk = (unsigned)std::min<int64_t>(ntiles, (int64_t)256 * per_cu);
     }
     if constexpr (sizeof(T) == 4 && KW <= kQ2) {
         if (grid2d_mfma_supported(g, KW)) {
@@ -564,7 +406,7 @@ static int grid_kw(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *ts, c
         CG_HIP(hipFuncSetAttribute((const void *)k_grid<T, KW>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL((k_grid<T, KW>), dim3(nblk), dim3(grid_threads(lds)), lds, s, geo, val, ts,
-                       fw, g, is2d);
+                       fw, g);
     CG_HIP(hipGetLastError());
     return CG_OK;
 }

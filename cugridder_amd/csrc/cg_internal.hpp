@@ -178,6 +178,13 @@ struct GridArgs {
 // planes held by the grid buffer
 __host__ __device__ inline int slab_planes(const GridArgs &g) { return g.zn > 0 ? g.zn : g.nf3; }
 bool grid2d_mfma_supported(const GridArgs &g, int kw);
+// W-stacking (nf3 >= 2 kw planes; any sort tiles of at least two cells):
+// every bin below dense_min, in FP64 registers (cg_sparse.hip).  tile_list
+// needs sparse_blocks + 1 ints.
+int64_t sparse_blocks(int nf1, int nf2);
+template <typename T>
+int launch_grid_sparse(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *tile_start,
+                       cx_t<T> *fw, const GridArgs &g, int kw, hipStream_t s);
 template <typename T>
 int launch_grid(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *tile_start,
                 cx_t<T> *fw, const GridArgs &g, int kw, hipStream_t s);

@@ -1,0 +1,73 @@
+"""W-stacking gridding of bins with few points (k_grid_sparse): the w-planes
+against the FP64 restatement, where its 8 x 8 x 16-cell blocks meet the edges
+of the grid, of the sort tiles, of the planes and of the kernel widths.
+
+Tolerances: complex128 sums of FP64 products, kernel values exact to about
+beta (at most 37) roundings, stay within 1e-12; complex64 kernel values and
+products carry FP32 offsets and rounding, 3e-6 as the dense path's tests."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+from conftest import rel_l2, wst_case
+
+pytestmark = pytest.mark.gpu
+
+def spread_case(nrow, nx, ny, fov, wscale):
+    """wst_case with u and v over the whole grid (footprints wrap at its
+    edges) and |w| up to wscale / 2 wavelengths."""
+    k = wst_case(nrow, nx, ny, fov)
+    uvw = k["uvw"].copy()
+    uvw[:, 0] /= k["xpix"]
+    uvw[:, 1] /= k["ypix"]
+    uvw[:, 2] *= wscale
+    k["uvw"] = uvw
+    return k
+
+
+CASES = [
+    # nrow, nx, ny, fov, eps, tile: grid sides in cells are about 2 nx, 2 ny
+    (1, 16, 16, 5.0, 1e-5, 8),        # one point
+    (40, 16, 16, 10.0, 0.2, 8),       # kernel width 2, a grid of 4 x 4 blocks
+    (300, 25, 45, 10.0, 1e-4, 8),     # 50 x 90 cells: tiles of 2, partial blocks
+    (300, 30, 36, 20.0, 1e-6, 16),    # 60 x 72: tiles of 4 and 8
+    (500, 64, 64, 20.0, 1e-6, 32),    # blocks inside tiles of 32
+    (2000, 125, 64, 10.0, 1e-5, 16),  # 250 x 128
+    (3000, 512, 300, 3.0, 1e-5, 8),   # more than 2048 blocks: whole blocks per wave
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("single", [True, False])
+def test_sparse_gridding_vs_oracle(gpu, case, single):
+    torch = gpu
+    from cugridder_amd import Context
+    nrow, nx, ny, fov, eps, tile = case
+    k = spread_case(nrow, nx, ny, fov, 1000.0)
+    ctx = Context(stop_after=1, dense_min=0, tile_grid=tile)
+    cdt, rdt = (torch.complex64, torch.float32) if single else (torch.complex128, torch.float64)
+    ctx.ms2dirty(torch.tensor(k["uvw"], device="cuda"), torch.tensor(k["ms"], dtype=cdt, device="cuda"),
+                 torch.tensor(k["wgt"], dtype=rdt, device="cuda"), nx, ny, fov, k["f0"], eps)
+    got = ctx.grid_view(cdt).cpu().numpy()
+    ms = k["ms"].astype("c8" if single else "c16").astype("c16")
+    wgt = k["wgt"].astype("f4" if single else "f8").astype("f8")
+    ref = O.ms2dirty_grid(k["uvw"], k["f0"], ms, wgt, nx, ny, fov, eps, single=single)
+    assert rel_l2(got, ref) <= (3e-6 if single else 1e-12)
+
+
+@pytest.mark.parametrize("eps", [1e-12, 1e-14, 1.2e-16])
+def test_sparse_gridding_wide_kernels(gpu, eps):
+    """Kernel widths 13, 15 and 16 (complex128 only), several windows of
+    planes, a uv plane with crowded and empty blocks."""
+    torch = gpu
+    from cugridder_amd import Context
+    k = spread_case(800, 60, 50, 25.0, 500.0)
+    uvw = k["uvw"].copy()
+    uvw[:500, :2] *= 0.05
+    ctx = Context(stop_after=1)
+    ctx.ms2dirty(torch.tensor(uvw, device="cuda"), torch.tensor(k["ms"], device="cuda"),
+                 torch.tensor(k["wgt"], device="cuda"), 60, 50, 25.0, k["f0"], eps)
+    got = ctx.grid_view(torch.complex128).cpu().numpy()
+    ref = O.ms2dirty_grid(uvw, k["f0"], k["ms"], k["wgt"], 60, 50, 25.0, eps)
+    assert rel_l2(got, ref) <= 1e-12
