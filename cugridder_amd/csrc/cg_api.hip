@@ -731,6 +731,24 @@ static int plan_dirty2ms(Ctx &C, CallPlan &cp, int64_t nrow, int nchan, const do
     return cp.ier;
 }
 
+// Degridding tiles with fewer points than this are read straight from the
+// planes instead of staged in LDS.  With uniform points, 120 per 16 x 16 tile:
+// 2.86 against 3.49 ms per complex64 call (1024^2, eps 1e-5), 32 per tile 0.34
+// against 0.40 ms; 488 per tile 3.47 against 2.68 ms.  complex128 at eps 1e-12
+// with 15 per tile 50 against 165 ms, no difference at 256 to 512.  When the
+// tiles the points reach hold kDegridStagedFrom points on average, the few
+// sparse ones at the rim are not worth a launch (131072 Gaussian points, 360
+// per tile: 365 against 360 us).
+constexpr int kDegridDirectBelow = 256, kDegridStagedFrom = 128;
+
+static int degrid_direct_below(const WPlan &P, const Tiling &t, int64_t M)
+{
+    if (!P.wstack) return 1;
+    const int64_t rows = P.band_len > 0 ? P.band_len : P.nf2, cols = P.cband_len > 0 ? P.cband_len : P.nf1;
+    const int64_t tiles = ceil_div(rows, t.ty) * ceil_div(cols, t.tx);
+    return M < tiles * kDegridStagedFrom ? kDegridDirectBelow : 1;
+}
+
 template <typename T, typename TU, typename TW>
 static int exec_dirty2ms(Ctx &C, const CallPlan &cp, const TU *uvw, cx_t<T> *vis, const TW *wgt,
                          const cx_t<T> *dirty, StageClock &clk)
@@ -824,20 +842,30 @@ static int exec_dirty2ms(Ctx &C, const CallPlan &cp, const TU *uvw, cx_t<T> *vis
         g.dense_min = 0;
         if (sizeof(T) == 4 && M > 0 && C.degrid_dense_min > 0 && degrid_dense_supported(g, kw))
             g.dense_min = C.degrid_dense_min;
-        CG_TRY(ensure(C.dlist, sizeof(int32_t) * dense_list_ints(t.ntiles(), g.m)));
-        if (M > 0)
-            CG_TRY((launch_degrid<T, cx_t<T>>(as<geo_t<T>>(C.geo), as<cx_t<T>>(C.val),
-                                              as<int32_t>(C.vals), as<int32_t>(C.tstart),
-                                              as<cx_t<T>>(C.grid), vis, g, kw,
-                                              as<int32_t>(C.dlist), C.stream)));
-        if (g.dense_min > 0) {
-            CG_TRY(clk.mark(ST_COUNT + 1));
-            C.dense_timed = C.timing && !cp.slab;
-            CG_TRY(launch_degrid_dense((const float4 *)C.geo.p, (const float2 *)C.val.p,
-                                       as<int32_t>(C.vals), as<uint32_t>(C.keys),
-                                       as<int32_t>(C.tstart), as<int32_t>(C.dlist),
-                                       (const float2 *)C.grid.p, (float2 *)vis, g, kw, C.stream));
-            CG_TRY(clk.mark(ST_COUNT + 2));
+        if (M > 0) {
+            const int below = degrid_direct_below(P, t, M);
+            DegridLists L{};
+            CG_TRY(ensure(C.dlist, sizeof(int32_t) * degrid_list_ints(t.ntiles(), g.m, kw)));
+            CG_TRY(launch_degrid_lists(as<int32_t>(C.tstart), g, kw, below, as<int32_t>(C.dlist), L,
+                                       C.stream));
+            if (below > 1)
+                CG_TRY(launch_degrid_direct<T>(as<geo_t<T>>(C.geo), as<cx_t<T>>(C.val),
+                                               as<int32_t>(C.vals), as<int32_t>(C.tstart),
+                                               as<cx_t<T>>(C.grid), vis, g, kw, L, C.stream));
+            if (!(g.dense_min > 0 && g.dense_min <= below))
+                CG_TRY((launch_degrid<T, cx_t<T>>(as<geo_t<T>>(C.geo), as<cx_t<T>>(C.val),
+                                                  as<int32_t>(C.vals), as<int32_t>(C.tstart),
+                                                  as<cx_t<T>>(C.grid), vis, g, kw, L.staged,
+                                                  C.stream)));
+            if (g.dense_min > 0) {
+                CG_TRY(clk.mark(ST_COUNT + 1));
+                C.dense_timed = C.timing && !cp.slab;
+                CG_TRY(launch_degrid_dense((const float4 *)C.geo.p, (const float2 *)C.val.p,
+                                           as<int32_t>(C.vals), as<uint32_t>(C.keys),
+                                           as<int32_t>(C.tstart), L.dense, (const float2 *)C.grid.p,
+                                           (float2 *)vis, g, kw, C.stream));
+                CG_TRY(clk.mark(ST_COUNT + 2));
+            }
         }
     }
     CG_TRY(clk.mark(ST_COUNT));

@@ -453,8 +453,7 @@ int dense_chunk(int64_t m)
 
 int64_t dense_list_ints(int64_t ntiles, int64_t m)
 {
-    const int64_t units = ntiles + (m + dense_chunk(m) - 1) / dense_chunk(m);
-    return std::max<int64_t>(2 + 2 * units, ntiles + 2);  // also the sparse tiles' list
+    return 2 + 2 * (ntiles + (m + dense_chunk(m) - 1) / dense_chunk(m));
 }
 
 __global__ void k_zero_i32(int32_t *p, int64_t second)
@@ -930,17 +929,58 @@ int launch_grid(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *ts, cx_t
 
 // ------------------------------------------------------------ degridding
 
-// Tiles of the degridder's list: the non-empty ones below dense_min (all
-// non-empty ones when dense_min <= 0).  list[0] counts them, list[1..]
-// holds them (any order), list[ntiles + 1] is the work counter.
-__global__ __launch_bounds__(256) void k_sparse_tiles(const int32_t *__restrict__ tile_start,
-                                                      int64_t ntiles, int dense_min,
-                                                      int32_t *__restrict__ list)
+// The tiles of a W-stacking call by their point counts n, each list [count,
+// work counter, entries]: n >= dense_min (> 0) in units (tile, first point) of
+// at most `chunk` points for k_degrid_dense, else n < below in units of at
+// most `unit` points for k_degrid_direct, the others whole for k_degrid.
+__global__ __launch_bounds__(256) void k_tile_units(const int32_t *__restrict__ tile_start,
+                                                    int64_t ntiles, int below, int unit, int dense_min,
+                                                    int chunk, DegridLists L)
 {
     const int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x;
     if (t >= ntiles) return;
     const int n = tile_start[t + 1] - tile_start[t];
-    if (n > 0 && (dense_min <= 0 || n < dense_min)) list[1 + atomicAdd(list, 1)] = (int32_t)t;
+    if (n == 0) return;
+    auto units = [&](int32_t *list, int size) {
+        const int nu = (int)(((int64_t)n + size - 1) / size), e0 = atomicAdd(list, nu);
+        for (int u = 0; u < nu; u++) {
+            list[2 + 2 * (e0 + u)] = (int32_t)t;
+            list[3 + 2 * (e0 + u)] = u * size;
+        }
+    };
+    if (dense_min > 0 && n >= dense_min) units(L.dense, chunk);
+    else if (n < below) units(L.direct, unit);
+    else L.staged[2 + atomicAdd(L.staged, 1)] = (int32_t)t;
+}
+
+__global__ void k_zero_lists(DegridLists L)
+{
+    if (threadIdx.x < 2) L.direct[threadIdx.x] = L.staged[threadIdx.x] = L.dense[threadIdx.x] = 0;
+}
+
+static int64_t direct_units(int64_t ntiles, int64_t m, int kw)
+{
+    return std::min(ntiles, m) + m / degrid_direct_unit(kw);
+}
+
+int64_t degrid_list_ints(int64_t ntiles, int64_t m, int kw)
+{
+    return 2 + 2 * direct_units(ntiles, m, kw) + 2 + ntiles + dense_list_ints(ntiles, m);
+}
+
+int launch_degrid_lists(const int32_t *ts, const GridArgs &g, int kw, int below, int32_t *buf,
+                        DegridLists &L, hipStream_t s)
+{
+    const int64_t ntiles = (int64_t)g.ntx * g.nty;
+    L.max_direct = direct_units(ntiles, g.m, kw);
+    L.direct = buf;
+    L.staged = L.direct + 2 + 2 * L.max_direct;
+    L.dense = L.staged + 2 + ntiles;
+    hipLaunchKernelGGL(k_zero_lists, dim3(1), dim3(64), 0, s, L);
+    hipLaunchKernelGGL(k_tile_units, dim3((unsigned)ceil_div(ntiles, 256)), dim3(256), 0, s, ts, ntiles,
+                       below, degrid_direct_unit(kw), g.dense_min, dense_chunk(g.m), L);
+    CG_HIP(hipGetLastError());
+    return CG_OK;
 }
 
 template <typename T, int KW, int PPT>
@@ -956,7 +996,6 @@ __device__ __forceinline__ void degrid_tile(const geo_t<T> *__restrict__ geo,
     cx_t<T> *lds = reinterpret_cast<cx_t<T> *>(smem_raw);
     const int beg = tile_start[tile], end = tile_start[tile + 1];
     if (beg == end) return;
-    if (g.dense_min > 0 && end - beg >= g.dense_min) return;  // k_degrid_dense's
     const int bx = tile % g.ntx, by = tile / g.ntx;
     const int hx = g.tx + KW - 1, hy = g.ty + KW - 1;
     // LDS row stride: odd, so that cells a power-of-two number of rows or
@@ -1062,7 +1101,7 @@ __device__ __forceinline__ void degrid_tile(const geo_t<T> *__restrict__ geo,
 }
 
 // Dense bins of the degridder (complex64), the adjoint of k_grid_dense2.  A
-// workgroup takes work units as k_grid_dense2 does, stages the unit's tile
+// workgroup takes work units (k_tile_units) as k_grid_dense2 does, stages the unit's tile
 // plus the (kw-1) halo of every plane in LDS (as k_degrid does) and its
 // waves take pieces of quads (2 x 2 start cells; cells at kw = 8).  A piece
 // with at least kDegrid2Item points is ordered by w-window
@@ -1340,10 +1379,6 @@ static int degrid_dense_kw(const float4 *geo, const float2 *fac, const int32_t *
     const int64_t ntiles = (int64_t)g.ntx * g.nty;
     const int chunk = dense_chunk(g.m);
     const int64_t units = ntiles + ceil_div((int64_t)g.m, (int64_t)chunk);
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, list, 1);
-    hipLaunchKernelGGL(k_dense_bins, dim3((unsigned)ceil_div(ntiles, 256)), dim3(256), 0, s, ts,
-                       ntiles, g.dense_min, chunk, list);
-    CG_HIP(hipGetLastError());
     const size_t lds = (size_t)degrid_lds_bytes(g, KW, 8);
     const unsigned nblk = (unsigned)std::min<int64_t>(units, 256);
     // pieces: about one per wave of a full unit, at least 64 points (the
@@ -1377,7 +1412,7 @@ bool degrid_dense_supported(const GridArgs &g, int kw)
 }
 
 // One tile per workgroup (LISTED false: tile blockIdx.x), or a persistent
-// grid taking the tiles of list (k_sparse_tiles) one at a time.  Two
+// grid taking the tiles of list (k_tile_units) one at a time.  Two
 // instantiations, so the one-tile form keeps its scalar registers free of
 // the work counter's state.
 template <typename T, int KW, int PPT, bool LISTED>
@@ -1387,7 +1422,7 @@ __global__ __launch_bounds__(1024) void k_degrid(const geo_t<T> *__restrict__ ge
                                                 const int32_t *__restrict__ tile_start,
                                                 const cx_t<T> *__restrict__ fw,
                                                 cx_t<T> *__restrict__ out, GridArgs g, int is2d,
-                                                int32_t *__restrict__ list, int64_t ntiles)
+                                                int32_t *__restrict__ list)
 {
     if constexpr (!LISTED) {
         degrid_tile<T, KW, PPT>(geo, fac, perm, tile_start, fw, out, g, is2d, blockIdx.x);
@@ -1395,13 +1430,13 @@ __global__ __launch_bounds__(1024) void k_degrid(const geo_t<T> *__restrict__ ge
         __shared__ int s_tile;
         const int nlist = list[0];
         for (;;) {
-            if (threadIdx.x == 0) s_tile = atomicAdd(&list[ntiles + 1], 1);
+            if (threadIdx.x == 0) s_tile = atomicAdd(&list[1], 1);
             __syncthreads();
             const int li = s_tile;
             if (li >= nlist) break;
             // uniform across the workgroup: tile-derived addresses stay scalar
             degrid_tile<T, KW, PPT>(geo, fac, perm, tile_start, fw, out, g, is2d,
-                                    __builtin_amdgcn_readfirstlane(list[1 + li]));
+                                    __builtin_amdgcn_readfirstlane(list[2 + li]));
             __syncthreads();  // the staged planes and s_tile are reused
         }
     }
@@ -1433,10 +1468,6 @@ static int degrid_kw(const geo_t<T> *geo, const cx_t<T> *fac, const int32_t *per
     const int threads = grid_threads(lds);
     if (list) {
         // a persistent grid over the listed tiles: as many workgroups as fit
-        hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, list, ntiles + 1);
-        hipLaunchKernelGGL(k_sparse_tiles, dim3((unsigned)ceil_div(ntiles, 256)), dim3(256), 0, s,
-                           ts, ntiles, g.dense_min, list);
-        CG_HIP(hipGetLastError());
         const int per_cu = std::max(1, std::min((int)(163840 / std::max<size_t>(lds, 1)), 2048 / threads));
         nblk = (unsigned)std::min<int64_t>(ntiles, (int64_t)256 * per_cu);
     }
@@ -1444,7 +1475,7 @@ static int degrid_kw(const geo_t<T> *geo, const cx_t<T> *fac, const int32_t *per
         if (lds > 65536)
             CG_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         hipLaunchKernelGGL(kern, dim3(nblk), dim3(threads), lds, s, geo, fac, perm, ts, fw, out, g,
-                           is2d, list, ntiles);
+                           is2d, list);
         CG_HIP(hipGetLastError());
         return CG_OK;
     };

@@ -188,12 +188,29 @@ int launch_grid_sparse(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *t
 template <typename T>
 int launch_grid(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *tile_start,
                 cx_t<T> *fw, const GridArgs &g, int kw, hipStream_t s);
-// list (ntiles + 2 ints of scratch, or nullptr): run over the listed
-// non-empty tiles below g.dense_min instead of one workgroup per tile
+// list (DegridLists::staged, or nullptr): the listed tiles instead of one
+// workgroup per tile
 template <typename T, typename TV>
 int launch_degrid(const geo_t<T> *geo, const cx_t<T> *fac, const int32_t *perm,
                   const int32_t *tile_start, const cx_t<T> *fw, TV *out,
                   const GridArgs &g, int kw, int32_t *list, hipStream_t s);
+// The degridding tiles of a W-stacking call by point count: below `below`
+// points in units for launch_degrid_direct, then whole tiles for
+// launch_degrid, from g.dense_min points (> 0) units for
+// launch_degrid_dense.  buf needs degrid_list_ints ints.
+struct DegridLists {
+    int32_t *direct, *staged, *dense;
+    int64_t max_direct;
+};
+int degrid_direct_unit(int kw);
+int64_t degrid_list_ints(int64_t ntiles, int64_t m, int kw);
+int launch_degrid_lists(const int32_t *tile_start, const GridArgs &g, int kw, int below, int32_t *buf,
+                        DegridLists &L, hipStream_t s);
+// points read straight from the planes (cg_sparse.hip)
+template <typename T>
+int launch_degrid_direct(const geo_t<T> *geo, const cx_t<T> *fac, const int32_t *perm,
+                         const int32_t *tile_start, const cx_t<T> *fw, cx_t<T> *out,
+                         const GridArgs &g, int kw, const DegridLists &L, hipStream_t s);
 int grid_lds_bytes(const GridArgs &g, int elem);
 // Dense bins (fp32, kw <= 8, nf3 <= 32, cshift > 0): the sparse kernel
 // launched with g.dense_min > 0 leaves them out; this adds them to fw with
@@ -208,9 +225,8 @@ int launch_grid_dense(const geo_t<float> *geo, const cx_t<float> *val, const uin
                       int kw, hipStream_t s);
 int degrid_lds_bytes(const GridArgs &g, int kw, int elem);
 // Dense bins of the complex64 degridder (kw <= 8, nf3 <= 32, start cell in
-// the sort key, whole grid staged, no slabs): k_degrid launched with
-// g.dense_min > 0 leaves the bins with at least that many points to this
-// one, which interpolates them on MFMA.  list needs dense_list_ints ints.
+// the sort key, whole grid staged, no slabs), interpolated on MFMA: the
+// units of DegridLists::dense.
 bool degrid_dense_supported(const GridArgs &g, int kw);
 int launch_degrid_dense(const float4 *geo, const float2 *fac, const int32_t *perm,
                         const uint32_t *keys, const int32_t *tile_start, int32_t *list,

@@ -348,6 +348,139 @@ int launch_grid_sparse(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *t
     return CG_OK;
 }
 
+// ------------------------------------------------------------ degridding
+//
+// Tiles with few points: each point is interpolated straight from the planes
+// in HBM / L2, G lanes (8 or 16) per point, lane t holding tap t along the
+// fast axis, so a row of the footprint is one contiguous read of the group;
+// the KW rows of a plane are in flight together.  Staging such a tile in LDS
+// would read its whole halo, and one thread per point leaves most of a
+// workgroup idle.  A wave takes one unit (k_tile_units) at a time; units are
+// short, so that the last ones do not leave the GPU waiting.  Bound by the
+// plane reads where points are few: 10^6 rows at eps 1e-12 over 4096 x 4096 x
+// 194 complex128 cells (15 points per 16 x 16 tile) take 8 ms, staged 124 ms.
+constexpr int kDirWaves = 4;
+
+constexpr int direct_lanes(int kw) { return kw <= 8 ? 8 : 16; }
+constexpr int kDirSteps = 2;  // steps (64 / G points each) per unit
+int degrid_direct_unit(int kw) { return kDirSteps * (64 / direct_lanes(kw)); }
+
+template <typename T, int KW>
+__global__ __launch_bounds__(64 * kDirWaves) void k_degrid_direct(const geo_t<T> *__restrict__ geo,
+                                                                  const cx_t<T> *__restrict__ fac,
+                                                                  const int32_t *__restrict__ perm,
+                                                                  const int32_t *__restrict__ tile_start,
+                                                                  const cx_t<T> *__restrict__ fw,
+                                                                  cx_t<T> *__restrict__ out, GridArgs g,
+                                                                  const int32_t *__restrict__ list)
+{
+    constexpr int G = direct_lanes(KW), PW = 64 / G, UNIT = kDirSteps * PW;
+    // planes in flight: all of a narrow complex64 footprint
+    constexpr int UZ = sizeof(T) == 4 && KW <= 8 ? KW : 1;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int gl = lane & (G - 1);
+    const KernelEval<T> ker(g, KW);
+    const int zn = slab_planes(g);
+    const size_t plane = (size_t)g.nf1 * g.nf2;
+    const int xcd = blockIdx.x & 7, nunit = list[0];
+    // units dealt to the XCDs in contiguous runs, as in k_grid_sparse
+    for (int64_t j = blockIdx.x >> 3;; j += gridDim.x >> 3) {
+        const int64_t e = ((j / kSpRun * 8 + xcd) * kSpRun + j % kSpRun) * kDirWaves + wave;
+        if (e >= nunit) break;  // e grows with j; the waves share no barrier
+        const int tile = list[2 + 2 * e];
+        const int beg = tile_start[tile] + list[3 + 2 * e], end = min(tile_start[tile + 1], beg + UNIT);
+        const int by = tile / g.ntx, bx = tile - by * g.ntx;
+        for (int i0 = beg; i0 < end; i0 += PW) {
+            const int i = i0 + lane / G;
+            const bool ok = i < end;
+            const geo_t<T> R = geo[ok ? i : i0];
+            const uint32_t pk = geo_bits(R.w);
+            const T kx = gl < KW ? ker(R.x, gl) : (T)0;
+            const T kyl = gl < KW ? ker(R.y, gl) : (T)0;
+            const T kzl = gl < KW ? ker(R.z, gl) : (T)0;
+            int x = bx * g.tx + (int)(pk & 0xffu) + gl;
+            if (x >= g.nf1) x -= g.nf1;
+            const int y0 = by * g.ty + (int)((pk >> 8) & 0xffu);
+            T ky[KW];
+            int off[KW];
+#pragma unroll
+            for (int t = 0; t < KW; t++) {
+                ky[t] = __shfl(kyl, t, G);
+                int y = y0 + t;
+                if (y >= g.nf2) y -= g.nf2;
+                off[t] = y * g.nf1 + x;
+            }
+            const bool rd = ok && gl < KW;
+            T ar = 0, ai = 0;
+            int p = (int)(pk >> 16) - g.zb;  // plane in the buffer
+#pragma unroll UZ
+            for (int tz = 0; tz < KW; tz++, p++) {
+                if (p + g.zb >= g.nf3) p -= g.nf3;
+                const T kz = __shfl(kzl, tz, G);
+                T sr = 0, si = 0;
+                if (rd && p >= 0 && p < zn) {
+                    const cx_t<T> *src = fw + (size_t)p * plane;
+                    cx_t<T> f[KW];
+#pragma unroll
+                    for (int t = 0; t < KW; t++) f[t] = src[off[t]];
+#pragma unroll
+                    for (int t = 0; t < KW; t++) {
+                        sr += f[t].x * ky[t];
+                        si += f[t].y * ky[t];
+                    }
+                }
+                ar += sr * kz;
+                ai += si * kz;
+            }
+            ar *= kx;
+            ai *= kx;
+#pragma unroll
+            for (int d = 1; d < G; d <<= 1) {
+                ar += __shfl_xor(ar, d);
+                ai += __shfl_xor(ai, d);
+            }
+            if (ok && gl == 0) {
+                const cx_t<T> f = fac[i];
+                const int dst = perm[i];
+                if (dst >= 0 && dst < g.m) {  // a valid permutation always passes
+                    cx_t<T> v = mkc(ar * f.x - ai * f.y, ar * f.y + ai * f.x);
+                    if (g.accumulate) {
+                        const cx_t<T> prev = out[dst];
+                        v.x += prev.x;
+                        v.y += prev.y;
+                    }
+                    out[dst] = v;
+                }
+            }
+        }
+    }
+}
+
+template <typename T>
+int launch_degrid_direct(const geo_t<T> *geo, const cx_t<T> *fac, const int32_t *perm,
+                         const int32_t *ts, const cx_t<T> *fw, cx_t<T> *out, const GridArgs &g, int kw,
+                         const DegridLists &L, hipStream_t s)
+{
+    if (g.nf1 < 2 * kw || g.nf2 < 2 * kw || g.nf3 < 2 * kw) return CG_ERR_ARG;
+    const int64_t wgs = ceil_div(L.max_direct, kDirWaves);
+    const unsigned grid = (unsigned)std::min<int64_t>(ceil_div(wgs, 8) * 8, 256 * 8);
+    switch (kw) {
+#define CG_CASE(K)                                                                                   \
+    case K:                                                                                          \
+        hipLaunchKernelGGL((k_degrid_direct<T, K>), dim3(grid), dim3(64 * kDirWaves), 0, s, geo, fac, \
+                           perm, ts, fw, out, g, L.direct);                                         \
+        break;
+        CG_CASE(2) CG_CASE(3) CG_CASE(4) CG_CASE(5) CG_CASE(6) CG_CASE(7) CG_CASE(8) CG_CASE(9)
+        CG_CASE(10) CG_CASE(11) CG_CASE(12) CG_CASE(13) CG_CASE(14) CG_CASE(15) CG_CASE(16)
+#undef CG_CASE
+    default: return CG_ERR_ARG;
+    }
+    CG_HIP(hipGetLastError());
+    return CG_OK;
+}
+
+template int launch_degrid_direct<float>(const float4 *, const float2 *, const int32_t *, const int32_t *, const float2 *, float2 *, const GridArgs &, int, const DegridLists &, hipStream_t);
+template int launch_degrid_direct<double>(const double4 *, const double2 *, const int32_t *, const int32_t *, const double2 *, double2 *, const GridArgs &, int, const DegridLists &, hipStream_t);
 template int launch_grid_sparse<float>(const float4 *, const float2 *, const int32_t *, float2 *, const GridArgs &, int, hipStream_t);
 template int launch_grid_sparse<double>(const double4 *, const double2 *, const int32_t *, double2 *, const GridArgs &, int, hipStream_t);
 
