@@ -251,7 +251,7 @@ static int row_mask(Ctx &C, const Tiling &t, int kw, int nf1, int nf2, const uin
 template <typename T>
 static int grid_masks(Ctx &C, GridArgs &g, const uint8_t *mask, int nf1, int nf2)
 {
-    if (mask && C.stop_after != 1 && fft_rows_masked<T>(nf1) && fft_spectrum_pruned<T>(nf2)) {
+    if (mask && C.stop_after != 1 && fft_rows_masked<T>(nf1) && fft_spectrum_pruned(nf2)) {
         // W-stacking grids are gridded in 8 x 8 blocks, 2-D ones in sort tiles
         const int64_t n = g.nf3 > 1 ? sparse_blocks(nf1, nf2) : (int64_t)g.ntx * g.nty;
         CG_TRY(ensure(C.tlist, sizeof(int32_t) * (size_t)(n + 1)));
@@ -284,8 +284,7 @@ static int twiddles(Ctx &C, int n1, int n2)
         // long rows also need the half-length table, stored after the first
         const bool lng = fft_row_long<T>(n1);
         CG_TRY(ensure(C.tw1, (size_t)(lng ? n1 + n1 / 2 : n1) * eb));
-        CG_TRY(launch_twiddles<T>(as<cx_t<T>>(C.tw1), n1, C.stream));
-        if (lng) CG_TRY(launch_twiddles<T>(as<cx_t<T>>(C.tw1) + n1, n1 / 2, C.stream));
+        CG_TRY(launch_row_twiddles<T>(as<cx_t<T>>(C.tw1), n1, C.stream));
         C.tw1_n = n1;
     }
     if (C.tw_bytes != eb || C.tw2_n != n2) {

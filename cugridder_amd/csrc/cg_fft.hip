@@ -3,9 +3,10 @@
 //
 // Unnormalised transform y[k] = sum_j x[j] exp(dir 2 pi i j k / n) along the
 // fast axis (rows, length n1) and the slow axis (columns, length n2) of each
-// [n2][n1] plane.  Every transform runs as a mixed-radix Stockham autosort
-// (radix 8, 4, 2, 3, 5) in LDS: each pass reads its butterflies into
-// registers, barriers, then writes them back in place.
+// [n2][n1] plane.  Every transform runs as a Stockham autosort in LDS: each
+// pass reads its butterflies into registers, barriers, then writes them back
+// in place.  Powers of two have compile-time plans here, other lengths go to
+// the mixed-radix passes of cg_fftmix.hip.
 //
 // Rows: persistent workgroups walk groups of whole rows (one 16384-point
 // fp32 row is 132 KB of padded LDS).
@@ -31,347 +32,10 @@
 // transforms of a split read the length-n2 table with a stride.
 #include <cstdlib>
 
-#include "cg_internal.hpp"
+#include "cg_fft.hpp"
+#include "cg_fftmix.hpp"
 
 namespace cg {
-
-// max elements per thread: 16 complex64 or 8 complex128
-template <typename T>
-constexpr int fft_ept() { return sizeof(T) == 4 ? 16 : 8; }
-
-template <typename T>
-__device__ __forceinline__ cx_t<T> cmul(cx_t<T> a, cx_t<T> b)
-{
-    return mkc(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-template <typename T>
-__device__ __forceinline__ cx_t<T> cadd(cx_t<T> a, cx_t<T> b) { return mkc(a.x + b.x, a.y + b.y); }
-template <typename T>
-__device__ __forceinline__ cx_t<T> csub(cx_t<T> a, cx_t<T> b) { return mkc(a.x - b.x, a.y - b.y); }
-// multiply by dir*i
-template <typename T, int DIR>
-__device__ __forceinline__ cx_t<T> cmul_i(cx_t<T> a)
-{
-    return DIR > 0 ? mkc(-a.y, a.x) : mkc(a.y, -a.x);
-}
-
-// workgroup barrier that orders LDS only: outstanding global loads (the
-// row prefetch) are not waited for
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-template <typename T, int R, int DIR>
-__device__ __forceinline__ void dft_small(cx_t<T> *a)
-{
-    if constexpr (R == 2) {
-        cx_t<T> t = a[0];
-        a[0] = cadd<T>(t, a[1]);
-        a[1] = csub<T>(t, a[1]);
-    } else if constexpr (R == 4) {
-        cx_t<T> t0 = cadd<T>(a[0], a[2]), t1 = csub<T>(a[0], a[2]);
-        cx_t<T> t2 = cadd<T>(a[1], a[3]), t3 = cmul_i<T, DIR>(csub<T>(a[1], a[3]));
-        a[0] = cadd<T>(t0, t2);
-        a[2] = csub<T>(t0, t2);
-        a[1] = cadd<T>(t1, t3);
-        a[3] = csub<T>(t1, t3);
-    } else if constexpr (R == 8) {
-        const T r2 = (T)0.70710678118654752440084436210485;
-        cx_t<T> e[4] = {a[0], a[2], a[4], a[6]};
-        cx_t<T> o[4] = {a[1], a[3], a[5], a[7]};
-        dft_small<T, 4, DIR>(e);
-        dft_small<T, 4, DIR>(o);
-        // W8^k o_k, W8 = (1 + dir i)/sqrt2
-        cx_t<T> w1 = mkc(r2 * (o[1].x - DIR * o[1].y), r2 * (o[1].y + DIR * o[1].x));
-        cx_t<T> w2 = cmul_i<T, DIR>(o[2]);
-        cx_t<T> w3 = mkc(r2 * (-o[3].x - DIR * o[3].y), r2 * (-o[3].y + DIR * o[3].x));
-        a[0] = cadd<T>(e[0], o[0]);
-        a[4] = csub<T>(e[0], o[0]);
-        a[1] = cadd<T>(e[1], w1);
-        a[5] = csub<T>(e[1], w1);
-        a[2] = cadd<T>(e[2], w2);
-        a[6] = csub<T>(e[2], w2);
-        a[3] = cadd<T>(e[3], w3);
-        a[7] = csub<T>(e[3], w3);
-    } else if constexpr (R == 16) {
-        // 16 = 4 x 4: X[k1 + 4 k2] = sum_n2 w16^(n2 k1) [sum_n1 x[4 n1 + n2] w4^(n1 k1)] w4^(n2 k2)
-        const T c1 = (T)0.92387953251128675612818318939679;  // cos(pi/8)
-        const T s1 = (T)0.38268343236508977172845998403040;  // sin(pi/8)
-        const T r2 = (T)0.70710678118654752440084436210485;
-        cx_t<T> y[4][4];
-#pragma unroll
-        for (int n2 = 0; n2 < 4; n2++) {
-            cx_t<T> t[4] = {a[n2], a[4 + n2], a[8 + n2], a[12 + n2]};
-            dft_small<T, 4, DIR>(t);
-#pragma unroll
-            for (int k1 = 0; k1 < 4; k1++) y[n2][k1] = t[k1];
-        }
-        // w16^(DIR m) for m = n2 k1 in {1, 2, 3, 4, 6, 9}
-        auto tw = [&](cx_t<T> v, T wr, T wi) { return mkc(v.x * wr - v.y * wi, v.x * wi + v.y * wr); };
-        const T d = (T)DIR;
-        y[1][1] = tw(y[1][1], c1, d * s1);
-        y[1][2] = tw(y[1][2], r2, d * r2);
-        y[1][3] = tw(y[1][3], s1, d * c1);
-        y[2][1] = tw(y[2][1], r2, d * r2);
-        y[2][2] = cmul_i<T, DIR>(y[2][2]);
-        y[2][3] = tw(y[2][3], -r2, d * r2);
-        y[3][1] = tw(y[3][1], s1, d * c1);
-        y[3][2] = tw(y[3][2], -r2, d * r2);
-        y[3][3] = tw(y[3][3], -c1, -d * s1);
-#pragma unroll
-        for (int k1 = 0; k1 < 4; k1++) {
-            cx_t<T> t[4] = {y[0][k1], y[1][k1], y[2][k1], y[3][k1]};
-            dft_small<T, 4, DIR>(t);
-#pragma unroll
-            for (int k2 = 0; k2 < 4; k2++) a[k1 + 4 * k2] = t[k2];
-        }
-    } else if constexpr (R == 3) {
-        const T h = (T)0.86602540378443864676372317075294;  // sqrt(3)/2
-        cx_t<T> t = cadd<T>(a[1], a[2]);
-        cx_t<T> d = csub<T>(a[1], a[2]);
-        cx_t<T> m = mkc(a[0].x - (T)0.5 * t.x, a[0].y - (T)0.5 * t.y);
-        cx_t<T> e = cmul_i<T, DIR>(mkc(h * d.x, h * d.y));
-        a[0] = cadd<T>(a[0], t);
-        a[1] = cadd<T>(m, e);
-        a[2] = csub<T>(m, e);
-    } else if constexpr (R == 5) {
-        const T c1 = (T)0.30901699437494742410229341718282;    // cos(2pi/5)
-        const T c2 = (T)-0.80901699437494742410229341718282;   // cos(4pi/5)
-        const T s1 = (T)0.95105651629515357211643933337938;    // sin(2pi/5)
-        const T s2 = (T)0.58778525229247312916870595463907;    // sin(4pi/5)
-        cx_t<T> t1 = cadd<T>(a[1], a[4]), t2 = cadd<T>(a[2], a[3]);
-        cx_t<T> d1 = csub<T>(a[1], a[4]), d2 = csub<T>(a[2], a[3]);
-        cx_t<T> b1 = mkc(a[0].x + c1 * t1.x + c2 * t2.x, a[0].y + c1 * t1.y + c2 * t2.y);
-        cx_t<T> b2 = mkc(a[0].x + c2 * t1.x + c1 * t2.x, a[0].y + c2 * t1.y + c1 * t2.y);
-        cx_t<T> e1 = cmul_i<T, DIR>(mkc(s1 * d1.x + s2 * d2.x, s1 * d1.y + s2 * d2.y));
-        cx_t<T> e2 = cmul_i<T, DIR>(mkc(s2 * d1.x - s1 * d2.x, s2 * d1.y - s1 * d2.y));
-        a[0] = mkc(a[0].x + t1.x + t2.x, a[0].y + t1.y + t2.y);
-        a[1] = cadd<T>(b1, e1);
-        a[4] = csub<T>(b1, e1);
-        a[2] = cadd<T>(b2, e2);
-        a[3] = csub<T>(b2, e2);
-    }
-}
-
-struct FftShape {
-    int n;        // transform length
-    int nb;       // transforms per workgroup
-    int lt, le;   // LDS position of element e of transform b: b*lt + e*le
-    int bfast;    // 1: consecutive threads take consecutive transforms (nb = 2^nbsh)
-    int nbsh;
-    int pad;      // > 0: one padding slot after every 2^pad LDS elements
-    int tws;      // twiddle table stride (table length n * tws)
-    int nrad;
-    int rad[16];
-};
-
-// fast-axis indices that carry image pixels: k < a or k >= b
-struct Live {
-    int a, b;
-    __host__ __device__ bool operator()(int k) const { return k < a || k >= b; }
-    __host__ __device__ int count(int n) const { return a + (n - b); }
-    // k-th live index
-    __host__ __device__ int at(int k) const { return k < a ? k : k - a + b; }
-};
-
-__device__ __forceinline__ int lds_pos(const FftShape &S, int x) { return S.pad ? x + (x >> S.pad) : x; }
-
-// one Stockham pass of radix R over all nb transforms held in LDS
-template <typename T, int R, int DIR>
-__device__ __forceinline__ void stockham_pass(cx_t<T> *buf, const FftShape &S, int p,
-                                              const cx_t<T> *__restrict__ tw)
-{
-    constexpr int K = (fft_ept<T>() + R - 1) / R;
-    const int Tn = S.n / R;
-    const int nbf = S.nb * Tn;
-    const int twstep = S.n / (p * R) * S.tws;
-    cx_t<T> u[K][R];
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int q = threadIdx.x + k * blockDim.x;
-        if (q < nbf) {
-            int b, i;
-            if (S.bfast) {
-                b = q & (S.nb - 1);
-                i = q >> S.nbsh;
-            } else {
-                b = q / Tn;
-                i = q - b * Tn;
-            }
-#pragma unroll
-            for (int r = 0; r < R; r++) u[k][r] = buf[lds_pos(S, b * S.lt + (i + r * Tn) * S.le)];
-        }
-    }
-    lds_barrier();
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int q = threadIdx.x + k * blockDim.x;
-        if (q < nbf) {
-            int b, i;
-            if (S.bfast) {
-                b = q & (S.nb - 1);
-                i = q >> S.nbsh;
-            } else {
-                b = q / Tn;
-                i = q - b * Tn;
-            }
-            const int kk = i % p;
-#pragma unroll
-            for (int r = 1; r < R; r++) {
-                cx_t<T> w = tw[(unsigned)(r * kk * twstep)];
-                if (DIR < 0) w.y = -w.y;
-                u[k][r] = cmul<T>(u[k][r], w);
-            }
-            dft_small<T, R, DIR>(u[k]);
-            const int j = (i - kk) * R + kk;
-#pragma unroll
-            for (int r = 0; r < R; r++) buf[lds_pos(S, b * S.lt + (j + r * p) * S.le)] = u[k][r];
-        }
-    }
-    lds_barrier();
-}
-
-template <typename T, int DIR>
-__device__ void lds_fft(cx_t<T> *buf, const FftShape &S, const cx_t<T> *tw)
-{
-    int p = 1;
-    for (int s = 0; s < S.nrad; s++) {
-        const int R = S.rad[s];
-        switch (R) {
-        case 8: stockham_pass<T, 8, DIR>(buf, S, p, tw); break;
-        case 4: stockham_pass<T, 4, DIR>(buf, S, p, tw); break;
-        case 2: stockham_pass<T, 2, DIR>(buf, S, p, tw); break;
-        case 3: stockham_pass<T, 3, DIR>(buf, S, p, tw); break;
-        case 5: stockham_pass<T, 5, DIR>(buf, S, p, tw); break;
-        default: break;
-        }
-        p *= R;
-    }
-}
-
-// Rows.  Group g holds rows [g nb, g nb + nb) of the nrows rows of all planes
-// (rows are contiguous across planes).  DIR > 0 stores only live outputs;
-// DIR < 0 reads only live inputs.
-template <typename T, int DIR>
-__global__ __launch_bounds__(1024) void k_fft_rows(cx_t<T> *data, int64_t nrows, int n1,
-                                                   FftShape S, const cx_t<T> *__restrict__ tw,
-                                                   Live live)
-{
-    constexpr int EPT = fft_ept<T>();
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    cx_t<T> *buf = reinterpret_cast<cx_t<T> *>(smem_raw);
-    const int E = S.nb * n1;
-    const int64_t ngroups = (nrows + S.nb - 1) / S.nb;
-    cx_t<T> pre[EPT];
-    // elements of group grp that exist (the last group may be short)
-    auto count = [&](int64_t grp) -> int {
-        return (int)min((int64_t)E, (nrows - grp * S.nb) * n1);
-    };
-    auto load = [&](int64_t grp) {
-        const cx_t<T> *src = data + grp * (int64_t)E;
-        const int lim = count(grp);
-#pragma unroll
-        for (int u = 0; u < EPT; u++) {
-            const int k = threadIdx.x + u * blockDim.x;
-            const int e = S.nb == 1 ? k : k % n1;
-            pre[u] = (k < lim && (DIR > 0 || live(e))) ? src[k] : mkc((T)0, (T)0);
-        }
-    };
-    for (int64_t g = blockIdx.x; g < ngroups; g += gridDim.x) {
-        load(g);
-#pragma unroll
-        for (int u = 0; u < EPT; u++) {
-            const int k = threadIdx.x + u * blockDim.x;
-            if (k < E) buf[lds_pos(S, k)] = pre[u];
-        }
-        lds_barrier();
-        lds_fft<T, DIR>(buf, S, tw);
-        cx_t<T> *dst = data + g * (int64_t)E;
-        const int lim = count(g);
-#pragma unroll
-        for (int u = 0; u < EPT; u++) {
-            const int k = threadIdx.x + u * blockDim.x;
-            const int e = S.nb == 1 ? k : k % n1;
-            if (k < lim && (DIR < 0 || live(e))) dst[k] = buf[lds_pos(S, k)];
-        }
-        lds_barrier();
-    }
-}
-
-// Columns, whole transform per workgroup: blockIdx.x = block of S.nb live
-// columns, blockIdx.y = plane.  Natural order in and out.
-template <typename T, int DIR>
-__global__ __launch_bounds__(1024) void k_fft_cols(cx_t<T> *data, int n2, int n1, FftShape S,
-                                                   const cx_t<T> *__restrict__ tw, Live live)
-{
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    cx_t<T> *buf = reinterpret_cast<cx_t<T> *>(smem_raw);
-    cx_t<T> *pl = data + (size_t)blockIdx.y * n2 * n1;
-    const int nlive = live.count(n1);
-    const int c0 = blockIdx.x * S.nb;
-    const int E = S.nb * n2;
-    for (int k = threadIdx.x; k < E; k += blockDim.x) {
-        const int e = k >> S.nbsh, b = k & (S.nb - 1);
-        const int c = c0 + b;
-        buf[k] = c < nlive ? pl[(size_t)e * n1 + live.at(c)] : mkc((T)0, (T)0);
-    }
-    lds_barrier();
-    lds_fft<T, DIR>(buf, S, tw);
-    for (int k = threadIdx.x; k < E; k += blockDim.x) {
-        const int e = k >> S.nbsh, b = k & (S.nb - 1);
-        const int c = c0 + b;
-        if (c < nlive) pl[(size_t)e * n1 + live.at(c)] = buf[k];
-    }
-}
-
-// One step of the in-place split of long columns.  Sub-transform j
-// (blockIdx.y) of length L = S.n reads and writes rows j*sj + e*se, e < L;
-// twmode 1 multiplies output e by w^(j e) after the transform, twmode 2
-// multiplies input e by w^(j e) before it, w = e^{dir 2 pi i/n2} (tw2 is the
-// length-n2 table).  blockIdx.x = block of S.nb live columns, blockIdx.z =
-// plane.
-template <typename T, int DIR>
-__global__ __launch_bounds__(1024) void k_fft_cols_step(cx_t<T> *data, int n2, int n1, FftShape S,
-                                                        int se, int sj, int twmode,
-                                                        const cx_t<T> *__restrict__ tw2, Live live)
-{
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    cx_t<T> *buf = reinterpret_cast<cx_t<T> *>(smem_raw);
-    const int j = blockIdx.y;
-    cx_t<T> *pl = data + (size_t)blockIdx.z * n2 * n1;
-    const int nlive = live.count(n1);
-    const int c0 = blockIdx.x * S.nb;
-    const int E = S.nb * S.n;
-    const size_t row0 = (size_t)j * sj;
-    for (int k = threadIdx.x; k < E; k += blockDim.x) {
-        const int e = k >> S.nbsh, b = k & (S.nb - 1);
-        const int c = c0 + b;
-        cx_t<T> v = c < nlive ? pl[(row0 + (size_t)e * se) * n1 + live.at(c)] : mkc((T)0, (T)0);
-        if (twmode == 2) {
-            cx_t<T> w = tw2[j * e];
-            if (DIR < 0) w.y = -w.y;
-            v = cmul<T>(v, w);
-        }
-        buf[k] = v;
-    }
-    lds_barrier();
-    lds_fft<T, DIR>(buf, S, tw2);
-    for (int k = threadIdx.x; k < E; k += blockDim.x) {
-        const int e = k >> S.nbsh, b = k & (S.nb - 1);
-        const int c = c0 + b;
-        if (c >= nlive) continue;
-        cx_t<T> v = buf[k];
-        if (twmode == 1) {
-            cx_t<T> w = tw2[j * e];
-            if (DIR < 0) w.y = -w.y;
-            v = cmul<T>(v, w);
-        }
-        pl[(row0 + (size_t)e * se) * n1 + live.at(c)] = v;
-    }
-}
 
 // ------------------------------------------------------------ compile-time plans
 //
@@ -1134,18 +798,6 @@ __global__ __launch_bounds__(256) void k_col_permute(const cx_t<T> *__restrict__
     else dst[(base + pos) * n1 + c] = src[idx];
 }
 
-static int factor_radices(int n, int *rad)
-{
-    int nr = 0;
-    while (n % 8 == 0) { rad[nr++] = 8; n /= 8; }
-    while (n % 4 == 0) { rad[nr++] = 4; n /= 4; }
-    while (n % 2 == 0) { rad[nr++] = 2; n /= 2; }
-    while (n % 3 == 0) { rad[nr++] = 3; n /= 3; }
-    while (n % 5 == 0) { rad[nr++] = 5; n /= 5; }
-    return n == 1 ? nr : -1;
-}
-
-static int round64(int x) { return (x + 63) / 64 * 64; }
 static int ilog2(int x)
 {
     int l = 0;
@@ -1182,22 +834,14 @@ static int fft_knob(const char *name, int dflt)
     return e ? std::atoi(e) : dflt;
 }
 
-// rows: row padded in LDS by one slot per 32 elements (bank spread of the
-// strided Stockham writes)
 template <typename T>
-static int row_lds_bytes(int n1, int nb)
-{
-    const int E = nb * n1;
-    return (E + (E >> 5)) * (int)sizeof(cx_t<T>);
-}
+static bool rows_ct_covers(int n1);
 
 // a row transform held whole in one workgroup's LDS
 template <typename T>
 static bool fft_row_whole(int n)
 {
-    int rad[32];
-    if (n < 1 || factor_radices(n, rad) < 0) return false;
-    return n <= 1024 * fft_ept<T>() && row_lds_bytes<T>(n, 1) <= kLdsMax;
+    return n >= 1 && n <= 1024 * fft_ept<T>() && (rows_ct_covers<T>(n) || fft_rows_mix_supported<T>(n));
 }
 
 template <typename T>
@@ -1206,10 +850,9 @@ bool fft_row_long(int n)
     // complex128 rows beyond one workgroup (n > 8192): one radix-2 step in
     // HBM around two half-length whole-row transforms; the columns of such
     // a grid go through the four-step split
-    int na, nb, rad[32];
+    int na, nb;
     return sizeof(T) == 8 && !fft_row_whole<T>(n) && n % 2 == 0 && n <= 16384 &&
-           fft_row_whole<T>(n / 2) && fft_col_split(n, na, nb) && factor_radices(na, rad) >= 0 &&
-           factor_radices(nb, rad) >= 0;
+           fft_row_whole<T>(n / 2) && fft_col_split(n, na, nb) && fft_cols_mix_supported(n);
 }
 
 template <typename T>
@@ -1459,33 +1102,7 @@ static int fft_rows(cx_t<T> *data, int batch, int n2, int n1, const cx_t<T> *tw,
         const int r = rows_ct_dispatch<T, DIR>(data, (int64_t)n2 * batch, n1, tw, live, rowmask, n2, s);
         if (r != 1) return r;
     }
-    FftShape S{};
-    S.n = n1;
-    S.nrad = factor_radices(n1, S.rad);
-    if (S.nrad < 0) return CG_ERR_SIZE;
-    int nb = std::max(1, 4096 / n1);
-    while (nb > 1 && row_lds_bytes<T>(n1, nb) > 65536) nb--;
-    const int E = nb * n1;
-    const size_t lds = (size_t)row_lds_bytes<T>(n1, nb);
-    if (E > 1024 * fft_ept<T>() || lds > (size_t)kLdsMax) return CG_ERR_SIZE;
-    const int threads = std::min(std::max(round64((E + fft_ept<T>() - 1) / fft_ept<T>()), 64), 1024);
-    S.nb = nb;
-    S.lt = n1;
-    S.le = 1;
-    S.pad = 5;
-    S.tws = 1;
-    const int64_t nrows = (int64_t)n2 * batch;
-    const int64_t ngroups = (nrows + nb - 1) / nb;
-    int per_cu = std::max<int>(1, (int)(kLdsMax / lds));
-    per_cu = std::min(per_cu, std::max(1, 2048 / threads));
-    const int64_t grid = std::min<int64_t>(ngroups, (int64_t)256 * per_cu);
-    if (lds > 65536)
-        CG_HIP(hipFuncSetAttribute((const void *)k_fft_rows<T, DIR>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((k_fft_rows<T, DIR>), dim3((unsigned)grid), dim3(threads), lds, s, data,
-                       nrows, n1, S, tw, live);
-    CG_HIP(hipGetLastError());
-    return CG_OK;
+    return launch_fft_rows_mix<T>(data, (int64_t)n2 * batch, n1, DIR, tw, live.a, live.b, rowmask, n2, s);
 }
 
 template <typename T, int DIR>
@@ -1493,7 +1110,6 @@ static int fft_cols(cx_t<T> *data, int batch, int n2, int n1, const cx_t<T> *tw2
                     const uint8_t *rowmask, int spec_a, int spec_b, int band_s, int band_len,
                     hipStream_t s)
 {
-    const int elem = (int)sizeof(cx_t<T>);
     const int nlive = live.count(n1);
     if (nlive <= 0 || batch <= 0) return CG_OK;
     int na, nb;
@@ -1504,7 +1120,7 @@ static int fft_cols(cx_t<T> *data, int batch, int n2, int n1, const cx_t<T> *tw2
         const size_t lds = sizeof(float2) * ((size_t)M * CB + M + (1 << kBandTwSh) + (n2 >> kBandTwSh));
         // (byte offsets inside a plane are 32-bit in the kernel)
         if (band_len > 0 && band_len <= M && lds <= (size_t)kLdsMax && band_s >= 0 && band_s < n2 &&
-            fft_spectrum_pruned<T>(n2) && (n2 & (n2 - 1)) == 0 &&
+            (n2 & (n2 - 1)) == 0 &&
             (size_t)n2 * n1 * sizeof(float2) <= 0xffffffffu && n2 >= 2 * M && fft_col_split(n2, na, nb)) {
             int nblk = (nlive + CB - 1) / CB;
             if (M == 2048) nblk = (nblk + 15) / 16 * 16;  // whole groups of the block remap
@@ -1523,70 +1139,30 @@ static int fft_cols(cx_t<T> *data, int batch, int n2, int n1, const cx_t<T> *tw2
         }
     }
     if (!fft_col_split(n2, na, nb)) {
-        FftShape S{};
-        S.n = n2;
-        S.nrad = factor_radices(n2, S.rad);
-        if (S.nrad < 0) return CG_ERR_SIZE;
-        // power-of-two block of adjacent columns, up to 64 KB of LDS
-        int cb = 1;
-        while (cb * 2 <= 64 && (int64_t)cb * 2 * n2 * elem <= 65536 && cb * 2 <= nlive) cb *= 2;
-        const int E = cb * n2;
-        const size_t lds = (size_t)E * elem;
-        if (E > 1024 * fft_ept<T>() || lds > (size_t)kLdsMax) return CG_ERR_SIZE;
-        const int threads = std::min(std::max(round64((E + fft_ept<T>() - 1) / fft_ept<T>()), 64), 1024);
-        S.nb = cb;
-        S.nbsh = ilog2(cb);
-        S.bfast = 1;
-        S.lt = 1;
-        S.le = cb;
-        S.tws = 1;
-        if (lds > 65536)
-            CG_HIP(hipFuncSetAttribute((const void *)k_fft_cols<T, DIR>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL((k_fft_cols<T, DIR>), dim3((unsigned)((nlive + cb - 1) / cb), (unsigned)batch),
-                           dim3(threads), lds, s, data, n2, n1, S, tw2, live);
-        CG_HIP(hipGetLastError());
-        return CG_OK;
+        // the whole column: rows in natural order on both sides
+        const int freq = spec_a < spec_b ? 2 : 0;
+        return launch_fft_cols_mix<T>(data, batch, n2, n1, n2, DIR, 1, 0, 1, 0, tw2, live.a, live.b, rowmask,
+                                      DIR > 0 ? 1 : freq, DIR > 0 ? freq : 1, spec_a, spec_b, s);
     }
     // dead rows: forward, the natural-order step skips loading masked-out
     // rows and the split-order step skips storing dead frequencies; inverse,
     // the split-order step skips loading dead frequencies and the
     // natural-order step skips storing masked-out rows
     auto step = [&](int L, int se, int sj, int nsub, int twmode) -> int {
-        {
-            DeadRows d{rowmask, spec_a, spec_b, 0, 0};
-            const bool natural = sj == 1;
-            const bool active = natural ? rowmask != nullptr : spec_a < spec_b;
-            if (active) {
-                const bool in = (DIR > 0) == natural;
-                d.mode_in = in ? 1 : 0;
-                d.mode_out = in ? 0 : 1;
-            }
-            const int r = cols_step_ct_dispatch<T, DIR>(data, batch, n2, n1, L, se, sj, nsub, twmode,
-                                                        tw2, live, d, s);
-            if (r != 1) return r;
+        DeadRows d{rowmask, spec_a, spec_b, 0, 0};
+        const bool natural = sj == 1;
+        const bool active = natural ? rowmask != nullptr : spec_a < spec_b;
+        const bool in = (DIR > 0) == natural;
+        if (active) {
+            d.mode_in = in ? 1 : 0;
+            d.mode_out = in ? 0 : 1;
         }
-        FftShape S{};
-        S.n = L;
-        S.nrad = factor_radices(L, S.rad);
-        if (S.nrad < 0) return CG_ERR_SIZE;
-        // 512-byte row segments, at most 64 KB of LDS
-        int cb = 512 / elem;
-        while (cb > 1 && (int64_t)cb * L * elem > 65536) cb /= 2;
-        const int E = cb * L;
-        const int threads = std::min(std::max(round64((E + fft_ept<T>() - 1) / fft_ept<T>()), 64), 1024);
-        if ((int64_t)threads * fft_ept<T>() < E) return CG_ERR_SIZE;
-        S.nb = cb;
-        S.nbsh = ilog2(cb);
-        S.bfast = 1;
-        S.lt = 1;
-        S.le = cb;
-        S.tws = n2 / L;
-        dim3 grid((unsigned)((nlive + cb - 1) / cb), (unsigned)nsub, (unsigned)batch);
-        hipLaunchKernelGGL((k_fft_cols_step<T, DIR>), grid, dim3(threads), (size_t)E * elem, s,
-                           data, n2, n1, S, se, sj, twmode, tw2, live);
-        CG_HIP(hipGetLastError());
-        return CG_OK;
+        const int r = cols_step_ct_dispatch<T, DIR>(data, batch, n2, n1, L, se, sj, nsub, twmode, tw2, live,
+                                                    d, s);
+        if (r != 1) return r;
+        const int mode = active ? (natural ? 1 : 2) : 0;
+        return launch_fft_cols_mix<T>(data, batch, n2, n1, L, DIR, se, sj, nsub, twmode, tw2, live.a, live.b,
+                                      rowmask, in ? mode : 0, in ? 0 : mode, spec_a, spec_b, s);
     };
     int r;
     if (DIR > 0) {
@@ -1619,11 +1195,10 @@ int launch_fft_pass(cx_t<T> *data, int batch, int n2, int n1, int dir, bool rows
                                      band_len, s);
 }
 
+// the lengths rows_ct handles
 template <typename T>
-bool fft_rows_masked(int n1)
+static bool rows_ct_covers(int n1)
 {
-    // the conditions under which fft_rows takes rows_ct (which honours the
-    // row and column masks)
     const int l = log2_exact(n1);
     if (l < 9 || l > 14) return false;
     const int nt = n1 / fft_ept<T>();
@@ -1633,12 +1208,14 @@ bool fft_rows_masked(int n1)
 }
 
 template <typename T>
+bool fft_rows_masked(int n1)
+{
+    return fft_row_whole<T>(n1);
+}
+
 bool fft_spectrum_pruned(int n2)
 {
-    int na, nb;
-    if (n2 <= 1 || !fft_col_split(n2, na, nb)) return false;
-    const int ln = log2_exact(na), lb = log2_exact(nb);
-    return ln >= 4 && ln <= 8 && lb >= 4 && lb <= 8;
+    return n2 > 1 && fft_cols_mix_supported(n2);
 }
 
 template <typename T>
@@ -1691,18 +1268,29 @@ int launch_twiddles(cx_t<T> *tw, int n, hipStream_t s)
     return CG_OK;
 }
 
+template <typename T>
+int launch_row_twiddles(cx_t<T> *tw, int n, hipStream_t s)
+{
+    if (fft_row_long<T>(n)) {
+        // natural order, then the table of the half-length rows
+        CG_TRY(launch_twiddles<T>(tw, n, s));
+        return launch_row_twiddles<T>(tw + n, n / 2, s);
+    }
+    return rows_ct_covers<T>(n) ? launch_twiddles<T>(tw, n, s) : launch_mix_twiddles<T>(tw, n, s);
+}
+
 template int launch_fft2d<float>(float2 *, int, int, int, int, const float2 *, const float2 *, float2 *, hipStream_t);
 template int launch_fft2d<double>(double2 *, int, int, int, int, const double2 *, const double2 *, double2 *, hipStream_t);
 template int launch_fft_pass<float>(float2 *, int, int, int, int, bool, const float2 *, int, int, const uint8_t *, int, int, hipStream_t, int, int);
 template int launch_fft_pass<double>(double2 *, int, int, int, int, bool, const double2 *, int, int, const uint8_t *, int, int, hipStream_t, int, int);
 template bool fft_rows_masked<float>(int);
 template bool fft_rows_masked<double>(int);
-template bool fft_spectrum_pruned<float>(int);
-template bool fft_spectrum_pruned<double>(int);
 template bool fft_supported<float>(int);
 template bool fft_supported<double>(int);
 template bool fft_row_long<float>(int);
 template bool fft_row_long<double>(int);
+template int launch_row_twiddles<float>(float2 *, int, hipStream_t);
+template int launch_row_twiddles<double>(double2 *, int, hipStream_t);
 template int launch_twiddles<float>(float2 *, int, hipStream_t);
 template int launch_twiddles<double>(double2 *, int, hipStream_t);
 

@@ -234,8 +234,8 @@ int launch_degrid_dense(const float4 *geo, const float2 *fac, const int32_t *per
 
 // ---- FFT (cg_fft.hip): in-place unnormalised 2-D FFT of `batch` planes
 // [batch][n2][n1], exponent sign dir (+1 / -1), natural order in and out.
-// tw1/tw2 are device tables of e^{+2 pi i t/n} (length n1 / n2) in
-// precision T; tmp (batch*n2*n1 elements) is needed when n2 is split.
+// tw1 (launch_row_twiddles, n1) and tw2 (launch_twiddles, n2) are device
+// tables in precision T; tmp (batch*n2*n1 elements) is needed when n2 is split.
 template <typename T>
 int launch_fft2d(cx_t<T> *data, int batch, int n2, int n1, int dir, const cx_t<T> *tw1,
                  const cx_t<T> *tw2, cx_t<T> *tmp, hipStream_t s);
@@ -263,7 +263,6 @@ int launch_fft_pass(cx_t<T> *data, int batch, int n2, int n1, int dir, bool rows
 // true when the column pass honours the dead spectrum rows (then a dir < 0
 // column pass does not read them and they need not be written); it then
 // also honours the row mask (a dir > 0 pass does not read masked rows)
-template <typename T>
 bool fft_spectrum_pruned(int n2);
 // true when the row pass honours the row and column masks (a dir > 0 pass
 // reads neither masked rows nor masked columns)
@@ -280,6 +279,10 @@ template <typename T>
 bool fft_row_long(int n);
 template <typename T>
 int launch_twiddles(cx_t<T> *tw, int n, hipStream_t s);
+// the table of a row pass (tw1): e^{+2 pi i t/n} in the order its kernel reads
+// (n entries, n + n / 2 with fft_row_long)
+template <typename T>
+int launch_row_twiddles(cx_t<T> *tw, int n, hipStream_t s);
 
 // ---- W-stacking per-pixel stages (cg_wstack.hip), FP64 phases & factors
 // Gauss-Legendre quadrature of the ES kernel's Fourier transform

@@ -123,7 +123,7 @@ WArgs make_wargs(const WPlan &p)
     w.qd = make_quad(p.conv);
     fit_psihat(w);
     if (!(p.nf2 > 1 && fft_col_split(p.nf2, w.cna, w.cnb))) w.cna = w.cnb = 0;
-    w.skip_dead = fft_spectrum_pruned<float>(p.nf2) ? 1 : 0;
+    w.skip_dead = fft_spectrum_pruned(p.nf2) ? 1 : 0;
     return w;
 }
 
