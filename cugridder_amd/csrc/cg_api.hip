@@ -308,13 +308,13 @@ static int sort_rows(Ctx &C, const TU *uvw, int64_t M, const CoordArgs &a, const
     CG_TRY(ensure(C.keys2, sizeof(uint32_t) * M));
     CG_TRY(ensure(C.vals, sizeof(int32_t) * M));
     CG_TRY(ensure(C.vals2, sizeof(int32_t) * M));
-    const int64_t hs = radix_hist_size(M);
+    const int bits = sort_key_bits(a, ntiles);
+    const int64_t hs = radix_hist_size_short(M);
     CG_TRY(ensure(C.hist, sizeof(int32_t) * hs));
     CG_TRY(ensure(C.scan, sizeof(int32_t) * std::max(scan_tmp_size(hs), scan_tmp_size(ntiles + 1))));
     CG_TRY(ensure(C.tstart, sizeof(int32_t) * (ntiles + 1)));
     // an odd number of radix passes starts in the second buffers, so the
     // sorted keys and permutation end in C.keys / C.vals without a copy
-    const int bits = sort_key_bits(a, ntiles);
     const bool odd = radix_passes(bits) & 1;
     uint32_t *k0 = as<uint32_t>(odd ? C.keys2 : C.keys), *k1 = as<uint32_t>(odd ? C.keys : C.keys2);
     int32_t *v0 = as<int32_t>(odd ? C.vals2 : C.vals), *v1 = as<int32_t>(odd ? C.vals : C.vals2);
@@ -324,8 +324,8 @@ static int sort_rows(Ctx &C, const TU *uvw, int64_t M, const CoordArgs &a, const
                                                            C.stream)));
     else
         CG_TRY(launch_keys<TU>(uvw, M, a, k0, nullptr, C.stream));
-    CG_TRY(launch_radix_sort(k0, v0, k1, v1, M, bits, as<int32_t>(C.hist), as<int32_t>(C.scan), C.stream, 0,
-                             1));
+    CG_TRY(launch_radix_sort(k0, v0, k1, v1, M, bits, as<int32_t>(C.hist), hs, as<int32_t>(C.scan), C.stream,
+                             0, 1));
     CG_TRY(launch_tile_bounds(as<uint32_t>(C.keys), M, ntiles, a.cshift, key_rect(a), as<int32_t>(C.tstart),
                               C.stream));
     return CG_OK;
@@ -1212,11 +1212,12 @@ int nufft2d_dev(Ctx &C, int type, int64_t M, const TU *x, const TU *y, cx_t<T> *
         CG_TRY(ensure(C.keys2, sizeof(uint32_t) * M));
         CG_TRY(ensure(C.vals, sizeof(int32_t) * M));
         CG_TRY(ensure(C.vals2, sizeof(int32_t) * M));
-        const int64_t hs = radix_hist_size(M);
+        const int bits = sort_key_bits(a, ntiles);
+        // (the fixed region keeps the size that nufft2d_workspace reckons with)
+        const int64_t hs = C.arena_mode ? radix_hist_size(M) : radix_hist_size_short(M);
         CG_TRY(ensure(C.hist, sizeof(int32_t) * hs));
         CG_TRY(ensure(C.scan, sizeof(int32_t) * scan_tmp_size(hs)));
         // odd pass counts start in the second buffers (no copy at the end)
-        const int bits = sort_key_bits(a, ntiles);
         const bool odd = radix_passes(bits) & 1;
         uint32_t *k0 = as<uint32_t>(odd ? C.keys2 : C.keys), *k1 = as<uint32_t>(odd ? C.keys : C.keys2);
         int32_t *v0 = as<int32_t>(odd ? C.vals2 : C.vals), *v1 = as<int32_t>(odd ? C.vals : C.vals2);
@@ -1226,8 +1227,8 @@ int nufft2d_dev(Ctx &C, int type, int64_t M, const TU *x, const TU *y, cx_t<T> *
                                                  k0, nullptr, rec, C.stream));
         }
         if (!rec) CG_TRY(launch_keys_xy<TU>(x, y, M, a, k0, nullptr, C.stream));
-        CG_TRY(launch_radix_sort(k0, v0, k1, v1, M, bits, as<int32_t>(C.hist), as<int32_t>(C.scan),
-                                 C.stream, 0, 1));
+        CG_TRY(launch_radix_sort(k0, v0, k1, v1, M, bits, as<int32_t>(C.hist), hs,
+                                 as<int32_t>(C.scan), C.stream, 0, 1));
         CG_TRY(launch_tile_bounds(as<uint32_t>(C.keys), M, ntiles, a.cshift, key_rect(a),
                                   as<int32_t>(C.tstart), C.stream));
     } else {
@@ -2096,11 +2097,11 @@ int cg_sort_pairs_dev(void *ctx, void *d_keys, void *d_vals, int m, int key_bits
     if (m == 0) return CG_OK;
     CG_TRY(ensure(C->keys2, sizeof(uint32_t) * m));
     CG_TRY(ensure(C->vals2, sizeof(int32_t) * m));
-    const int64_t hs = radix_hist_size(m);
+    const int64_t hs = radix_hist_size_short(m);
     CG_TRY(ensure(C->hist, sizeof(int32_t) * hs));
     CG_TRY(ensure(C->scan, sizeof(int32_t) * scan_tmp_size(hs)));
     return launch_radix_sort((uint32_t *)d_keys, (int32_t *)d_vals, as<uint32_t>(C->keys2),
-                             as<int32_t>(C->vals2), m, key_bits, as<int32_t>(C->hist),
+                             as<int32_t>(C->vals2), m, key_bits, as<int32_t>(C->hist), hs,
                              as<int32_t>(C->scan), C->stream);
 }
 

@@ -122,11 +122,14 @@ int launch_gather_records_xy(const float4 *rec, const int32_t *perm, int64_t m, 
 // buffers gets the result in its keys without a copy.  identity_vals: vals
 // are not read, the first pass takes value i for item i (the key kernels
 // then need not write them).
+// hist_ints: the size of hist; from radix_hist_size_short on, short sorts take
+// two launches per pass.
 int64_t radix_hist_size(int64_t m);
+int64_t radix_hist_size_short(int64_t m);
 int radix_passes(int key_bits);
 int launch_radix_sort(uint32_t *keys, int32_t *vals, uint32_t *tmp_keys,
                       int32_t *tmp_vals, int64_t m, int key_bits, int32_t *hist,
-                      int32_t *scan_tmp, hipStream_t s, int copy_back = 1, int identity_vals = 0);
+                      int64_t hist_ints, int32_t *scan_tmp, hipStream_t s, int copy_back = 1, int identity_vals = 0);
 int64_t scan_tmp_size(int64_t n);
 // exclusive scan of n ints in place
 int launch_exclusive_scan(int32_t *data, int64_t n, int32_t *scan_tmp, hipStream_t s);
