@@ -77,6 +77,10 @@ struct Ctx {
     DevBuf keys, keys2, vals, vals2, hist, scan, tstart, geo, val, grid, zq, phi3, phi1, phi2,
         part, tw1, tw2, fftmp, dlist, rmask, chans, tlist;
     int tw1_n = 0, tw2_n = 0, tw_bytes = 0;
+    // 6 doubles of pinned memory for the coordinate ranges, in contexts that
+    // outlive a call (keep_pinned)
+    double *pinned = nullptr;
+    bool keep_pinned = false;
     // stage timing (HIP events on the context stream)
     bool timing = false;
     // stage marks ev[0..ST_COUNT]; ev[ST_COUNT + 1, + 2] bracket the dense
@@ -138,6 +142,7 @@ struct Ctx {
         each_buf([](DevBuf &b) {
             if (b.p && !b.arena) (void)hipFree(b.p);
         });
+        if (pinned) (void)hipHostFree(pinned);
         if (ev_ok)
             for (auto &e : ev) (void)hipEventDestroy(e);
     }
@@ -232,17 +237,20 @@ struct StageClock {
     }
 };
 
-// rows (mask[0, nf2)) and columns (mask[nf2, nf2 + nf1)) of the grid that
-// points of non-empty tiles reach (null: all); needs the tile starts of the
-// last sort
-static int row_mask(Ctx &C, const Tiling &t, int kw, int nf1, int nf2, const uint8_t *&mask)
+// the buffer of the row and column masks of the last sort's points
+// (launch_tile_bounds fills it; null: every row and column)
+static int row_mask(Ctx &C, int nf1, int nf2, uint8_t *&mask)
 {
     mask = nullptr;
     if (!C.row_mask) return CG_OK;
     CG_TRY(ensure(C.rmask, (size_t)nf1 + nf2));
-    CG_TRY(launch_row_mask(as<int32_t>(C.tstart), t, kw, nf1, nf2, as<uint8_t>(C.rmask), C.stream));
     mask = as<uint8_t>(C.rmask);
     return CG_OK;
+}
+
+static TileMask tile_mask(uint8_t *mask, const Tiling &t, int kw, int nf1, int nf2)
+{
+    return TileMask{mask, t.ntx, t.tx, t.ty, kw, nf1, nf2};
 }
 
 // lets the gridder leave the tiles the FFT will not read unwritten, when
@@ -301,7 +309,7 @@ static int twiddles(Ctx &C, int n1, int n2)
 // the key pass also writes the caller-order record slots of vis and wgt.
 template <typename TU>
 static int sort_rows(Ctx &C, const TU *uvw, int64_t M, const CoordArgs &a, const Tiling &t,
-                     const float2 *vis = nullptr, const float *wgt = nullptr, float4 *rec = nullptr)
+                     uint8_t *mask, const float2 *vis = nullptr, const float *wgt = nullptr, float4 *rec = nullptr)
 {
     const int64_t ntiles = t.ntiles();
     CG_TRY(ensure(C.keys, sizeof(uint32_t) * M));
@@ -327,7 +335,7 @@ static int sort_rows(Ctx &C, const TU *uvw, int64_t M, const CoordArgs &a, const
     CG_TRY(launch_radix_sort(k0, v0, k1, v1, M, bits, as<int32_t>(C.hist), hs, as<int32_t>(C.scan), C.stream,
                              0, 1));
     CG_TRY(launch_tile_bounds(as<uint32_t>(C.keys), M, ntiles, a.cshift, key_rect(a), as<int32_t>(C.tstart),
-                              C.stream));
+                              tile_mask(mask, t, a.kw, a.nf1, a.nf2), C.stream));
     return CG_OK;
 }
 
@@ -401,9 +409,18 @@ static int plan_call(Ctx &C, WPlan &P, int64_t nrow, int nchan, const double *fr
     if (nrow * (int64_t)nchan > (int64_t)INT32_MAX - 1) return CG_ERR_SIZE;
     for (int c = 0; c < nchan; c++)
         if (!(freq[c] > 0)) return CG_ERR_ARG;
-    CG_TRY(ensure(C.part, sizeof(double) * 6152));
+    if (!C.part.p) {
+        CG_TRY(ensure(C.part, sizeof(double) * 6152));
+        CG_TRY(launch_fill_i32(as<int32_t>(C.part), 2 * 6152, 0, C.stream));
+    }
+    if (C.keep_pinned && !C.pinned && hipHostMalloc((void **)&C.pinned, 6 * sizeof(double), 0) != hipSuccess) {
+        (void)hipGetLastError();
+        C.pinned = nullptr;
+        C.keep_pinned = false;
+    }
     double wlo = 0, whi = 0, wmin = 0, wmax = 0, uv[4] = {0, 0, 0, 0};
-    CG_TRY(launch_wminmax<TU>(uvw, nrow, 1.0, as<double>(C.part), wlo, whi, C.stream, uv));
+    CG_TRY(launch_wminmax<TU>(uvw, nrow, 1.0, as<double>(C.part), wlo, whi, C.stream, uv,
+                              C.pinned));
     if (nrow > 0) {
         wmin = INFINITY;
         wmax = -INFINITY;
@@ -532,6 +549,19 @@ static size_t slab_bytes(const WPlan &P, int slab, int eb)
     return (size_t)P.nf1 * P.nf2 * (slab ? slab : P.nf3) * eb;
 }
 
+// room for the correction factors and the quarter tables
+static int image_tables(Ctx &C, const WPlan &P)
+{
+    CG_TRY(ensure(C.phi1, sizeof(double) * (P.nf1 / 2 + 1)));
+    CG_TRY(ensure(C.phi2, sizeof(double) * (P.nf2 / 2 + 1)));
+    if (P.wstack) {
+        const int64_t nq = (int64_t)(P.N1 / 2 + 1) * (P.N2 / 2 + 1);
+        CG_TRY(ensure(C.zq, sizeof(double) * nq));
+        CG_TRY(ensure(C.phi3, sizeof(double) * nq));
+    }
+    return CG_OK;
+}
+
 // vis and wgt are [nrow][nchan]; every (row, channel) is one point
 template <typename T, typename TU>
 static int plan_ms2dirty(Ctx &C, CallPlan &cp, int64_t nrow, int nchan, const double *freq,
@@ -576,15 +606,33 @@ static int exec_ms2dirty(Ctx &C, const CallPlan &cp, const TU *uvw, const cx_t<T
     C.last_m = M;
     C.last_cshift = a.cshift;
     CG_TRY(clk.mark(ST_SORT));
+    // the call's tables and cleared masks and lists, before the sort fills the
+    // masks
+    uint8_t *rm = nullptr;
+    CG_TRY(row_mask(C, P.nf1, P.nf2, rm));
+    GridArgs g = grid_args(C, P, t, M, a.cshift);
+    g.kr = key_rect(a);
+    g.dense_min = cp.dense_min;
+    CG_TRY(grid_masks<T>(C, g, rm, P.nf1, P.nf2));
+    WArgs w = make_wargs(P);
+    CG_TRY(image_tables(C, P));
+    CallClear clr{rm, rm ? P.nf1 + P.nf2 : 0, {g.tile_list}};
+    if (cp.dense_min > 0) {
+        CG_TRY(ensure(C.dlist, sizeof(int32_t) * dense_list_ints(t.ntiles(), g.m)));
+        clr.counter[1] = as<int32_t>(C.dlist);
+        clr.counter[2] = as<int32_t>(C.dlist) + 1;
+    }
+    CG_TRY(launch_call_setup(w, as<double>(C.phi1), as<double>(C.phi2), P.wstack ? as<double>(C.zq) : nullptr,
+                             as<double>(C.phi3), clr, C.stream));
     // complex64: the key pass writes the caller-order records too, and the
     // record stage only gathers them
     float4 *rec = nullptr;
     if (M > 0) {
         if constexpr (sizeof(T) == 4 && std::is_same<TW, float>::value) {
             CG_TRY(records_scratch<T>(C, slab_bytes(P, cp.slab, eb), M, 0, rec));
-            if (rec) CG_TRY(sort_rows<TU>(C, uvw, M, a, t, (const float2 *)vis, wgt, rec));
+            if (rec) CG_TRY(sort_rows<TU>(C, uvw, M, a, t, rm, (const float2 *)vis, wgt, rec));
         }
-        if (!rec) CG_TRY(sort_rows<TU>(C, uvw, M, a, t));
+        if (!rec) CG_TRY(sort_rows<TU>(C, uvw, M, a, t, rm));
     } else {
         CG_TRY(ensure(C.tstart, sizeof(int32_t) * (t.ntiles() + 1)));
         CG_TRY(launch_fill_i32(as<int32_t>(C.tstart), t.ntiles() + 1, 0, C.stream));
@@ -601,21 +649,6 @@ static int exec_ms2dirty(Ctx &C, const CallPlan &cp, const TU *uvw, const cx_t<T
                                                     C.stream)));
     CG_TRY(clk.mark(ST_GRID));
     CG_TRY(ensure(C.grid, slab_bytes(P, cp.slab, eb)));
-    const uint8_t *rm = nullptr;
-    CG_TRY(row_mask(C, t, P.conv.kw, P.nf1, P.nf2, rm));
-    GridArgs g = grid_args(C, P, t, M, a.cshift);
-    g.kr = key_rect(a);
-    g.dense_min = cp.dense_min;
-    CG_TRY(grid_masks<T>(C, g, rm, P.nf1, P.nf2));
-    // correction factors and the quarter tables, for the image stage
-    WArgs w = make_wargs(P);
-    CG_TRY(ensure(C.phi1, sizeof(double) * (P.nf1 / 2 + 1)));
-    CG_TRY(ensure(C.phi2, sizeof(double) * (P.nf2 / 2 + 1)));
-    const int64_t nq = (int64_t)(P.N1 / 2 + 1) * (P.N2 / 2 + 1);
-    if (P.wstack) {
-        CG_TRY(ensure(C.zq, sizeof(double) * nq));
-        CG_TRY(ensure(C.phi3, sizeof(double) * nq));
-    }
     CG_TRY(twiddles<T>(C, P.nf1, P.nf2));
     // only the columns holding image pixels are transformed along n2, only
     // the rows points reach hold non-zero data, and only the frequencies of
@@ -644,7 +677,6 @@ static int exec_ms2dirty(Ctx &C, const CallPlan &cp, const TU *uvw, const cx_t<T
             CG_TRY(launch_grid<T>(as<geo_t<T>>(C.geo), as<cx_t<T>>(C.val), as<int32_t>(C.tstart),
                                   as<cx_t<T>>(C.grid), g, P.conv.kw, C.stream));
         if (cp.dense_min > 0) {
-            CG_TRY(ensure(C.dlist, sizeof(int32_t) * dense_list_ints(t.ntiles(), g.m)));
             CG_TRY(clk.mark(ST_COUNT + 1));
             CG_TRY(launch_grid_dense((const geo_t<float> *)C.geo.p, (const cx_t<float> *)C.val.p,
                                      as<uint32_t>(C.keys), as<int32_t>(C.tstart), as<int32_t>(C.dlist),
@@ -663,11 +695,6 @@ static int exec_ms2dirty(Ctx &C, const CallPlan &cp, const TU *uvw, const cx_t<T
                                   C.band_fft ? P.band_len : 0));
         if (C.stop_after == 2) return P.ier;
         if (!cp.slab) CG_TRY(clk.mark(ST_IMAGE));
-        if (zb == 0) {
-            CG_TRY(launch_fseries_grid(w.qd, P.nf1, as<double>(C.phi1), C.stream));
-            CG_TRY(launch_fseries_grid(w.qd, P.nf2, as<double>(C.phi2), C.stream));
-            if (P.wstack) CG_TRY(launch_quarter_table(w, as<double>(C.zq), as<double>(C.phi3), C.stream));
-        }
         if (!P.wstack) {
             // plain 2-D: the u/v deconvolution only (deconv_2d type 1)
             CG_TRY((launch_deconv2d<T, cx_t<T>>(as<cx_t<T>>(C.grid), dirty, as<double>(C.phi1),
@@ -763,7 +790,28 @@ static int exec_dirty2ms(Ctx &C, const CallPlan &cp, const TU *uvw, cx_t<T> *vis
     C.last_m = M;
     C.last_cshift = a.cshift;
     CG_TRY(clk.mark(ST_SORT));
-    if (M > 0) CG_TRY(sort_rows<TU>(C, uvw, M, a, t));
+    // the call's tables and cleared masks and lists, before the sort fills the
+    // masks; the degridder reads only the rows its tiles' points reach
+    uint8_t *rm = nullptr;
+    if (M > 0) CG_TRY(row_mask(C, P.nf1, P.nf2, rm));
+    GridArgs g = grid_args(C, P, t, M, a.cshift);
+    g.kr = key_rect(a);
+    WArgs w = make_wargs(P);
+    CG_TRY(image_tables(C, P));
+    CallClear clr{rm, rm ? P.nf1 + P.nf2 : 0, {}};
+    DegridLists L{};
+    if (M > 0) {
+        CG_TRY(ensure(C.dlist, sizeof(int32_t) * degrid_list_ints(t.ntiles(), g.m, kw)));
+        L = degrid_lists(g, kw, as<int32_t>(C.dlist));
+        int n = 0;
+        for (int32_t *list : {L.direct, L.staged, L.dense}) {
+            clr.counter[n++] = list;
+            clr.counter[n++] = list + 1;
+        }
+    }
+    CG_TRY(launch_call_setup(w, as<double>(C.phi1), as<double>(C.phi2), P.wstack ? as<double>(C.zq) : nullptr,
+                             as<double>(C.phi3), clr, C.stream));
+    if (M > 0) CG_TRY(sort_rows<TU>(C, uvw, M, a, t, rm));
     CG_TRY(clk.mark(ST_RECORDS));
     CG_TRY(ensure(C.geo, sizeof(geo_t<T>) * M));
     CG_TRY(ensure(C.val, sizeof(cx_t<T>) * M));
@@ -772,21 +820,8 @@ static int exec_dirty2ms(Ctx &C, const CallPlan &cp, const TU *uvw, cx_t<T> *vis
     CG_TRY((launch_records<T, TU, cx_t<T>, TW>(uvw, (const cx_t<T> *)nullptr, wgt,
                                                 as<int32_t>(C.vals), M, a, 1, as<geo_t<T>>(C.geo),
                                                 as<cx_t<T>>(C.val), rec, C.stream)));
-    CG_TRY(ensure(C.phi1, sizeof(double) * (P.nf1 / 2 + 1)));
-    CG_TRY(ensure(C.phi2, sizeof(double) * (P.nf2 / 2 + 1)));
     CG_TRY(ensure(C.grid, slab_bytes(P, cp.slab, eb)));
-    WArgs w = make_wargs(P);
-    const int64_t nq = (int64_t)(P.N1 / 2 + 1) * (P.N2 / 2 + 1);
-    if (P.wstack) {
-        CG_TRY(ensure(C.zq, sizeof(double) * nq));
-        CG_TRY(ensure(C.phi3, sizeof(double) * nq));
-    }
     CG_TRY(twiddles<T>(C, P.nf1, P.nf2));
-    // the degridder reads only the rows its tiles' points reach
-    const uint8_t *rm = nullptr;
-    if (M > 0) CG_TRY(row_mask(C, t, kw, P.nf1, P.nf2, rm));
-    GridArgs g = grid_args(C, P, t, M, a.cshift);
-    g.kr = key_rect(a);
     // columns first (only those holding image pixels; frequencies outside
     // the image rows are zero), then the rows the degridder reads
     const int la = P.N1 - P.N1 / 2, lb = P.nf1 - P.N1 / 2;
@@ -798,9 +833,6 @@ static int exec_dirty2ms(Ctx &C, const CallPlan &cp, const TU *uvw, cx_t<T> *vis
     C.last_slab = cp.slab;
     C.last_nslab = (P.nf3 + per - 1) / per;
     CG_TRY(clk.mark(ST_IMAGE));
-    CG_TRY(launch_fseries_grid(w.qd, P.nf1, as<double>(C.phi1), C.stream));
-    CG_TRY(launch_fseries_grid(w.qd, P.nf2, as<double>(C.phi2), C.stream));
-    if (P.wstack) CG_TRY(launch_quarter_table(w, as<double>(C.zq), as<double>(C.phi3), C.stream));
     if (cp.slab) {
         // the whole loop is reported as the grid stage
         CG_TRY(clk.mark(ST_FFT2));
@@ -843,10 +875,7 @@ static int exec_dirty2ms(Ctx &C, const CallPlan &cp, const TU *uvw, cx_t<T> *vis
             g.dense_min = C.degrid_dense_min;
         if (M > 0) {
             const int below = degrid_direct_below(P, t, M);
-            DegridLists L{};
-            CG_TRY(ensure(C.dlist, sizeof(int32_t) * degrid_list_ints(t.ntiles(), g.m, kw)));
-            CG_TRY(launch_degrid_lists(as<int32_t>(C.tstart), g, kw, below, as<int32_t>(C.dlist), L,
-                                       C.stream));
+            CG_TRY(launch_degrid_lists(as<int32_t>(C.tstart), g, kw, below, L, zb > 0, C.stream));
             if (below > 1)
                 CG_TRY(launch_degrid_direct<T>(as<geo_t<T>>(C.geo), as<cx_t<T>>(C.val),
                                                as<int32_t>(C.vals), as<int32_t>(C.tstart),
@@ -1197,6 +1226,24 @@ int nufft2d_dev(Ctx &C, int type, int64_t M, const TU *x, const TU *y, cx_t<T> *
     const int64_t ntiles = t.ntiles();
     CG_TRY(clk.mark(ST_SORT));
     CG_TRY(ensure(C.tstart, sizeof(int32_t) * (ntiles + 1)));
+    // the correction factors and the cleared masks and list, before the sort
+    // fills the masks
+    uint8_t *rm = nullptr;
+    CG_TRY(row_mask(C, P.nf1, P.nf2, rm));
+    GridArgs g = grid_args(C, P, t, M, a.cshift);
+    g.kr = key_rect(a);
+    g.mfma2d = C.mfma2d;
+    if (type == 1) CG_TRY(grid_masks<T>(C, g, rm, P.nf1, P.nf2));
+    CG_TRY(ensure(C.phi1, sizeof(double) * (P.nf1 / 2 + 1)));
+    CG_TRY(ensure(C.phi2, sizeof(double) * (P.nf2 / 2 + 1)));
+    {
+        WArgs w{};
+        w.nf1 = P.nf1;
+        w.nf2 = P.nf2;
+        w.qd = make_quad(conv);
+        CG_TRY(launch_call_setup(w, as<double>(C.phi1), as<double>(C.phi2), nullptr, nullptr,
+                                 CallClear{rm, rm ? P.nf1 + P.nf2 : 0, {g.tile_list}}, C.stream));
+    }
     // complex64 with FP32 coordinates: the key pass also writes the caller-order
     // records into the grid buffer, which is idle until gridding / deconvolution
     float4 *rec = nullptr;
@@ -1230,7 +1277,7 @@ int nufft2d_dev(Ctx &C, int type, int64_t M, const TU *x, const TU *y, cx_t<T> *
         CG_TRY(launch_radix_sort(k0, v0, k1, v1, M, bits, as<int32_t>(C.hist), hs,
                                  as<int32_t>(C.scan), C.stream, 0, 1));
         CG_TRY(launch_tile_bounds(as<uint32_t>(C.keys), M, ntiles, a.cshift, key_rect(a),
-                                  as<int32_t>(C.tstart), C.stream));
+                                  as<int32_t>(C.tstart), tile_mask(rm, t, kw, P.nf1, P.nf2), C.stream));
     } else {
         CG_TRY(launch_fill_i32(as<int32_t>(C.tstart), ntiles + 1, 0, C.stream));
     }
@@ -1245,23 +1292,12 @@ int nufft2d_dev(Ctx &C, int type, int64_t M, const TU *x, const TU *y, cx_t<T> *
                                                   as<int32_t>(C.vals), M, a, as<geo_t<T>>(C.geo),
                                                   as<cx_t<T>>(C.val), C.stream)));
     CG_TRY(ensure(C.grid, (size_t)P.nf1 * P.nf2 * eb));
-    CG_TRY(ensure(C.phi1, sizeof(double) * (P.nf1 / 2 + 1)));
-    CG_TRY(ensure(C.phi2, sizeof(double) * (P.nf2 / 2 + 1)));
-    Quad qd = make_quad(conv);
-    CG_TRY(launch_fseries_grid(qd, P.nf1, as<double>(C.phi1), C.stream));
-    CG_TRY(launch_fseries_grid(qd, P.nf2, as<double>(C.phi2), C.stream));
     CG_TRY(twiddles<T>(C, P.nf1, P.nf2));
-    GridArgs g = grid_args(C, P, t, M, a.cshift);
-    g.kr = key_rect(a);
-    g.mfma2d = C.mfma2d;
     // fast-axis columns that hold modes; grid rows that points reach; mode
     // frequencies along nf2
     const int la = N1 - N1 / 2, lb = P.nf1 - N1 / 2;
     const int sa = N2 - N2 / 2, sb = P.nf2 - N2 / 2;
-    const uint8_t *rm = nullptr;
-    CG_TRY(row_mask(C, t, kw, P.nf1, P.nf2, rm));
     if (type == 1) {
-        CG_TRY(grid_masks<T>(C, g, rm, P.nf1, P.nf2));
         CG_TRY(clk.mark(ST_GRID));
         CG_TRY(launch_grid<T>(as<geo_t<T>>(C.geo), as<cx_t<T>>(C.val), as<int32_t>(C.tstart),
                               as<cx_t<T>>(C.grid), g, kw, C.stream));
@@ -1610,6 +1646,7 @@ int cg_ctx_create(void **ctx, void *stream)
     try {
         Ctx *C = new Ctx();
         C->stream = (hipStream_t)stream;
+        C->keep_pinned = true;
         env_overrides(*C);
         *ctx = C;
         return CG_OK;

@@ -67,8 +67,6 @@ __device__ __forceinline__ Span tile_span(int r, int t, int n)
 // most source bins feeding one tile: (1 + ceil(15/2))^2 for tiles >= 2
 constexpr int kMaxBins = 81;
 
-__global__ void k_zero_i32(int32_t *p, int64_t second);
-
 template <typename T, int KW>
 __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
                                                const cx_t<T> *__restrict__ val,
@@ -380,8 +378,6 @@ static int grid_kw(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *ts, c
     unsigned nblk = (unsigned)ntiles;
     if (g.tile_list) {
         // build the list of tiles to write; workgroups then walk it
-        hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, const_cast<int32_t *>(g.tile_list),
-                           (int64_t)0);
         hipLaunchKernelGGL(k_need_tiles, dim3((unsigned)ceil_div(ntiles, 256)), dim3(256), 0, s,
                            g.rowmask, g.colmask, g.ntx, ntiles, g.tx, g.ty,
                            const_cast<int32_t *>(g.tile_list));
@@ -454,14 +450,6 @@ int dense_chunk(int64_t m)
 int64_t dense_list_ints(int64_t ntiles, int64_t m)
 {
     return 2 + 2 * (ntiles + (m + dense_chunk(m) - 1) / dense_chunk(m));
-}
-
-__global__ void k_zero_i32(int32_t *p, int64_t second)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        p[0] = 0;
-        p[second] = 0;
-    }
 }
 
 // Dense bins, second form.  A workgroup takes work units (k_dense_bins: a
@@ -869,7 +857,6 @@ static int grid_dense2_kw(const float4 *geo, const float2 *val, const uint32_t *
     const int64_t ntiles = (int64_t)g.ntx * g.nty;
     const int chunk = dense_chunk(g.m);
     const int64_t units = ntiles + ceil_div((int64_t)g.m, (int64_t)chunk);
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, list, 1);
     hipLaunchKernelGGL(k_dense_bins, dim3((unsigned)ceil_div(ntiles, 256)), dim3(256), 0, s, ts,
                        ntiles, g.dense_min, chunk, list);
     CG_HIP(hipGetLastError());
@@ -968,15 +955,22 @@ int64_t degrid_list_ints(int64_t ntiles, int64_t m, int kw)
     return 2 + 2 * direct_units(ntiles, m, kw) + 2 + ntiles + dense_list_ints(ntiles, m);
 }
 
-int launch_degrid_lists(const int32_t *ts, const GridArgs &g, int kw, int below, int32_t *buf,
-                        DegridLists &L, hipStream_t s)
+DegridLists degrid_lists(const GridArgs &g, int kw, int32_t *buf)
 {
     const int64_t ntiles = (int64_t)g.ntx * g.nty;
+    DegridLists L;
     L.max_direct = direct_units(ntiles, g.m, kw);
     L.direct = buf;
     L.staged = L.direct + 2 + 2 * L.max_direct;
     L.dense = L.staged + 2 + ntiles;
-    hipLaunchKernelGGL(k_zero_lists, dim3(1), dim3(64), 0, s, L);
+    return L;
+}
+
+int launch_degrid_lists(const int32_t *ts, const GridArgs &g, int kw, int below, const DegridLists &L,
+                        bool clear, hipStream_t s)
+{
+    const int64_t ntiles = (int64_t)g.ntx * g.nty;
+    if (clear) hipLaunchKernelGGL(k_zero_lists, dim3(1), dim3(64), 0, s, L);
     hipLaunchKernelGGL(k_tile_units, dim3((unsigned)ceil_div(ntiles, 256)), dim3(256), 0, s, ts, ntiles,
                        below, degrid_direct_unit(kw), g.dense_min, dense_chunk(g.m), L);
     CG_HIP(hipGetLastError());

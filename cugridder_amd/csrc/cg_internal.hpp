@@ -55,10 +55,12 @@ int sort_key_bits(const CoordArgs &a, int64_t ntiles);
 // ---- prep (cg_prep.hip)
 // min/max of w * scale_w (FP64) over nrow rows of uvw [nrow][3], and
 // uv[4] = {umin, umax, vmin, vmax} when uv is given; partial buffer needs
-// 6150 doubles.  Results copied to host (synchronises).
+// 6151 doubles, the last one 0 (and 0 again afterwards).  The results go to
+// host (6 doubles of pinned memory) or, without it, are copied; synchronises.
 template <typename TU>
 int launch_wminmax(const TU *uvw, int64_t nrow, double scale_w, double *d_part,
-                   double &wmin, double &wmax, hipStream_t s, double *uv = nullptr);
+                   double &wmin, double &wmax, hipStream_t s, double *uv = nullptr,
+                   double *host = nullptr);
 // keys[j] = (tile of the footprint start of row j) << cshift | start cell
 // inside the tile; vals[j] = j (vals may be null)
 template <typename TU>
@@ -70,15 +72,17 @@ int launch_keys_xy(const TU *x, const TU *y, int64_t m, const CoordArgs &a,
                    uint32_t *keys, int32_t *vals, hipStream_t s);
 // p[0..n) = v (a kernel, so that it can sit in a captured graph)
 int launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t s);
-// mask[y] (y < nf2) = 1 for the grid rows and mask[nf2 + x] (x < nf1) = 1
-// for the grid columns that points of non-empty tiles reach; other rows and
-// columns are zero after gridding and unread by degridding
-int launch_row_mask(const int32_t *tile_start, const Tiling &t, int kw, int nf1, int nf2,
-                    uint8_t *mask, hipStream_t s);
-// tile_start[t] = first sorted position with key >> shift >= t, t in [0, ntiles]
+// tile_start[t] = first sorted position with key >> shift >= t, t in [0, ntiles].
+// With K.mask (nf2 + nf1 bytes, zero on entry), mask[y] (y < nf2) = 1 for the
+// grid rows and mask[nf2 + x] (x < nf1) = 1 for the grid columns that points of
+// non-empty tiles reach; other rows and columns are zero after gridding and
+// unread by degridding
+struct TileMask {
+    uint8_t *mask;
+    int ntx, tx, ty, kw, nf1, nf2;
+};
 int launch_tile_bounds(const uint32_t *sorted_keys, int64_t m, int64_t ntiles, int shift,
-                       const KeyRect &kr,
-                       int32_t *tile_start, hipStream_t s);
+                       const KeyRect &kr, int32_t *tile_start, const TileMask &K, hipStream_t s);
 
 // Sorted point records: geo = {d1, d2, d3, packed(lx | ly<<8 | z0<<16)} and a
 // complex value (ms2dirty: vis*wgt*e^{i o_c w}; dirty2ms: wgt*e^{-i o_c w}).
@@ -150,7 +154,8 @@ struct GridArgs {
     double beta, es_c;
     // tiles whose rows all have rowmask 0, or whose columns all have
     // colmask 0, are not written (null: every tile is written); the sparse
-    // gridder then collects the others in tile_list (ntiles + 1 ints)
+    // gridder then collects the others in tile_list (ntiles + 1 ints, the
+    // first 0)
     const uint8_t *rowmask, *colmask;
     int32_t *tile_list;
     // learned kernel (learned != 0): the value at offset d is
@@ -183,7 +188,8 @@ __host__ __device__ inline int slab_planes(const GridArgs &g) { return g.zn > 0 
 bool grid2d_mfma_supported(const GridArgs &g, int kw);
 // W-stacking (nf3 >= 2 kw planes; any sort tiles of at least two cells):
 // every bin below dense_min, in FP64 registers (cg_sparse.hip).  tile_list
-// needs sparse_blocks + 1 ints.
+// needs sparse_blocks + 1 ints, the first of them 0 on entry of the call whose
+// slab starts at plane 0; it builds the list, the other slabs' calls use it.
 int64_t sparse_blocks(int nf1, int nf2);
 template <typename T>
 int launch_grid_sparse(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *tile_start,
@@ -202,13 +208,15 @@ int launch_degrid(const geo_t<T> *geo, const cx_t<T> *fac, const int32_t *perm,
 // launch_degrid, from g.dense_min points (> 0) units for
 // launch_degrid_dense.  buf needs degrid_list_ints ints.
 struct DegridLists {
-    int32_t *direct, *staged, *dense;
+    int32_t *direct, *staged, *dense;  // [0] and [1] of each are counters
     int64_t max_direct;
 };
 int degrid_direct_unit(int kw);
 int64_t degrid_list_ints(int64_t ntiles, int64_t m, int kw);
-int launch_degrid_lists(const int32_t *tile_start, const GridArgs &g, int kw, int below, int32_t *buf,
-                        DegridLists &L, hipStream_t s);
+DegridLists degrid_lists(const GridArgs &g, int kw, int32_t *buf);
+// clear: the counters are not zero yet
+int launch_degrid_lists(const int32_t *tile_start, const GridArgs &g, int kw, int below,
+                        const DegridLists &L, bool clear, hipStream_t s);
 // points read straight from the planes (cg_sparse.hip)
 template <typename T>
 int launch_degrid_direct(const geo_t<T> *geo, const cx_t<T> *fac, const int32_t *perm,
@@ -218,7 +226,7 @@ int grid_lds_bytes(const GridArgs &g, int elem);
 // Dense bins (fp32, kw <= 8, nf3 <= 32, cshift > 0): the sparse kernel
 // launched with g.dense_min > 0 leaves them out; this adds them to fw with
 // per-start-cell MFMA products.  list needs dense_list_ints(ntiles, g.m)
-// ints of scratch.  The dense kernels' work units are chunks of at most
+// ints of scratch, the first two 0.  The dense kernels' work units are chunks of at most
 // dense_chunk(g.m) sorted points of one bin.
 int dense_chunk(int64_t m);
 int64_t dense_list_ints(int64_t ntiles, int64_t m);
@@ -295,10 +303,6 @@ struct Quad {
 };
 constexpr int kChebMax = 96;
 Quad make_quad(const ConvOpts &o);
-// phi[k] = 2 sum_i g_i cos(pi k (x_i - N + 1)/(N - 1)), N = nf/2 + 1
-// (src/fourier/deconv.cu:12-26), k in [0, nf/2]
-int launch_fseries_grid(const Quad &q, int nf, double *phi, hipStream_t s);
-
 struct WArgs {
     int N1, N2, nf1, nf2, nf3;
     int cna, cnb;  // split of the column axis (0: natural order)
@@ -316,8 +320,18 @@ struct WArgs {
     double cheb[kChebMax];
 };
 WArgs make_wargs(const WPlan &p);
-// z' and psihat(z') on the (N2/2+1) x (N1/2+1) quarter image
-int launch_quarter_table(const WArgs &w, double *zq, double *phi3, hipStream_t s);
+// what a call clears before it starts (the counters of its work lists)
+struct CallClear {
+    static constexpr int kCounters = 8;
+    uint8_t *mask;
+    int mask_bytes;
+    int32_t *counter[kCounters];  // null: none
+};
+// phi1, phi2: Fourier coefficients of the kernel on [0, nf/2] of the two axes;
+// zq, phi3 (unless null): z' and psihat(z') on the (N2/2+1) x (N1/2+1) quarter
+// image; clears clr.  Only qd, nf1 and nf2 of w are used without zq.
+int launch_call_setup(const WArgs &w, double *phi1, double *phi2, double *zq, double *phi3,
+                      const CallClear &clr, hipStream_t s);
 // ms2dirty epilogue: w-DFT over planes + deconvolution + w-correction + 1/n
 template <typename T, typename TV>
 int launch_ms2dirty_epilogue(const cx_t<T> *fw, const double *zq, const double *phi3,

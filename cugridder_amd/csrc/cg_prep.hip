@@ -135,12 +135,16 @@ __device__ __forceinline__ uint32_t tile_key(const Foot &f, const CoordArgs &a)
 // ------------------------------------------------------------ w min/max
 
 // min/max of w * scale_w, of u and of v over the rows: part[1024 q + block]
-// for q = wmin, wmax, umin, umax, vmin, vmax; finals at part[6144 + q]
+// for q = wmin, wmax, umin, umax, vmin, vmax; the last block to finish (count,
+// 0 before and after) reduces them to out[q], in host memory or part + 6144.
+// One launch and no copy: with a second reduction kernel and a copy the range
+// of 2000 rows took 12 us of kernels.
 template <typename TU>
 __global__ __launch_bounds__(256) void k_wminmax(const TU *uvw, int64_t nrow, double scale_w,
-                                                 double *part)
+                                                 double *part, unsigned *count, double *out)
 {
     __shared__ double sv[6][256];
+    __shared__ bool last;
     double r[6] = {INFINITY, -INFINITY, INFINITY, -INFINITY, INFINITY, -INFINITY};
     for (int64_t j = blockIdx.x * (int64_t)256 + threadIdx.x; j < nrow; j += (int64_t)gridDim.x * 256) {
         const double w = (double)uvw[3 * j + 2] * scale_w;
@@ -152,42 +156,49 @@ __global__ __launch_bounds__(256) void k_wminmax(const TU *uvw, int64_t nrow, do
         r[4] = fmin(r[4], v);
         r[5] = fmax(r[5], v);
     }
+    auto reduce = [&] {
 #pragma unroll
-    for (int q = 0; q < 6; q++) sv[q][threadIdx.x] = r[q];
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
+        for (int q = 0; q < 6; q++) sv[q][threadIdx.x] = r[q];
+        __syncthreads();
+        for (int s = 128; s > 0; s >>= 1) {
+            if ((int)threadIdx.x < s) {
 #pragma unroll
-            for (int q = 0; q < 6; q++)
-                sv[q][threadIdx.x] = (q & 1) ? fmax(sv[q][threadIdx.x], sv[q][threadIdx.x + s])
-                                             : fmin(sv[q][threadIdx.x], sv[q][threadIdx.x + s]);
+                for (int q = 0; q < 6; q++)
+                    sv[q][threadIdx.x] = (q & 1) ? fmax(sv[q][threadIdx.x], sv[q][threadIdx.x + s])
+                                                 : fmin(sv[q][threadIdx.x], sv[q][threadIdx.x + s]);
+            }
+            __syncthreads();
+        }
+    };
+    reduce();
+    if (gridDim.x > 1) {
+        if (threadIdx.x < 6) {
+            part[1024 * threadIdx.x + blockIdx.x] = sv[threadIdx.x][0];
+            __threadfence();  // the partials before the count
         }
         __syncthreads();
-    }
-    if (threadIdx.x < 6) part[1024 * threadIdx.x + blockIdx.x] = sv[threadIdx.x][0];
-}
-
-__global__ __launch_bounds__(1024) void k_minmax_final(double *part, int nb)
-{
-    __shared__ double sv[6][1024];
-    int t = threadIdx.x;
-#pragma unroll
-    for (int q = 0; q < 6; q++) sv[q][t] = t < nb ? part[1024 * q + t] : ((q & 1) ? -INFINITY : INFINITY);
-    __syncthreads();
-    for (int s = 512; s > 0; s >>= 1) {
-        if (t < s) {
-#pragma unroll
-            for (int q = 0; q < 6; q++)
-                sv[q][t] = (q & 1) ? fmax(sv[q][t], sv[q][t + s]) : fmin(sv[q][t], sv[q][t + s]);
-        }
+        if (threadIdx.x == 0) last = atomicAdd(count, 1u) == gridDim.x - 1;
         __syncthreads();
+        if (!last) return;
+        __threadfence();  // every block's partials after the count
+#pragma unroll
+        for (int q = 0; q < 6; q++) r[q] = (q & 1) ? -INFINITY : INFINITY;
+        for (int t = threadIdx.x; t < (int)gridDim.x; t += 256) {
+#pragma unroll
+            for (int q = 0; q < 6; q++) {
+                const double x = __hip_atomic_load(part + 1024 * q + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                r[q] = (q & 1) ? fmax(r[q], x) : fmin(r[q], x);
+            }
+        }
+        reduce();
+        if (threadIdx.x == 0) *count = 0;
     }
-    if (t < 6) part[6144 + t] = sv[t][0];
+    if (threadIdx.x < 6) out[threadIdx.x] = sv[threadIdx.x][0];
 }
 
 template <typename TU>
 int launch_wminmax(const TU *uvw, int64_t nrow, double scale_w, double *d_part, double &wmin,
-                   double &wmax, hipStream_t s, double *uv)
+                   double &wmax, hipStream_t s, double *uv, double *host)
 {
     if (nrow == 0) {
         wmin = wmax = 0.0;
@@ -195,12 +206,13 @@ int launch_wminmax(const TU *uvw, int64_t nrow, double scale_w, double *d_part, 
         return CG_OK;
     }
     int nb = (int)std::min<int64_t>(1024, ceil_div(nrow, 256));
-    hipLaunchKernelGGL(k_wminmax<TU>, dim3(nb), dim3(256), 0, s, uvw, nrow, scale_w, d_part);
-    hipLaunchKernelGGL(k_minmax_final, dim3(1), dim3(1024), 0, s, d_part, nb);
+    hipLaunchKernelGGL(k_wminmax<TU>, dim3(nb), dim3(256), 0, s, uvw, nrow, scale_w, d_part,
+                       (unsigned *)(d_part + 6150), host ? host : d_part + 6144);
     CG_HIP(hipGetLastError());
     double h[6];
-    CG_HIP(hipMemcpyAsync(h, d_part + 6144, 6 * sizeof(double), hipMemcpyDeviceToHost, s));
+    if (!host) CG_HIP(hipMemcpyAsync(h, d_part + 6144, 6 * sizeof(double), hipMemcpyDeviceToHost, s));
     CG_HIP(hipStreamSynchronize(s));
+    if (host) std::copy(host, host + 6, h);
     wmin = h[0];
     wmax = h[1];
     if (uv) {
@@ -273,10 +285,15 @@ int launch_keys_xy(const TU *x, const TU *y, int64_t m, const CoordArgs &a, uint
 // ------------------------------------------------------------ tile bounds
 
 // start[t] = first sorted position whose tile comes at or after grid tile t
-// (with a compact key map: at or after the first rectangle tile >= t)
-__global__ __launch_bounds__(256) void k_tile_bounds(const uint32_t *keys, int64_t m,
+// (with a compact key map: at or after the first rectangle tile >= t).  With a
+// mask (zero on entry), mask[y] = 1 for every grid row y < nf2 and mask[nf2 + x]
+// = 1 for every grid column x < nf1 that the footprint of a point of a
+// non-empty tile can reach: rows [y0, y0 + ty + kw - 1) of the tile, periodic.
+// All other rows and columns of the grid are zero (ms2dirty) or never read
+// (dirty2ms), so the FFT passes may skip them.
+__global__ __launch_bounds__(256) void k_tile_bounds(const uint32_t *__restrict__ keys, int64_t m,
                                                      int64_t ntiles, int shift, KeyRect kr,
-                                                     int32_t *start)
+                                                     int32_t *__restrict__ start, TileMask K)
 {
     int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x;
     if (t > ntiles) return;
@@ -288,51 +305,31 @@ __global__ __launch_bounds__(256) void k_tile_bounds(const uint32_t *keys, int64
         else hi = mid;
     }
     start[t] = (int32_t)lo;
+    // the tile's own points: keys in [c, number of the next tile)
+    if (!K.mask || t == ntiles || lo == m || (int64_t)(keys[lo] >> shift) >= kr.lower(t + 1, ntiles)) return;
+    const int y0 = (int)(t / K.ntx) * K.ty;
+    const int spany = min(K.ty + K.kw - 1, K.nf2);
+    for (int r = 0; r < spany; r++) {
+        int y = y0 + r;
+        if (y >= K.nf2) y -= K.nf2;
+        K.mask[y] = 1;
+    }
+    const int x0 = (int)(t % K.ntx) * K.tx;
+    const int spanx = min(K.tx + K.kw - 1, K.nf1);
+    for (int r = 0; r < spanx; r++) {
+        int x = x0 + r;
+        if (x >= K.nf1) x -= K.nf1;
+        K.mask[K.nf2 + x] = 1;
+    }
 }
 
 int launch_tile_bounds(const uint32_t *sorted_keys, int64_t m, int64_t ntiles, int shift,
-                       const KeyRect &kr, int32_t *tile_start, hipStream_t s)
+                       const KeyRect &kr, int32_t *tile_start, const TileMask &mask, hipStream_t s)
 {
     hipLaunchKernelGGL(k_tile_bounds, dim3((unsigned)ceil_div(ntiles + 1, 256)), dim3(256), 0, s,
-                       sorted_keys, m, ntiles, shift, kr, tile_start);
+                       sorted_keys, m, ntiles, shift, kr, tile_start, mask);
     CG_HIP(hipGetLastError());
     return CG_OK;
-}
-
-// ------------------------------------------------------------ row mask
-
-// mask[y] = 1 for every grid row y (along nf2) that the footprint of a point
-// of a non-empty tile can reach: rows [y0, y0 + ty + kw - 1) of the tile,
-// periodic.  All other rows of the grid are zero (ms2dirty) or never read
-// (dirty2ms), so the FFT passes may skip them.
-__global__ __launch_bounds__(256) void k_fill_u8(uint8_t *p, int n)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = 0;
-}
-
-// mask[y] (y < nf2) marks the grid rows and mask[nf2 + x] (x < nf1) the
-// grid columns that the footprints of the points of non-empty tiles reach
-__global__ __launch_bounds__(256) void k_row_mask(const int32_t *__restrict__ tile_start,
-                                                  int64_t ntiles, int ntx, int tx, int ty, int kw,
-                                                  int nf1, int nf2, uint8_t *__restrict__ mask)
-{
-    const int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x;
-    if (t >= ntiles || tile_start[t + 1] == tile_start[t]) return;
-    const int y0 = (int)(t / ntx) * ty;
-    const int spany = min(ty + kw - 1, nf2);
-    for (int r = 0; r < spany; r++) {
-        int y = y0 + r;
-        if (y >= nf2) y -= nf2;
-        mask[y] = 1;
-    }
-    const int x0 = (int)(t % ntx) * tx;
-    const int spanx = min(tx + kw - 1, nf1);
-    for (int r = 0; r < spanx; r++) {
-        int x = x0 + r;
-        if (x >= nf1) x -= nf1;
-        mask[nf2 + x] = 1;
-    }
 }
 
 __global__ __launch_bounds__(256) void k_fill_i32(int32_t *p, int64_t n, int32_t v)
@@ -345,18 +342,6 @@ int launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t s)
 {
     if (n <= 0) return CG_OK;
     hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, s, p, n, v);
-    CG_HIP(hipGetLastError());
-    return CG_OK;
-}
-
-int launch_row_mask(const int32_t *tile_start, const Tiling &t, int kw, int nf1, int nf2,
-                    uint8_t *mask, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_fill_u8, dim3((unsigned)ceil_div(nf1 + nf2, 256)), dim3(256), 0, s, mask,
-                       nf1 + nf2);
-    const int64_t ntiles = t.ntiles();
-    hipLaunchKernelGGL(k_row_mask, dim3((unsigned)ceil_div(ntiles, 256)), dim3(256), 0, s, tile_start,
-                       ntiles, t.ntx, t.tx, t.ty, kw, nf1, nf2, mask);
     CG_HIP(hipGetLastError());
     return CG_OK;
 }
@@ -638,8 +623,8 @@ int launch_records_xy(const TU *x, const TU *y, const TV *c, const int32_t *perm
 }
 
 // explicit instantiations
-template int launch_wminmax<float>(const float *, int64_t, double, double *, double &, double &, hipStream_t, double *);
-template int launch_wminmax<double>(const double *, int64_t, double, double *, double &, double &, hipStream_t, double *);
+template int launch_wminmax<float>(const float *, int64_t, double, double *, double &, double &, hipStream_t, double *, double *);
+template int launch_wminmax<double>(const double *, int64_t, double, double *, double &, double &, hipStream_t, double *, double *);
 template int launch_keys<float>(const float *, int64_t, const CoordArgs &, uint32_t *, int32_t *, hipStream_t);
 template int launch_keys<double>(const double *, int64_t, const CoordArgs &, uint32_t *, int32_t *, hipStream_t);
 template int launch_keys_xy<float>(const float *, const float *, int64_t, const CoordArgs &, uint32_t *, int32_t *, hipStream_t);

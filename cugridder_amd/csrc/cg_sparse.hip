@@ -333,8 +333,7 @@ int launch_grid_sparse(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *t
     const int nbx = (int)ceil_div(g.nf1, kBlk);
     const int64_t nblocks = sparse_blocks(g.nf1, g.nf2);
     const int nwin = (int)ceil_div(slab_planes(g), kWin);
-    if (g.tile_list) {
-        CG_TRY(launch_fill_i32(g.tile_list, 1, 0, s));
+    if (g.tile_list && g.zb == 0) {
         hipLaunchKernelGGL(k_need_blocks, dim3((unsigned)ceil_div(nblocks, 256)), dim3(256), 0, s,
                            g.rowmask, g.colmask, nbx, (int)nblocks, g.nf1, g.nf2, g.tile_list);
         CG_HIP(hipGetLastError());

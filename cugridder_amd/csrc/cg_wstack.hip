@@ -14,6 +14,8 @@
 // the column FFT leaves it (split order for long columns).
 #include <vector>
 
+#include <algorithm>
+
 #include "cg_internal.hpp"
 
 namespace cg {
@@ -134,9 +136,10 @@ Quad make_quad(const ConvOpts &o)
     return q;
 }
 
-__global__ __launch_bounds__(256) void k_fseries_grid(Quad qd, int nf, double *phi)
+// phi[k] = 2 sum_i g_i cos(pi k (x_i - N + 1)/(N - 1)), N = nf/2 + 1
+// (src/fourier/deconv.cu:12-26), k in [0, nf/2]
+__device__ __forceinline__ void fseries_at(const Quad &qd, int nf, int k, double *phi)
 {
-    const int k = blockIdx.x * 256 + threadIdx.x;
     const int N = nf / 2 + 1;
     if (k >= N) return;
     double s = 0.0;
@@ -144,22 +147,14 @@ __global__ __launch_bounds__(256) void k_fseries_grid(Quad qd, int nf, double *p
     phi[k] = 2.0 * s;
 }
 
-int launch_fseries_grid(const Quad &q, int nf, double *phi, hipStream_t s)
-{
-    const int N = nf / 2 + 1;
-    hipLaunchKernelGGL(k_fseries_grid, dim3((N + 255) / 256), dim3(256), 0, s, q, nf, phi);
-    CG_HIP(hipGetLastError());
-    return CG_OK;
-}
-
-// k_generation (src/astro/precomp.cu:215-225) + pre_stage_2 on z
-// (cuft.cu:102-105) + fourier_series_appro at z' (deconv.cu:49-65)
-__global__ __launch_bounds__(256) void k_quarter(WArgs w, double *zq, double *phi3)
+// z' and psihat(z') on the quarter image: k_generation
+// (src/astro/precomp.cu:215-225) + pre_stage_2 on z (cuft.cu:102-105) +
+// fourier_series_appro at z' (deconv.cu:49-65)
+__device__ __forceinline__ void quarter_at(const WArgs &w, int64_t q, double *zq, double *phi3)
 {
     const int W = w.N1 / 2 + 1, H = w.N2 / 2 + 1;
-    const int q = blockIdx.x * 256 + threadIdx.x;
-    if (q >= W * H) return;
-    const int r = q / W, c = q - r * W;
+    if (q >= (int64_t)W * H) return;
+    const int r = (int)(q / W), c = (int)(q - (int64_t)r * W);
     const double l = r * w.pix_x, m = c * w.pix_y;
     const double t = 1.0 - l * l - m * m;
     // n-1, written without cancellation for t >= 0
@@ -183,10 +178,35 @@ __global__ __launch_bounds__(256) void k_quarter(WArgs w, double *zq, double *ph
     phi3[q] = s;
 }
 
-int launch_quarter_table(const WArgs &w, double *zq, double *phi3, hipStream_t s)
+// Everything of a call that depends on its plan alone, in one launch: the
+// correction factors of the two axes, the quarter image's tables (zq given)
+// and the cleared masks and list counters.  As six kernels these were a
+// quarter of the launches of a small call, whose time is its launches: 2000
+// rows onto 128 x 96 pixels 178 us, with this and the masks set by
+// k_tile_bounds 147 us.
+__global__ __launch_bounds__(256) void k_call_setup(WArgs w, double *phi1, double *phi2, double *zq,
+                                                    double *phi3, CallClear clr, int b1, int b2, int b3)
 {
-    int nq = (w.N1 / 2 + 1) * (w.N2 / 2 + 1);
-    hipLaunchKernelGGL(k_quarter, dim3((nq + 255) / 256), dim3(256), 0, s, w, zq, phi3);
+    const int b = blockIdx.x, t = threadIdx.x;
+    if (b < b1) fseries_at(w.qd, w.nf1, b * 256 + t, phi1);
+    else if (b < b2) fseries_at(w.qd, w.nf2, (b - b1) * 256 + t, phi2);
+    else if (b < b3) {
+        const int i = (b - b2) * 1024 + t * 4;
+        for (int k = i; k < min(i + 4, clr.mask_bytes); k++) clr.mask[k] = 0;
+        if (i < CallClear::kCounters && b == b2)
+            for (int k = i; k < min(i + 4, (int)CallClear::kCounters); k++)
+                if (clr.counter[k]) *clr.counter[k] = 0;
+    } else quarter_at(w, (int64_t)(b - b3) * 256 + t, zq, phi3);
+}
+
+int launch_call_setup(const WArgs &w, double *phi1, double *phi2, double *zq, double *phi3,
+                      const CallClear &clr, hipStream_t s)
+{
+    const int b1 = (w.nf1 / 2 + 1 + 255) / 256, b2 = b1 + (w.nf2 / 2 + 1 + 255) / 256;
+    const int b3 = b2 + std::max(1, (clr.mask_bytes + 1023) / 1024);
+    const int64_t nq = zq ? (int64_t)(w.N1 / 2 + 1) * (w.N2 / 2 + 1) : 0;
+    hipLaunchKernelGGL(k_call_setup, dim3((unsigned)(b3 + ceil_div(nq, 256))), dim3(256), 0, s, w, phi1, phi2,
+                       zq, phi3, clr, b1, b2, b3);
     CG_HIP(hipGetLastError());
     return CG_OK;
 }
