@@ -253,6 +253,10 @@ static TileMask tile_mask(uint8_t *mask, const Tiling &t, int kw, int nf1, int n
     return TileMask{mask, t.ntx, t.tx, t.ty, kw, nf1, nf2};
 }
 
+// Below this many tiles the gridder writes them all: the GPU holds them at once,
+// and the list costs a launch (240 tiles of a 160 x 96 grid: 326 us, listed 348).
+constexpr int kListedTiles = 1024;
+
 // lets the gridder leave the tiles the FFT will not read unwritten, when
 // every pass of this FFT honours the masks (test hook stop_after = 1 keeps
 // the whole grid written)
@@ -262,6 +266,7 @@ static int grid_masks(Ctx &C, GridArgs &g, const uint8_t *mask, int nf1, int nf2
     if (mask && C.stop_after != 1 && fft_rows_masked<T>(nf1) && fft_spectrum_pruned(nf2)) {
         // W-stacking grids are gridded in 8 x 8 blocks, 2-D ones in sort tiles
         const int64_t n = g.nf3 > 1 ? sparse_blocks(nf1, nf2) : (int64_t)g.ntx * g.nty;
+        if (n < kListedTiles) return CG_OK;
         CG_TRY(ensure(C.tlist, sizeof(int32_t) * (size_t)(n + 1)));
         g.rowmask = mask;
         g.colmask = mask + nf2;

@@ -135,10 +135,11 @@ __device__ __forceinline__ uint32_t tile_key(const Foot &f, const CoordArgs &a)
 // ------------------------------------------------------------ w min/max
 
 // min/max of w * scale_w, of u and of v over the rows: part[1024 q + block]
-// for q = wmin, wmax, umin, umax, vmin, vmax; the last block to finish (count,
-// 0 before and after) reduces them to out[q], in host memory or part + 6144.
-// One launch and no copy: with a second reduction kernel and a copy the range
-// of 2000 rows took 12 us of kernels.
+// for q = wmin, wmax, umin, umax, vmin, vmax.  With count (0 before and after)
+// the last block to finish reduces them to out[q], in host memory or part +
+// 6144: one launch, against 12 us of kernels and a copy for 2000 rows.  Each
+// block's fence writes its XCD's L2 back, so that only up to kOneMinmax blocks
+// are reduced so (1024 of them: 33 us, with k_minmax_final 12 us).
 template <typename TU>
 __global__ __launch_bounds__(256) void k_wminmax(const TU *uvw, int64_t nrow, double scale_w,
                                                  double *part, unsigned *count, double *out)
@@ -171,6 +172,10 @@ __global__ __launch_bounds__(256) void k_wminmax(const TU *uvw, int64_t nrow, do
         }
     };
     reduce();
+    if (!count) {
+        if (threadIdx.x < 6) part[1024 * threadIdx.x + blockIdx.x] = sv[threadIdx.x][0];
+        return;
+    }
     if (gridDim.x > 1) {
         if (threadIdx.x < 6) {
             part[1024 * threadIdx.x + blockIdx.x] = sv[threadIdx.x][0];
@@ -196,6 +201,26 @@ __global__ __launch_bounds__(256) void k_wminmax(const TU *uvw, int64_t nrow, do
     if (threadIdx.x < 6) out[threadIdx.x] = sv[threadIdx.x][0];
 }
 
+__global__ __launch_bounds__(1024) void k_minmax_final(const double *part, int nb, double *out)
+{
+    __shared__ double sv[6][1024];
+    int t = threadIdx.x;
+#pragma unroll
+    for (int q = 0; q < 6; q++) sv[q][t] = t < nb ? part[1024 * q + t] : ((q & 1) ? -INFINITY : INFINITY);
+    __syncthreads();
+    for (int s = 512; s > 0; s >>= 1) {
+        if (t < s) {
+#pragma unroll
+            for (int q = 0; q < 6; q++)
+                sv[q][t] = (q & 1) ? fmax(sv[q][t], sv[q][t + s]) : fmin(sv[q][t], sv[q][t + s]);
+        }
+        __syncthreads();
+    }
+    if (t < 6) out[t] = sv[t][0];
+}
+
+constexpr int kOneMinmax = 32;
+
 template <typename TU>
 int launch_wminmax(const TU *uvw, int64_t nrow, double scale_w, double *d_part, double &wmin,
                    double &wmax, hipStream_t s, double *uv, double *host)
@@ -205,9 +230,13 @@ int launch_wminmax(const TU *uvw, int64_t nrow, double scale_w, double *d_part, 
         if (uv) uv[0] = uv[1] = uv[2] = uv[3] = 0.0;
         return CG_OK;
     }
-    int nb = (int)std::min<int64_t>(1024, ceil_div(nrow, 256));
+    // (up to four rows a thread rather than the second launch)
+    const bool one = nrow <= 4 * 256 * kOneMinmax;
+    const int nb = (int)std::min<int64_t>(one ? kOneMinmax : 1024, ceil_div(nrow, 256));
+    double *out = host ? host : d_part + 6144;
     hipLaunchKernelGGL(k_wminmax<TU>, dim3(nb), dim3(256), 0, s, uvw, nrow, scale_w, d_part,
-                       (unsigned *)(d_part + 6150), host ? host : d_part + 6144);
+                       one ? (unsigned *)(d_part + 6150) : nullptr, out);
+    if (!one) hipLaunchKernelGGL(k_minmax_final, dim3(1), dim3(1024), 0, s, d_part, nb, out);
     CG_HIP(hipGetLastError());
     double h[6];
     if (!host) CG_HIP(hipMemcpyAsync(h, d_part + 6144, 6 * sizeof(double), hipMemcpyDeviceToHost, s));

@@ -183,7 +183,7 @@ __device__ __forceinline__ void quarter_at(const WArgs &w, int64_t q, double *zq
 // and the cleared masks and list counters.  As six kernels these were a
 // quarter of the launches of a small call, whose time is its launches: 2000
 // rows onto 128 x 96 pixels 178 us, with this and the masks set by
-// k_tile_bounds 147 us.
+// k_tile_bounds 142 us.
 __global__ __launch_bounds__(256) void k_call_setup(WArgs w, double *phi1, double *phi2, double *zq,
                                                     double *phi3, CallClear clr, int b1, int b2, int b3)
 {
