@@ -171,7 +171,7 @@ def lib():
                  "cg_dirty2ms_px_dev", "cg_batch_create", "cg_batch_run",
                  "cg_batch_info", "cg_batch_destroy",
                  "cg_nufft2d_dev", "cg_nufft2d_noalloc", "cg_plan_query", "cg_ctx_grid", "cg_ctx_sorted",
-                 "cg_fft2d_dev", "cg_sort_pairs_dev", "cg_memcpy_dev", "cg_fft_col_split", "cg_tap_poly",
+                 "cg_fft2d_dev", "cg_sort_pairs_dev", "cg_host_release", "cg_memcpy_dev", "cg_fft_col_split", "cg_tap_poly",
                  "cg_version", "cg_learn_nparams", "cg_learn_grad", "cg_learn_train",
                  "cg_learn_eval", "cg_learn_tabulate", "cg_ctx_set_kernel"):
         getattr(L, name).restype = c_int

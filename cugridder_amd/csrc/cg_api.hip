@@ -16,6 +16,7 @@
 #include <memory>
 #include <mutex>
 #include <new>
+#include <utility>
 #include <type_traits>
 #include <vector>
 
@@ -151,6 +152,90 @@ struct Ctx {
 constexpr size_t kArenaAlign = 256;
 inline size_t arena_round(size_t bytes) { return (bytes + kArenaAlign - 1) / kArenaAlign * kArenaAlign; }
 
+// Device memory of the host entry points, kept between their calls: allocating
+// and freeing gigabytes per call costs more than the call (and the driver clears
+// freed memory at some 30 GB/s, which a program that calls back to back ends up
+// waiting for: 8 ms a call, then 68 ms).  A call leases an idle set of buffers of
+// its device, or starts an empty one, so that threads never share a set.  Returned
+// sets are kept while they hold at most a twelfth of the device's memory together;
+// they are freed by cg_host_release, and when an allocation or a grid does not
+// fit beside them.  Every host call runs on the default stream and returns with
+// it idle.
+struct HostPool {
+    struct Set {
+        int device = 0;
+        size_t bytes = 0;
+        std::vector<std::pair<void *, size_t>> bufs;
+        double *pinned = nullptr;
+        int tw1_n = 0, tw2_n = 0, tw_bytes = 0;  // the twiddle tables held
+    };
+    static constexpr size_t kMostSets = 8;
+    std::mutex m;
+    std::vector<Set> idle;
+
+    static HostPool &get()
+    {
+        // never destroyed: the runtime may be gone when static objects are
+        static HostPool *pool = new HostPool;
+        return *pool;
+    }
+    static void free_set(Set &s)
+    {
+        for (auto &b : s.bufs)
+            if (b.first) (void)hipFree(b.first);
+        if (s.pinned) (void)hipHostFree(s.pinned);
+        s.bufs.clear();
+        s.pinned = nullptr;
+    }
+    Set lease(int device)
+    {
+        std::lock_guard<std::mutex> lock(m);
+        for (size_t i = idle.size(); i-- > 0;)
+            if (idle[i].device == device) {
+                Set s = std::move(idle[i]);
+                idle.erase(idle.begin() + (ptrdiff_t)i);
+                return s;
+            }
+        Set s;
+        s.device = device;
+        return s;
+    }
+    void give_back(Set s, size_t most)
+    {
+        {
+            std::lock_guard<std::mutex> lock(m);
+            size_t held = s.bytes;
+            for (const Set &t : idle)
+                if (t.device == s.device) held += t.bytes;
+            if (held <= most && idle.size() < kMostSets) {
+                idle.push_back(std::move(s));
+                return;
+            }
+        }
+        free_set(s);
+    }
+    // frees the idle sets of a device (-1: of all); true if there were any
+    bool release(int device)
+    {
+        std::vector<Set> gone;
+        {
+            std::lock_guard<std::mutex> lock(m);
+            for (size_t i = idle.size(); i-- > 0;)
+                if (device < 0 || idle[i].device == device) {
+                    gone.push_back(std::move(idle[i]));
+                    idle.erase(idle.begin() + (ptrdiff_t)i);
+                }
+        }
+        for (Set &s : gone) free_set(s);
+        return !gone.empty();
+    }
+};
+static bool release_idle()
+{
+    int device = 0;
+    return hipGetDevice(&device) == hipSuccess && HostPool::get().release(device);
+}
+
 static int ensure(DevBuf &b, size_t bytes)
 {
     if (bytes == 0) bytes = 256;
@@ -173,7 +258,11 @@ static int ensure(DevBuf &b, size_t bytes)
     }
     if (hipMalloc(&b.p, bytes) != hipSuccess) {
         (void)hipGetLastError();
-        return CG_ERR_ALLOC;
+        if (!release_idle() || hipMalloc(&b.p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            b.p = nullptr;
+            return CG_ERR_ALLOC;
+        }
     }
     b.bytes = bytes;
     return CG_OK;
@@ -534,11 +623,17 @@ static int plan_slab(Ctx &C, const WPlan &P, int eb, int64_t M, int &slab)
     if (C.grid_limit_mb > 0) {
         limit = (size_t)C.grid_limit_mb << 20;
     } else {
-        size_t fr = 0, tot = 0;
-        CG_HIP(hipMemGetInfo(&fr, &tot));
-        const size_t avail = fr + C.grid.bytes;
-        const size_t other = (size_t)M * 96 + ((size_t)256 << 20);
-        limit = avail > other ? (size_t)((avail - other) * 0.9) : 0;
+        if (whole <= C.grid.bytes) return CG_OK;  // the buffer at hand holds it
+        auto fits = [&]() -> int {
+            size_t fr = 0, tot = 0;
+            CG_HIP(hipMemGetInfo(&fr, &tot));
+            const size_t avail = fr + C.grid.bytes;
+            const size_t other = (size_t)M * 96 + ((size_t)256 << 20);
+            limit = avail > other ? (size_t)((avail - other) * 0.9) : 0;
+            return CG_OK;
+        };
+        CG_TRY(fits());
+        if (whole > limit && release_idle()) CG_TRY(fits());
     }
     if (whole <= limit) return CG_OK;
     if (plane > limit) return CG_ERR_ALLOC;  // not even one plane fits
@@ -1338,25 +1433,87 @@ int nufft2d_dev(Ctx &C, int type, int64_t M, const TU *x, const TU *y, cx_t<T> *
 
 // ------------------------------------------------------------ host wrappers
 
-struct HostBuf {
-    void *p = nullptr;
-    ~HostBuf()
+// the context and device buffers of one host call, on memory leased from the
+// pool
+struct HostCall {
+    Ctx C;
+    DevBuf in[4];
+    int device = 0;
+
+    int begin()
     {
-        if (p) (void)hipFree(p);
-    }
-    int alloc(size_t bytes)
-    {
-        if (bytes == 0) bytes = 256;
-        if (hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            p = nullptr;
-            return CG_ERR_ALLOC;
-        }
+        env_overrides(C);
+        CG_HIP(hipGetDevice(&device));
+        HostPool::Set s = HostPool::get().lease(device);
+        C.keep_pinned = true;
+        C.pinned = s.pinned;
+        C.tw1_n = s.tw1_n;
+        C.tw2_n = s.tw2_n;
+        C.tw_bytes = s.tw_bytes;
+        size_t i = 0;
+        each([&](DevBuf &b) {
+            if (i < s.bufs.size()) {
+                b.p = s.bufs[i].first;
+                b.bytes = s.bufs[i].second;
+            }
+            i++;
+        });
+        leased = true;
         return CG_OK;
+    }
+    template <typename X>
+    int alloc(int k, size_t count, X *&p)
+    {
+        CG_TRY(ensure(in[k], sizeof(X) * count));
+        p = (X *)in[k].p;
+        return CG_OK;
+    }
+    ~HostCall()
+    {
+        if (!leased) return;
+        // (a call that ended early may have left kernels behind)
+        const bool idle = hipStreamSynchronize(C.stream) == hipSuccess;
+        HostPool::Set s;
+        s.device = device;
+        s.pinned = C.pinned;
+        s.tw1_n = C.tw1_n;
+        s.tw2_n = C.tw2_n;
+        s.tw_bytes = C.tw_bytes;
+        C.pinned = nullptr;
+        try {
+            s.bufs.reserve(64);
+        } catch (const std::bad_alloc &) {
+            if (s.pinned) (void)hipHostFree(s.pinned);
+            each([](DevBuf &b) {
+                if (b.p) (void)hipFree(b.p);
+                b = DevBuf();
+            });
+            return;
+        }
+        each([&](DevBuf &b) {
+            s.bufs.emplace_back(b.p, b.bytes);
+            s.bytes += b.bytes;
+            b = DevBuf();
+        });
+        size_t total = 0;
+        if (!idle || hipDeviceTotalMem(&total, device) != hipSuccess) total = 0;
+        try {
+            HostPool::get().give_back(std::move(s), total / 12);
+        } catch (const std::bad_alloc &) {
+        }
+    }
+
+private:
+    bool leased = false;
+    template <typename F>
+    void each(F f)
+    {
+        C.each_buf(f);
+        for (DevBuf &b : in) f(b);
     }
 };
 
-// host-pointer ms2dirty / dirty2ms: H2D, run, D2H, free (reference semantics);
+// host-pointer ms2dirty / dirty2ms: H2D, run, D2H (reference semantics);
 // vis and wgt are [nrow][nchan] for nchan frequencies freq[nchan]
 template <typename T, typename TU, typename TW>
 static int host_ms2dirty(int nrow, int nchan, const double *freq, int nx, int ny, double fov,
@@ -1366,25 +1523,27 @@ static int host_ms2dirty(int nrow, int nchan, const double *freq, int nx, int ny
     if (nrow < 0 || nchan < 1 || !freq || nx <= 0 || ny <= 0 || !uvw || !dirty || (nrow > 0 && !vis))
         return CG_ERR_ARG;
     try {
-        Ctx C;
-        env_overrides(C);
+        HostCall H;
+        CG_TRY(H.begin());
+        Ctx &C = H.C;
         C.geom = geom;
         const size_t R = (size_t)nrow, M = R * (size_t)nchan;
-        HostBuf du, dv, dw, dd;
-        CG_TRY(du.alloc(sizeof(TU) * 3 * R));
-        CG_TRY(dv.alloc(sizeof(cx_t<T>) * M));
-        if (wgt) CG_TRY(dw.alloc(sizeof(TW) * M));
-        CG_TRY(dd.alloc(sizeof(cx_t<T>) * (size_t)nx * ny));
+        TU *du = nullptr;
+        cx_t<T> *dv = nullptr, *dd = nullptr;
+        TW *dw = nullptr;
+        CG_TRY(H.alloc(0, 3 * R, du));
+        CG_TRY(H.alloc(1, M, dv));
+        if (wgt) CG_TRY(H.alloc(2, M, dw));
+        CG_TRY(H.alloc(3, (size_t)nx * ny, dd));
         if (M) {
-            CG_HIP(hipMemcpy(du.p, uvw, sizeof(TU) * 3 * R, hipMemcpyHostToDevice));
-            CG_HIP(hipMemcpy(dv.p, vis, sizeof(cx_t<T>) * M, hipMemcpyHostToDevice));
-            if (wgt) CG_HIP(hipMemcpy(dw.p, wgt, sizeof(TW) * M, hipMemcpyHostToDevice));
+            CG_HIP(hipMemcpy(du, uvw, sizeof(TU) * 3 * R, hipMemcpyHostToDevice));
+            CG_HIP(hipMemcpy(dv, vis, sizeof(cx_t<T>) * M, hipMemcpyHostToDevice));
+            if (wgt) CG_HIP(hipMemcpy(dw, wgt, sizeof(TW) * M, hipMemcpyHostToDevice));
         }
-        int ier = ms2dirty_dev<T, TU, TW>(C, nrow, nchan, freq, nx, ny, fov, (const TU *)du.p,
-                                          (const cx_t<T> *)dv.p, wgt ? (const TW *)dw.p : nullptr,
-                                          (cx_t<T> *)dd.p, eps, sigma, sign, single);
+        int ier = ms2dirty_dev<T, TU, TW>(C, nrow, nchan, freq, nx, ny, fov, du, dv, dw, dd, eps,
+                                          sigma, sign, single);
         if (ier >= 2) return ier;
-        CG_HIP(hipMemcpy(dirty, dd.p, sizeof(cx_t<T>) * (size_t)nx * ny, hipMemcpyDeviceToHost));
+        CG_HIP(hipMemcpy(dirty, dd, sizeof(cx_t<T>) * (size_t)nx * ny, hipMemcpyDeviceToHost));
         return ier;
     } catch (const std::bad_alloc &) {
         return CG_ERR_ALLOC;
@@ -1399,25 +1558,27 @@ static int host_dirty2ms(int nrow, int nchan, const double *freq, int nx, int ny
     if (nrow < 0 || nchan < 1 || !freq || nx <= 0 || ny <= 0 || !uvw || !dirty || (nrow > 0 && !vis))
         return CG_ERR_ARG;
     try {
-        Ctx C;
-        env_overrides(C);
+        HostCall H;
+        CG_TRY(H.begin());
+        Ctx &C = H.C;
         C.geom = geom;
         const size_t R = (size_t)nrow, M = R * (size_t)nchan;
-        HostBuf du, dv, dw, dd;
-        CG_TRY(du.alloc(sizeof(TU) * 3 * R));
-        CG_TRY(dv.alloc(sizeof(cx_t<T>) * M));
-        if (wgt) CG_TRY(dw.alloc(sizeof(TW) * M));
-        CG_TRY(dd.alloc(sizeof(cx_t<T>) * (size_t)nx * ny));
+        TU *du = nullptr;
+        cx_t<T> *dv = nullptr, *dd = nullptr;
+        TW *dw = nullptr;
+        CG_TRY(H.alloc(0, 3 * R, du));
+        CG_TRY(H.alloc(1, M, dv));
+        if (wgt) CG_TRY(H.alloc(2, M, dw));
+        CG_TRY(H.alloc(3, (size_t)nx * ny, dd));
         if (M) {
-            CG_HIP(hipMemcpy(du.p, uvw, sizeof(TU) * 3 * R, hipMemcpyHostToDevice));
-            if (wgt) CG_HIP(hipMemcpy(dw.p, wgt, sizeof(TW) * M, hipMemcpyHostToDevice));
+            CG_HIP(hipMemcpy(du, uvw, sizeof(TU) * 3 * R, hipMemcpyHostToDevice));
+            if (wgt) CG_HIP(hipMemcpy(dw, wgt, sizeof(TW) * M, hipMemcpyHostToDevice));
         }
-        CG_HIP(hipMemcpy(dd.p, dirty, sizeof(cx_t<T>) * (size_t)nx * ny, hipMemcpyHostToDevice));
-        int ier = dirty2ms_dev<T, TU, TW>(C, nrow, nchan, freq, nx, ny, fov, (const TU *)du.p,
-                                          (cx_t<T> *)dv.p, wgt ? (const TW *)dw.p : nullptr,
-                                          (const cx_t<T> *)dd.p, eps, sigma, sign, single);
+        CG_HIP(hipMemcpy(dd, dirty, sizeof(cx_t<T>) * (size_t)nx * ny, hipMemcpyHostToDevice));
+        int ier = dirty2ms_dev<T, TU, TW>(C, nrow, nchan, freq, nx, ny, fov, du, dv, dw, dd, eps,
+                                          sigma, sign, single);
         if (ier >= 2) return ier;
-        if (M) CG_HIP(hipMemcpy(vis, dv.p, sizeof(cx_t<T>) * M, hipMemcpyDeviceToHost));
+        if (M) CG_HIP(hipMemcpy(vis, dv, sizeof(cx_t<T>) * M, hipMemcpyDeviceToHost));
         return ier;
     } catch (const std::bad_alloc &) {
         return CG_ERR_ALLOC;
@@ -1430,27 +1591,28 @@ static int host_nufft2d(int type, int M, const TU *x, const TU *y, void *c, int 
 {
     if (M < 0 || N1 <= 0 || N2 <= 0 || !fk || (M > 0 && (!x || !y || !c))) return CG_ERR_ARG;
     try {
-        Ctx C;
-        env_overrides(C);
-        HostBuf dx, dy, dc, dk;
-        CG_TRY(dx.alloc(sizeof(TU) * (size_t)M));
-        CG_TRY(dy.alloc(sizeof(TU) * (size_t)M));
-        CG_TRY(dc.alloc(sizeof(cx_t<T>) * (size_t)M));
-        CG_TRY(dk.alloc(sizeof(cx_t<T>) * (size_t)N1 * N2));
+        HostCall H;
+        CG_TRY(H.begin());
+        Ctx &C = H.C;
+        TU *dx = nullptr, *dy = nullptr;
+        cx_t<T> *dc = nullptr, *dk = nullptr;
+        CG_TRY(H.alloc(0, (size_t)M, dx));
+        CG_TRY(H.alloc(1, (size_t)M, dy));
+        CG_TRY(H.alloc(2, (size_t)M, dc));
+        CG_TRY(H.alloc(3, (size_t)N1 * N2, dk));
         if (M) {
-            CG_HIP(hipMemcpy(dx.p, x, sizeof(TU) * (size_t)M, hipMemcpyHostToDevice));
-            CG_HIP(hipMemcpy(dy.p, y, sizeof(TU) * (size_t)M, hipMemcpyHostToDevice));
-            if (type == 1) CG_HIP(hipMemcpy(dc.p, c, sizeof(cx_t<T>) * (size_t)M, hipMemcpyHostToDevice));
+            CG_HIP(hipMemcpy(dx, x, sizeof(TU) * (size_t)M, hipMemcpyHostToDevice));
+            CG_HIP(hipMemcpy(dy, y, sizeof(TU) * (size_t)M, hipMemcpyHostToDevice));
+            if (type == 1) CG_HIP(hipMemcpy(dc, c, sizeof(cx_t<T>) * (size_t)M, hipMemcpyHostToDevice));
         }
         if (type == 2)
-            CG_HIP(hipMemcpy(dk.p, fk, sizeof(cx_t<T>) * (size_t)N1 * N2, hipMemcpyHostToDevice));
-        int ier = nufft2d_dev<T, TU>(C, type, M, (const TU *)dx.p, (const TU *)dy.p,
-                                     (cx_t<T> *)dc.p, N1, N2, (cx_t<T> *)dk.p, eps, sigma, single);
+            CG_HIP(hipMemcpy(dk, fk, sizeof(cx_t<T>) * (size_t)N1 * N2, hipMemcpyHostToDevice));
+        int ier = nufft2d_dev<T, TU>(C, type, M, dx, dy, dc, N1, N2, dk, eps, sigma, single);
         if (ier >= 2) return ier;
         if (type == 1)
-            CG_HIP(hipMemcpy(fk, dk.p, sizeof(cx_t<T>) * (size_t)N1 * N2, hipMemcpyDeviceToHost));
+            CG_HIP(hipMemcpy(fk, dk, sizeof(cx_t<T>) * (size_t)N1 * N2, hipMemcpyDeviceToHost));
         else if (M)
-            CG_HIP(hipMemcpy(c, dc.p, sizeof(cx_t<T>) * (size_t)M, hipMemcpyDeviceToHost));
+            CG_HIP(hipMemcpy(c, dc, sizeof(cx_t<T>) * (size_t)M, hipMemcpyDeviceToHost));
         return ier;
     } catch (const std::bad_alloc &) {
         return CG_ERR_ALLOC;
@@ -2145,6 +2307,13 @@ int cg_sort_pairs_dev(void *ctx, void *d_keys, void *d_vals, int m, int key_bits
     return launch_radix_sort((uint32_t *)d_keys, (int32_t *)d_vals, as<uint32_t>(C->keys2),
                              as<int32_t>(C->vals2), m, key_bits, as<int32_t>(C->hist), hs,
                              as<int32_t>(C->scan), C->stream);
+}
+
+// frees the device memory the host entry points keep between calls
+int cg_host_release(void)
+{
+    HostPool::get().release(-1);
+    return CG_OK;
 }
 
 // device-to-device copy on a stream (test hook)

@@ -315,6 +315,10 @@ int cg_fft2d_dev(void *ctx, int prec, void *d_data, int batch, int n2, int n1,
 int cg_sort_pairs_dev(void *ctx, void *d_keys, void *d_vals, int m,
                       int key_bits);
 
+/* Frees the device memory that the host-pointer entry points keep between
+ * their calls (at most a twelfth of each GPU's memory). */
+int cg_host_release(void);
+
 /* Device-to-device copy of bytes on a HIP stream (test hook). */
 int cg_memcpy_dev(void *dst, const void *src, void *stream, size_t bytes);
 
