@@ -328,8 +328,38 @@ __global__ __launch_bounds__(CB * (1 << LOGL) / 16, CB % 64 == 0 ? 4 : 2) void k
     const int64_t ntile = (int64_t)nx * nsub * batch;
     const int ts = n2 >> LOGL;
     const int b0 = threadIdx.x % CB, e0 = threadIdx.x / CB;
-    auto dead = [&](int j, size_t row, int e) -> bool {
-        if (sj == 1) return rowmask && !rowmask[row];
+    // the mask of a tile's rows as bits, loaded a tile ahead (a byte waited for
+    // before each load of a row made the step on 61 GB of planes 17 instead of
+    // 12 ms)
+    constexpr int W = (L + 63) / 64;
+    struct RowBits {
+        uint64_t w[W];
+    };
+    const bool natural = sj == 1 && rowmask && (mode_in || mode_out);
+    uint8_t ahead[W] = {};
+    auto row_bytes = [&](int64_t t) {
+        if (!natural || t >= ntile) return;
+        const int j = (int)(t / nx % nsub);
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const int e = 64 * w + (threadIdx.x & 63);
+            ahead[w] = e < L ? rowmask[j + e * se] : 0;
+        }
+    };
+    auto row_bits = [&]() -> RowBits {
+        RowBits r;
+#pragma unroll
+        for (int w = 0; w < W; w++) r.w[w] = __ballot(ahead[w] != 0);
+        return r;
+    };
+    auto dead = [&](int j, const RowBits &rows, int e) -> bool {
+        if (natural) {
+            uint64_t w = rows.w[0];
+#pragma unroll
+            for (int k = 1; k < W; k++)
+                if (e >= 64 * k) w = rows.w[k];
+            return !((w >> (e & 63)) & 1);
+        }
         const int k = j + nsub * e;
         return k >= spec_a && k < spec_b;
     };
@@ -337,7 +367,7 @@ __global__ __launch_bounds__(CB * (1 << LOGL) / 16, CB % 64 == 0 ? 4 : 2) void k
     // row (and its mask byte) is wave-uniform and stays in scalar registers
     const int e0w = CB % 64 == 0 ? __builtin_amdgcn_readfirstlane(e0) : e0;
     float2 pre[16];
-    auto load = [&](int64_t t) {
+    auto load = [&](int64_t t, const RowBits &rows) {
         const int x = (int)(t % nx);
         const int64_t r = t / nx;
         const int j = (int)(r % nsub);
@@ -345,18 +375,32 @@ __global__ __launch_bounds__(CB * (1 << LOGL) / 16, CB % 64 == 0 ? 4 : 2) void k
         const size_t row0 = (size_t)j * sj;
         const int c = x * CB + b0;
         const bool cok = c < nlive;
-        const int lc = live.at(c);
+        const int lc = cok ? live.at(c) : 0;
+        // (with every row wanted, no branch between the loads)
+        uint32_t on = 0xffffu;
+        if (mode_in) {
 #pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const int e = e0w + u * R2;
-            const size_t row = row0 + (size_t)e * se;
-            const bool rd = cok && !(mode_in && dead(j, row, e));
-            pre[u] = rd ? pl[row * n1 + lc] : make_float2(0.f, 0.f);
+            for (int u = 0; u < 16; u++)
+                if (dead(j, rows, e0w + u * R2)) on &= ~(1u << u);
+        }
+        const float2 *src = pl + (row0 + (size_t)e0w * se) * n1 + lc;
+        const size_t step = (size_t)(R2 * se) * n1;
+        if (on == 0xffffu) {
+#pragma unroll
+            for (int u = 0; u < 16; u++) pre[u] = src[u * step];
+        } else {
+#pragma unroll
+            for (int u = 0; u < 16; u++) pre[u] = (on >> u) & 1u ? src[u * step] : make_float2(0.f, 0.f);
         }
     };
     int64_t t = blockIdx.x;
-    if (t < ntile) load(t);
+    row_bytes(t);
+    RowBits rows = row_bits();
+    if (t < ntile) load(t, rows);
+    row_bytes(t + gridDim.x);
     for (; t < ntile; t += gridDim.x) {
+        const RowBits next = row_bits();
+        row_bytes(t + 2 * (int64_t)gridDim.x);
         const int x = (int)(t % nx);
         const int64_t r = t / nx;
         const int j = (int)(r % nsub);
@@ -373,7 +417,7 @@ __global__ __launch_bounds__(CB * (1 << LOGL) / 16, CB % 64 == 0 ? 4 : 2) void k
             }
             u1[u] = v;
         }
-        if (t + gridDim.x < ntile) load(t + gridDim.x);
+        if (t + gridDim.x < ntile) load(t + gridDim.x, next);
         // first pass: butterfly i = e0, outputs at 16 e0 + r
         dft_small<T, 16, DIR>(u1);
 #pragma unroll
@@ -416,7 +460,7 @@ __global__ __launch_bounds__(CB * (1 << LOGL) / 16, CB % 64 == 0 ? 4 : 2) void k
                 for (int rr = 0; rr < R2; rr++) {
                     const int e = i + 16 * rr;
                     const size_t row = row0 + (size_t)e * se;
-                    if (mode_out && dead(j, row, e)) continue;
+                    if (mode_out && dead(j, rows, e)) continue;
                     float2 o = v[rr];
                     if (twmode == 1) {
                         float2 w = tab.get(j * e);
@@ -427,6 +471,7 @@ __global__ __launch_bounds__(CB * (1 << LOGL) / 16, CB % 64 == 0 ? 4 : 2) void k
                 }
             }
         }
+        rows = next;
         lds_barrier();
     }
 }

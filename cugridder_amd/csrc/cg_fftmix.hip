@@ -301,7 +301,30 @@ __global__ __launch_bounds__(768) void k_fft_cols_mix(cx_t<T> *data, int n2, int
     const int nx = (nlive + CB - 1) >> bsh;
     const int64_t ntile = (int64_t)nx * nsub * batch;
     const int b = threadIdx.x & (CB - 1);  // nt is a multiple of CB
+    // complex128 forward: the mask of a tile's rows as a bit per element, loaded a
+    // tile ahead by the lanes of each wave.  A byte waited for before each load
+    // of a row took the first step of a call (4096 x 2048 x 194) from 11.2 to
+    // 16.2 ms.  Not in complex64, where the wider code costs a wave per SIMD (16
+    // channels on 3000 x 2500 cells: 0.68 ms the call, so 0.88), and not in the
+    // inverse step, which only stores by the mask (ragged 4800 x 6250: 3.02 ms,
+    // so 3.24).
+    constexpr bool BITS = DIR > 0 && sizeof(T) == 8;
+    uint8_t ahead[4] = {};
+    auto row_bytes = [&](int64_t t) {
+        if (!BITS || mode_in != 1 || t >= ntile) return;
+        const int j = (int)(t / nx % nsub);
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const int e = 64 * w + (threadIdx.x & 63);
+            ahead[w] = e < P.n ? rowmask[j * sj + e * se] : 0;
+        }
+    };
+    row_bytes(blockIdx.x);
     for (int64_t t = blockIdx.x; t < ntile; t += gridDim.x) {
+        uint64_t rows[4];
+#pragma unroll
+        for (int w = 0; w < 4; w++) rows[w] = __ballot(ahead[w] != 0);
+        row_bytes(t + gridDim.x);
         const int x = (int)(t % nx);
         const int64_t rest = t / nx;
         const int j = (int)(rest % nsub);
@@ -309,7 +332,11 @@ __global__ __launch_bounds__(768) void k_fft_cols_mix(cx_t<T> *data, int n2, int
         const bool cok = c < nlive;
         cx_t<T> *pl = data + (size_t)(rest / nsub) * n2 * n1 + (cok ? live.at(c) : 0);
         auto skip = [&](int mode, int row, int e) -> bool {
-            if (mode == 1) return rowmask[row] == 0;
+            if (mode == 1) {
+                if (!BITS) return rowmask[row] == 0;
+                const uint64_t w = e < 128 ? (e < 64 ? rows[0] : rows[1]) : (e < 192 ? rows[2] : rows[3]);
+                return !((w >> (e & 63)) & 1);
+            }
             const int k = j + nsub * e;
             return mode == 2 && k >= spec_a && k < spec_b;
         };
@@ -327,10 +354,27 @@ __global__ __launch_bounds__(768) void k_fft_cols_mix(cx_t<T> *data, int n2, int
                     const int i = index(k);
                     if (i >= tn) continue;
                     if (s == 0) {
+                        if constexpr (BITS) {
+                            // a skipped row reads the plane's first one and is
+                            // cleared once every load is on its way
+                            uint32_t on = 0;
 #pragma unroll
-                        for (int r = 0; r < R; r++) {
-                            const int e = i + r * tn, row = j * sj + e * se;
-                            u[k][r] = cok && !skip(mode_in, row, e) ? pl[(size_t)row * n1] : mkc((T)0, (T)0);
+                            for (int r = 0; r < R; r++)
+                                if (!skip(mode_in, 0, i + r * tn)) on |= 1u << r;
+#pragma unroll
+                            for (int r = 0; r < R; r++) {
+                                const size_t row = (size_t)(j * sj + (i + r * tn) * se);
+                                u[k][r] = pl[row * n1 * ((on >> r) & 1u)];
+                            }
+#pragma unroll
+                            for (int r = 0; r < R; r++)
+                                if (!((on >> r) & 1u)) u[k][r] = mkc((T)0, (T)0);
+                        } else {
+#pragma unroll
+                            for (int r = 0; r < R; r++) {
+                                const int e = i + r * tn, row = j * sj + e * se;
+                                u[k][r] = cok && !skip(mode_in, row, e) ? pl[(size_t)row * n1] : mkc((T)0, (T)0);
+                            }
                         }
                         if (twmode == 2) {
 #pragma unroll
