@@ -43,6 +43,9 @@ struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
     Arena *arena = nullptr;  // non-null: carved from the arena, never freed
+    // what the memory holds beyond a call, 0: nothing.  ensure() clears it with
+    // the memory, so that contents never outlive it.
+    uint64_t holds = 0;
 };
 
 enum Stage { ST_PLAN = 0, ST_SORT, ST_RECORDS, ST_GRID, ST_FFT, ST_FFT2, ST_IMAGE, ST_COUNT };
@@ -77,7 +80,6 @@ struct Ctx {
     // workspace (grow-only)
     DevBuf keys, keys2, vals, vals2, hist, scan, tstart, geo, val, grid, zq, phi3, phi1, phi2,
         part, tw1, tw2, fftmp, dlist, rmask, chans, tlist;
-    int tw1_n = 0, tw2_n = 0, tw_bytes = 0;
     // 6 doubles of pinned memory for the coordinate ranges, in contexts that
     // outlive a call (keep_pinned)
     double *pinned = nullptr;
@@ -134,8 +136,8 @@ struct Ctx {
         each_buf([](DevBuf &b) {
             b.p = nullptr;
             b.bytes = 0;
+            b.holds = 0;
         });
-        tw1_n = tw2_n = tw_bytes = 0;
     }
 
     ~Ctx()
@@ -165,9 +167,8 @@ struct HostPool {
     struct Set {
         int device = 0;
         size_t bytes = 0;
-        std::vector<std::pair<void *, size_t>> bufs;
+        std::vector<DevBuf> bufs;
         double *pinned = nullptr;
-        int tw1_n = 0, tw2_n = 0, tw_bytes = 0;  // the twiddle tables held
     };
     static constexpr size_t kMostSets = 8;
     std::mutex m;
@@ -181,8 +182,8 @@ struct HostPool {
     }
     static void free_set(Set &s)
     {
-        for (auto &b : s.bufs)
-            if (b.first) (void)hipFree(b.first);
+        for (DevBuf &b : s.bufs)
+            if (b.p) (void)hipFree(b.p);
         if (s.pinned) (void)hipHostFree(s.pinned);
         s.bufs.clear();
         s.pinned = nullptr;
@@ -240,6 +241,7 @@ static int ensure(DevBuf &b, size_t bytes)
 {
     if (bytes == 0) bytes = 256;
     if (b.bytes >= bytes) return CG_OK;
+    b.holds = 0;
     if (b.arena) {
         // a buffer that grows within a call takes a new region; the old one
         // stays unused until the arena is reset
@@ -381,25 +383,24 @@ static int records_scratch(Ctx &C, size_t grid_bytes, int64_t M, int dir, float4
     return CG_OK;
 }
 
-// twiddle tables (cached per length and precision)
+// twiddle tables (cached per length and precision: what the buffers hold)
 template <typename T>
 static int twiddles(Ctx &C, int n1, int n2)
 {
-    const int eb = (int)sizeof(cx_t<T>);
-    if (C.tw_bytes != eb || C.tw1_n != n1) {
-        // long rows also need the half-length table, stored after the first
-        const bool lng = fft_row_long<T>(n1);
-        CG_TRY(ensure(C.tw1, (size_t)(lng ? n1 + n1 / 2 : n1) * eb));
-        CG_TRY(launch_row_twiddles<T>(as<cx_t<T>>(C.tw1), n1, C.stream));
-        C.tw1_n = n1;
-    }
-    if (C.tw_bytes != eb || C.tw2_n != n2) {
-        CG_TRY(ensure(C.tw2, (size_t)n2 * eb));
-        CG_TRY(launch_twiddles<T>(as<cx_t<T>>(C.tw2), n2, C.stream));
-        C.tw2_n = n2;
-    }
-    C.tw_bytes = eb;
-    return CG_OK;
+    const size_t eb = sizeof(cx_t<T>);
+    // long rows also need the half-length table, stored after the first
+    const int e1 = fft_row_long<T>(n1) ? n1 + n1 / 2 : n1;
+    auto table = [&](DevBuf &b, int n, int entries, auto launch) -> int {
+        CG_TRY(ensure(b, entries * eb));
+        const uint64_t tag = (uint64_t)n << 8 | eb;
+        if (b.holds == tag) return CG_OK;
+        b.holds = 0;
+        CG_TRY(launch(as<cx_t<T>>(b), n, C.stream));
+        b.holds = tag;
+        return CG_OK;
+    };
+    CG_TRY(table(C.tw1, n1, e1, launch_row_twiddles<T>));
+    return table(C.tw2, n2, n2, launch_twiddles<T>);
 }
 
 // sort rows by the tile of their footprint start; leaves the permutation in
@@ -507,9 +508,10 @@ static int plan_call(Ctx &C, WPlan &P, int64_t nrow, int nchan, const double *fr
     if (nrow * (int64_t)nchan > (int64_t)INT32_MAX - 1) return CG_ERR_SIZE;
     for (int c = 0; c < nchan; c++)
         if (!(freq[c] > 0)) return CG_ERR_ARG;
-    if (!C.part.p) {
-        CG_TRY(ensure(C.part, sizeof(double) * 6152));
+    CG_TRY(ensure(C.part, sizeof(double) * 6152));
+    if (!C.part.holds) {
         CG_TRY(launch_fill_i32(as<int32_t>(C.part), 2 * 6152, 0, C.stream));
+        C.part.holds = 1;  // launch_wminmax leaves its block counter 0
     }
     if (C.keep_pinned && !C.pinned && hipHostMalloc((void **)&C.pinned, 6 * sizeof(double), 0) != hipSuccess) {
         (void)hipGetLastError();
@@ -1451,15 +1453,9 @@ struct HostCall {
         HostPool::Set s = HostPool::get().lease(device);
         C.keep_pinned = true;
         C.pinned = s.pinned;
-        C.tw1_n = s.tw1_n;
-        C.tw2_n = s.tw2_n;
-        C.tw_bytes = s.tw_bytes;
         size_t i = 0;
         each([&](DevBuf &b) {
-            if (i < s.bufs.size()) {
-                b.p = s.bufs[i].first;
-                b.bytes = s.bufs[i].second;
-            }
+            if (i < s.bufs.size()) b = s.bufs[i];
             i++;
         });
         leased = true;
@@ -1480,9 +1476,6 @@ struct HostCall {
         HostPool::Set s;
         s.device = device;
         s.pinned = C.pinned;
-        s.tw1_n = C.tw1_n;
-        s.tw2_n = C.tw2_n;
-        s.tw_bytes = C.tw_bytes;
         C.pinned = nullptr;
         try {
             s.bufs.reserve(64);
@@ -1495,7 +1488,7 @@ struct HostCall {
             return;
         }
         each([&](DevBuf &b) {
-            s.bufs.emplace_back(b.p, b.bytes);
+            s.bufs.push_back(b);
             s.bytes += b.bytes;
             b = DevBuf();
         });

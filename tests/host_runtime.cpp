@@ -1,0 +1,268 @@
+// A HIP runtime of host memory for tests of the library's host side without a
+// GPU: the program defines the runtime calls libcurafft.so makes (they take
+// precedence over libamdhip64's), counts and checks allocations, logs kernel
+// launches by name and runs no kernel.  With every kernel skipped the
+// coordinate ranges read back as zero, so a W-stacking call plans the fewest
+// planes of its kernel.
+//
+//   host_runtime LIB SCENARIO
+//
+// prints one "name value" pair per line for the test to check.
+#include <dlfcn.h>
+
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <string>
+#include <vector>
+
+#include <hip/hip_runtime_api.h>
+
+namespace {
+
+struct Alloc {
+    size_t bytes;
+    uint32_t id;
+    bool host;
+};
+std::mutex mtx;
+std::map<char *, Alloc> live;
+std::map<const void *, std::string> kernels;
+std::vector<std::string> launches;
+size_t used = 0, total = (size_t)1 << 40;
+uint32_t next_id = 1;
+int bad_frees = 0, bad_copies = 0, allocs = 0;
+// hipMalloc of exactly this size fails, fail_times times
+size_t fail_size = 0;
+int fail_times = 0;
+
+// p lies in a live allocation with `bytes` to go
+bool holds(const void *p, size_t bytes)
+{
+    auto it = live.upper_bound((char *)p);
+    if (it == live.begin()) return false;
+    --it;
+    return (char *)p + bytes <= it->first + it->second.bytes;
+}
+
+hipError_t take(void **p, size_t bytes, bool host)
+{
+    std::lock_guard<std::mutex> lock(mtx);
+    if (!host) {
+        if (bytes == fail_size && fail_times > 0) {
+            fail_times--;
+            return hipErrorOutOfMemory;
+        }
+        if (used + bytes > total) return hipErrorOutOfMemory;
+        allocs++;
+    }
+    // (untouched pages of calloc cost nothing)
+    char *q = (char *)std::calloc(1, bytes);
+    if (!q) return hipErrorOutOfMemory;
+    live[q] = Alloc{bytes, next_id++, host};
+    if (!host) used += bytes;
+    *p = q;
+    return hipSuccess;
+}
+
+hipError_t give(void *p)
+{
+    std::lock_guard<std::mutex> lock(mtx);
+    if (!p) return hipSuccess;
+    auto it = live.find((char *)p);
+    if (it == live.end()) {
+        bad_frees++;
+        return hipErrorInvalidValue;
+    }
+    if (!it->second.host) used -= it->second.bytes;
+    live.erase(it);
+    std::free(p);
+    return hipSuccess;
+}
+
+hipError_t copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind)
+{
+    std::lock_guard<std::mutex> lock(mtx);
+    const bool to = kind != hipMemcpyDeviceToHost, from = kind != hipMemcpyHostToDevice;
+    if ((to && !holds(dst, bytes)) || (from && !holds(src, bytes))) {
+        bad_copies++;
+        return hipErrorInvalidValue;
+    }
+    std::memcpy(dst, src, bytes);
+    return hipSuccess;
+}
+
+// launches of kernels whose name holds `part`
+int launched(const char *part)
+{
+    int n = 0;
+    for (const std::string &s : launches) n += s.find(part) != std::string::npos;
+    return n;
+}
+
+}  // namespace
+
+extern "C" {
+
+void **__hipRegisterFatBinary(const void *)
+{
+    static void *handle[1];
+    return handle;
+}
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *, void *, void *,
+                           void *, int *)
+{
+    kernels[host] = name;
+}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+static dim3 cfg_grid, cfg_block;
+static size_t cfg_lds;
+static hipStream_t cfg_stream;
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s)
+{
+    cfg_grid = g;
+    cfg_block = b;
+    cfg_lds = lds;
+    cfg_stream = s;
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t *s)
+{
+    *g = cfg_grid;
+    *b = cfg_block;
+    *lds = cfg_lds;
+    *s = cfg_stream;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t)
+{
+    launches.push_back(kernels[f]);
+    return hipSuccess;
+}
+
+hipError_t hipMalloc(void **p, size_t n) { return take(p, n, false); }
+hipError_t hipFree(void *p) { return give(p); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return take(p, n, true); }
+hipError_t hipHostFree(void *p) { return give(p); }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { return copy(d, s, n, k); }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) { return copy(d, s, n, k); }
+hipError_t hipMemGetInfo(size_t *fr, size_t *tot)
+{
+    *fr = total - used;
+    *tot = total;
+    return hipSuccess;
+}
+hipError_t hipDeviceTotalMem(size_t *n, hipDevice_t)
+{
+    *n = total;
+    return hipSuccess;
+}
+hipError_t hipPointerGetAttribute(void *data, hipPointer_attribute what, hipDeviceptr_t p)
+{
+    std::lock_guard<std::mutex> lock(mtx);
+    auto it = live.find((char *)p);
+    if (it == live.end() || what != HIP_POINTER_ATTRIBUTE_BUFFER_ID) return hipErrorInvalidValue;
+    *(uint32_t *)data = it->second.id;
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int *d)
+{
+    *d = 0;
+    return hipSuccess;
+}
+hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+
+}  // extern "C"
+
+namespace {
+
+using Host = int (*)(int, int, int, double, double, double *, double *, double *, double *, double, double, int);
+using HostF = int (*)(int, int, int, float, float, float *, float *, float *, float *, float, float, int);
+
+struct Lib {
+    void *h;
+    template <typename F>
+    F sym(const char *name) const
+    {
+        F f = (F)dlsym(h, name);
+        if (!f) {
+            std::fprintf(stderr, "%s\n", dlerror());
+            std::exit(3);
+        }
+        return f;
+    }
+    // ms2dirty_1 / ms2dirtyf_1 of nrow zero rows onto nx x ny pixels
+    int image(int nrow, int nx, int ny, double eps = 1e-5) const
+    {
+        std::vector<double> uvw(3 * (size_t)nrow), vis(2 * (size_t)nrow), img(2 * (size_t)nx * ny);
+        auto f = sym<int (*)(int, int, int, double, double, double *, double *, double *, double, double, int)>(
+            "ms2dirty_1");
+        return f(nrow, nx, ny, 1.0, 1e9, uvw.data(), vis.data(), img.data(), eps, 2.0, -1);
+    }
+    int imagef(int nrow, int nx, int ny, float eps = 1e-5f) const
+    {
+        std::vector<float> uvw(3 * (size_t)nrow), vis(2 * (size_t)nrow), img(2 * (size_t)nx * ny);
+        auto f = sym<int (*)(int, int, int, float, float, float *, float *, float *, float, float, int)>(
+            "ms2dirtyf_1");
+        return f(nrow, nx, ny, 1.f, 1e9f, uvw.data(), vis.data(), img.data(), eps, 2.f, -1);
+    }
+};
+
+void show(const char *name, long long v) { std::printf("%s %lld\n", name, v); }
+
+// the number of twiddle tables a call of this shape builds
+int tables(const Lib &L, int nx, int ny, bool single, const char *name)
+{
+    launches.clear();
+    const int ier = single ? L.imagef(10, nx, ny) : L.image(10, nx, ny);
+    show((std::string(name) + "_ier").c_str(), ier);
+    const int n = launched("twiddles");
+    show((std::string(name) + "_tables").c_str(), n);
+    return n;
+}
+
+// A table whose memory is gone, or that was filled in another precision, is
+// built again: 64 x 64 pixels give 128-point tables of 2 KB (complex128), 100
+// pixels 200-point ones of 3200 bytes.
+void twiddle_tags(const Lib &L)
+{
+    tables(L, 64, 64, false, "first");
+    tables(L, 64, 64, false, "again");
+    fail_size = 3200;  // the row table of the larger call (and the retry after a release)
+    fail_times = 1;
+    tables(L, 64, 100, false, "failed");
+    fail_times = 0;
+    tables(L, 64, 64, false, "after_row");
+    // the column table fails once the row table of the new precision is there:
+    // complex64 tables of 960 points take 7680 bytes
+    tables(L, 480, 64, true, "single");
+    fail_size = 15360;
+    fail_times = 1;
+    tables(L, 480, 64, false, "failed_column");
+    fail_times = 0;
+    tables(L, 480, 64, true, "single_again");
+}
+
+}  // namespace
+
+int main(int argc, char **argv)
+{
+    if (argc != 3) return 2;
+    Lib L{dlopen(argv[1], RTLD_NOW | RTLD_GLOBAL)};
+    if (!L.h) {
+        std::fprintf(stderr, "%s\n", dlerror());
+        return 3;
+    }
+    const std::string what = argv[2];
+    if (what == "twiddle_tags") twiddle_tags(L);
+    else return 2;
+    show("bad_frees", bad_frees);
+    show("bad_copies", bad_copies);
+    return 0;
+}

@@ -1,0 +1,45 @@
+"""The library's host side on a HIP runtime of host memory (host_runtime.cpp):
+what calls keep, free and rebuild when allocations fail, without a GPU."""
+import os
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+LIB = os.path.join(ROOT, "cugridder_amd", "libcurafft.so")
+
+
+@pytest.fixture(scope="module")
+def scenario(tmp_path_factory):
+    """scenario(name, **environment) -> {name: value} of one run of the program"""
+    import cugridder_amd
+    cugridder_amd.lib()  # built
+    exe = str(tmp_path_factory.mktemp("host_runtime") / "host_runtime")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-Wall", "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include",
+                           "-rdynamic", os.path.join(HERE, "host_runtime.cpp"), "-o", exe, "-ldl", "-lpthread"])
+
+    def run(name, **env):
+        p = subprocess.run([exe, LIB, name], capture_output=True, text=True, timeout=60,
+                           env={**os.environ, **env})
+        assert p.returncode == 0, (p.returncode, p.stdout, p.stderr)
+        out = {k: int(v) for k, v in (line.split() for line in p.stdout.splitlines())}
+        assert out["bad_frees"] == 0 and out["bad_copies"] == 0, out
+        return out
+
+    return run
+
+
+def test_twiddle_tables_do_not_outlive_their_memory(scenario):
+    """A call whose table cannot be allocated, or which ends between the two
+    tables of a new precision, must not leave a later call a table that is
+    gone or of the other precision."""
+    r = scenario("twiddle_tags")
+    assert r["first_tables"] == 2 and r["again_tables"] == 0
+    assert r["failed_ier"] == 5
+    assert r["after_row_ier"] == 0 and r["after_row_tables"] >= 1
+    assert r["single_tables"] == 2
+    assert r["failed_column_ier"] == 5
+    assert r["single_again_ier"] == 0 and r["single_again_tables"] == 2
