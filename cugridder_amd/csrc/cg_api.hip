@@ -16,7 +16,6 @@
 #include <memory>
 #include <mutex>
 #include <new>
-#include <utility>
 #include <type_traits>
 #include <vector>
 
@@ -110,12 +109,14 @@ struct Ctx {
     Arena arena;
     bool arena_mode = false;
 
+    static constexpr int kBufs = 22;
     template <typename F>
     void each_buf(F f)
     {
         DevBuf *bufs[] = {&keys, &keys2, &vals, &vals2, &hist, &scan, &tstart, &geo, &val,
                           &grid, &zq, &phi3, &phi1, &phi2, &part, &tw1, &tw2, &fftmp, &dlist,
                           &rmask, &chans, &tlist};
+        static_assert(sizeof(bufs) / sizeof(bufs[0]) == kBufs, "");
         for (DevBuf *b : bufs) f(*b);
     }
     // switches this (fresh) context to carving its buffers from [base,
@@ -162,54 +163,53 @@ inline size_t arena_round(size_t bytes) { return (bytes + kArenaAlign - 1) / kAr
 // sets are kept while they hold at most a twelfth of the device's memory together;
 // they are freed by cg_host_release, and when an allocation or a grid does not
 // fit beside them.  Every host call runs on the default stream and returns with
-// it idle.
+// it idle.  Sets are plain values in fixed arrays: giving one back or freeing it
+// allocates nothing and cannot fail.
+constexpr int kHostInputs = 4;
 struct HostPool {
     struct Set {
         int device = 0;
         size_t bytes = 0;
-        std::vector<DevBuf> bufs;
+        DevBuf bufs[Ctx::kBufs + kHostInputs];
         double *pinned = nullptr;
     };
-    static constexpr size_t kMostSets = 8;
+    static constexpr int kMostSets = 8;
     std::mutex m;
-    std::vector<Set> idle;
+    Set idle[kMostSets];
+    int n = 0;
 
     static HostPool &get()
     {
-        // never destroyed: the runtime may be gone when static objects are
-        static HostPool *pool = new HostPool;
-        return *pool;
+        // no destructor: the runtime may be gone when static objects are
+        static_assert(std::is_trivially_destructible<HostPool>::value, "");
+        static HostPool pool;
+        return pool;
     }
     static void free_set(Set &s)
     {
         for (DevBuf &b : s.bufs)
             if (b.p) (void)hipFree(b.p);
         if (s.pinned) (void)hipHostFree(s.pinned);
-        s.bufs.clear();
-        s.pinned = nullptr;
+        s = Set();
     }
     Set lease(int device)
     {
         std::lock_guard<std::mutex> lock(m);
-        for (size_t i = idle.size(); i-- > 0;)
-            if (idle[i].device == device) {
-                Set s = std::move(idle[i]);
-                idle.erase(idle.begin() + (ptrdiff_t)i);
-                return s;
-            }
+        for (int i = n; i-- > 0;)
+            if (idle[i].device == device) return take(i);
         Set s;
         s.device = device;
         return s;
     }
-    void give_back(Set s, size_t most)
+    void give_back(Set &s, size_t most)
     {
         {
             std::lock_guard<std::mutex> lock(m);
             size_t held = s.bytes;
-            for (const Set &t : idle)
-                if (t.device == s.device) held += t.bytes;
-            if (held <= most && idle.size() < kMostSets) {
-                idle.push_back(std::move(s));
+            for (int i = 0; i < n; i++)
+                if (idle[i].device == s.device) held += idle[i].bytes;
+            if (held <= most && n < kMostSets) {
+                idle[n++] = s;
                 return;
             }
         }
@@ -218,17 +218,25 @@ struct HostPool {
     // frees the idle sets of a device (-1: of all); true if there were any
     bool release(int device)
     {
-        std::vector<Set> gone;
+        Set gone[kMostSets];
+        int k = 0;
         {
             std::lock_guard<std::mutex> lock(m);
-            for (size_t i = idle.size(); i-- > 0;)
-                if (device < 0 || idle[i].device == device) {
-                    gone.push_back(std::move(idle[i]));
-                    idle.erase(idle.begin() + (ptrdiff_t)i);
-                }
+            for (int i = n; i-- > 0;)
+                if (device < 0 || idle[i].device == device) gone[k++] = take(i);
         }
-        for (Set &s : gone) free_set(s);
-        return !gone.empty();
+        for (int i = 0; i < k; i++) free_set(gone[i]);
+        return k > 0;
+    }
+
+private:
+    // set i, the others keeping their order (under the lock)
+    Set take(int i)
+    {
+        const Set s = idle[i];
+        std::copy(idle + i + 1, idle + n, idle + i);
+        n--;
+        return s;
     }
 };
 static bool release_idle()
@@ -1443,22 +1451,19 @@ int nufft2d_dev(Ctx &C, int type, int64_t M, const TU *x, const TU *y, cx_t<T> *
 // pool
 struct HostCall {
     Ctx C;
-    DevBuf in[4];
-    int device = 0;
+    DevBuf in[kHostInputs];
 
     int begin()
     {
         env_overrides(C);
+        int device = 0;
         CG_HIP(hipGetDevice(&device));
-        HostPool::Set s = HostPool::get().lease(device);
-        C.keep_pinned = true;
-        C.pinned = s.pinned;
-        size_t i = 0;
-        each([&](DevBuf &b) {
-            if (i < s.bufs.size()) b = s.bufs[i];
-            i++;
-        });
+        set = HostPool::get().lease(device);
         leased = true;
+        C.keep_pinned = true;
+        C.pinned = set.pinned;
+        const DevBuf *b = set.bufs;
+        each([&](DevBuf &d) { d = *b++; });
         return CG_OK;
     }
     template <typename X>
@@ -1473,34 +1478,22 @@ struct HostCall {
         if (!leased) return;
         // (a call that ended early may have left kernels behind)
         const bool idle = hipStreamSynchronize(C.stream) == hipSuccess;
-        HostPool::Set s;
-        s.device = device;
-        s.pinned = C.pinned;
+        set.pinned = C.pinned;
         C.pinned = nullptr;
-        try {
-            s.bufs.reserve(64);
-        } catch (const std::bad_alloc &) {
-            if (s.pinned) (void)hipHostFree(s.pinned);
-            each([](DevBuf &b) {
-                if (b.p) (void)hipFree(b.p);
-                b = DevBuf();
-            });
-            return;
-        }
-        each([&](DevBuf &b) {
-            s.bufs.push_back(b);
-            s.bytes += b.bytes;
-            b = DevBuf();
+        set.bytes = 0;
+        DevBuf *b = set.bufs;
+        each([&](DevBuf &d) {
+            set.bytes += d.bytes;
+            *b++ = d;
+            d = DevBuf();
         });
         size_t total = 0;
-        if (!idle || hipDeviceTotalMem(&total, device) != hipSuccess) total = 0;
-        try {
-            HostPool::get().give_back(std::move(s), total / 12);
-        } catch (const std::bad_alloc &) {
-        }
+        if (!idle || hipDeviceTotalMem(&total, set.device) != hipSuccess) total = 0;
+        HostPool::get().give_back(set, total / 12);
     }
 
 private:
+    HostPool::Set set;
     bool leased = false;
     template <typename F>
     void each(F f)

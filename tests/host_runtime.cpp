@@ -16,6 +16,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -38,6 +39,7 @@ int bad_frees = 0, bad_copies = 0, allocs = 0;
 // hipMalloc of exactly this size fails, fail_times times
 size_t fail_size = 0;
 int fail_times = 0;
+bool fail_new = false;  // operator new throws
 
 // p lies in a live allocation with `bytes` to go
 bool holds(const void *p, size_t bytes)
@@ -104,6 +106,15 @@ int launched(const char *part)
 }
 
 }  // namespace
+
+void *operator new(size_t n)
+{
+    void *p = fail_new ? nullptr : std::malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 extern "C" {
 
@@ -249,6 +260,20 @@ void twiddle_tags(const Lib &L)
     tables(L, 480, 64, true, "single_again");
 }
 
+// the release itself needs no host memory
+void release_without_heap(const Lib &L)
+{
+    show("ier", L.image(100, 64, 64));
+    show("kept", used > 0);
+    const auto release = L.sym<int (*)()>("cg_host_release");
+    fail_new = true;
+    const int ier = release();
+    fail_new = false;
+    show("release_ier", ier);
+    show("left", (long long)used);
+    show("allocations_left", (long long)live.size());
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -261,6 +286,7 @@ int main(int argc, char **argv)
     }
     const std::string what = argv[2];
     if (what == "twiddle_tags") twiddle_tags(L);
+    else if (what == "release_without_heap") release_without_heap(L);
     else return 2;
     show("bad_frees", bad_frees);
     show("bad_copies", bad_copies);

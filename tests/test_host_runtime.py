@@ -43,3 +43,11 @@ def test_twiddle_tables_do_not_outlive_their_memory(scenario):
     assert r["single_tables"] == 2
     assert r["failed_column_ier"] == 5
     assert r["single_again_ier"] == 0 and r["single_again_tables"] == 2
+
+
+def test_release_without_host_memory(scenario):
+    """cg_host_release is a C function: no exception may leave it, and with no
+    host memory at hand it still gives everything back."""
+    r = scenario("release_without_heap")
+    assert r["ier"] == 0 and r["kept"] == 1
+    assert r["release_ier"] == 0 and r["left"] == 0 and r["allocations_left"] == 0
