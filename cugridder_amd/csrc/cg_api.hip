@@ -83,6 +83,9 @@ struct Ctx {
     // outlive a call (keep_pinned)
     double *pinned = nullptr;
     bool keep_pinned = false;
+    // the buffers came with an earlier host call's memory: a call that does not
+    // fit beside it ends with CG_ERR_ALLOC and is run again without (host_call)
+    bool kept_memory = false;
     // stage timing (HIP events on the context stream)
     bool timing = false;
     // stage marks ev[0..ST_COUNT]; ev[ST_COUNT + 1, + 2] bracket the dense
@@ -162,7 +165,8 @@ inline size_t arena_round(size_t bytes) { return (bytes + kArenaAlign - 1) / kAr
 // its device, or starts an empty one, so that threads never share a set.  Returned
 // sets are kept while they hold at most a twelfth of the device's memory together;
 // they are freed by cg_host_release, and when an allocation or a grid does not
-// fit beside them.  Every host call runs on the default stream and returns with
+// fit beside them; so is the set a call leased, which may hold more than it
+// needs.  Every host call runs on the default stream and returns with
 // it idle.  Sets are plain values in fixed arrays: giving one back or freeing it
 // allocates nothing and cannot fail.
 constexpr int kHostInputs = 4;
@@ -648,6 +652,7 @@ static int plan_slab(Ctx &C, const WPlan &P, int eb, int64_t M, int &slab)
         };
         CG_TRY(fits());
         if (whole > limit && release_idle()) CG_TRY(fits());
+        if (whole > limit && C.kept_memory) return CG_ERR_ALLOC;
     }
     if (whole <= limit) return CG_OK;
     if (plane > limit) return CG_ERR_ALLOC;  // not even one plane fits
@@ -1453,13 +1458,13 @@ struct HostCall {
     Ctx C;
     DevBuf in[kHostInputs];
 
-    int begin()
+    int begin(bool lease)
     {
         env_overrides(C);
-        int device = 0;
-        CG_HIP(hipGetDevice(&device));
-        set = HostPool::get().lease(device);
+        CG_HIP(hipGetDevice(&set.device));
+        if (lease) set = HostPool::get().lease(set.device);
         leased = true;
+        C.kept_memory = set.bytes > 0;
         C.keep_pinned = true;
         C.pinned = set.pinned;
         const DevBuf *b = set.bufs;
@@ -1472,6 +1477,15 @@ struct HostCall {
         CG_TRY(ensure(in[k], sizeof(X) * count));
         p = (X *)in[k].p;
         return CG_OK;
+    }
+    // frees everything the call holds
+    void discard()
+    {
+        leased = false;
+        (void)hipStreamSynchronize(C.stream);
+        for (DevBuf &d : in)
+            if (d.p) (void)hipFree(d.p);
+        // (the rest with the context)
     }
     ~HostCall()
     {
@@ -1503,6 +1517,27 @@ private:
     }
 };
 
+// One host call: body(H) on leased memory; when it does not fit beside that, once
+// more without.
+template <typename F>
+static int host_call(F body)
+{
+    try {
+        {
+            HostCall H;
+            CG_TRY(H.begin(true));
+            const int ier = body(H);
+            if (ier != CG_ERR_ALLOC || !H.C.kept_memory) return ier;
+            H.discard();
+        }
+        HostCall H;
+        CG_TRY(H.begin(false));
+        return body(H);
+    } catch (const std::bad_alloc &) {
+        return CG_ERR_ALLOC;
+    }
+}
+
 // host-pointer ms2dirty / dirty2ms: H2D, run, D2H (reference semantics);
 // vis and wgt are [nrow][nchan] for nchan frequencies freq[nchan]
 template <typename T, typename TU, typename TW>
@@ -1512,9 +1547,7 @@ static int host_ms2dirty(int nrow, int nchan, const double *freq, int nx, int ny
 {
     if (nrow < 0 || nchan < 1 || !freq || nx <= 0 || ny <= 0 || !uvw || !dirty || (nrow > 0 && !vis))
         return CG_ERR_ARG;
-    try {
-        HostCall H;
-        CG_TRY(H.begin());
+    return host_call([&](HostCall &H) -> int {
         Ctx &C = H.C;
         C.geom = geom;
         const size_t R = (size_t)nrow, M = R * (size_t)nchan;
@@ -1535,9 +1568,7 @@ static int host_ms2dirty(int nrow, int nchan, const double *freq, int nx, int ny
         if (ier >= 2) return ier;
         CG_HIP(hipMemcpy(dirty, dd, sizeof(cx_t<T>) * (size_t)nx * ny, hipMemcpyDeviceToHost));
         return ier;
-    } catch (const std::bad_alloc &) {
-        return CG_ERR_ALLOC;
-    }
+    });
 }
 
 template <typename T, typename TU, typename TW>
@@ -1547,9 +1578,7 @@ static int host_dirty2ms(int nrow, int nchan, const double *freq, int nx, int ny
 {
     if (nrow < 0 || nchan < 1 || !freq || nx <= 0 || ny <= 0 || !uvw || !dirty || (nrow > 0 && !vis))
         return CG_ERR_ARG;
-    try {
-        HostCall H;
-        CG_TRY(H.begin());
+    return host_call([&](HostCall &H) -> int {
         Ctx &C = H.C;
         C.geom = geom;
         const size_t R = (size_t)nrow, M = R * (size_t)nchan;
@@ -1570,9 +1599,7 @@ static int host_dirty2ms(int nrow, int nchan, const double *freq, int nx, int ny
         if (ier >= 2) return ier;
         if (M) CG_HIP(hipMemcpy(vis, dv, sizeof(cx_t<T>) * M, hipMemcpyDeviceToHost));
         return ier;
-    } catch (const std::bad_alloc &) {
-        return CG_ERR_ALLOC;
-    }
+    });
 }
 
 template <typename T, typename TU>
@@ -1580,9 +1607,7 @@ static int host_nufft2d(int type, int M, const TU *x, const TU *y, void *c, int 
                         void *fk, double eps, double sigma, bool single)
 {
     if (M < 0 || N1 <= 0 || N2 <= 0 || !fk || (M > 0 && (!x || !y || !c))) return CG_ERR_ARG;
-    try {
-        HostCall H;
-        CG_TRY(H.begin());
+    return host_call([&](HostCall &H) -> int {
         Ctx &C = H.C;
         TU *dx = nullptr, *dy = nullptr;
         cx_t<T> *dc = nullptr, *dk = nullptr;
@@ -1604,9 +1629,7 @@ static int host_nufft2d(int type, int M, const TU *x, const TU *y, void *c, int 
         else if (M)
             CG_HIP(hipMemcpy(c, dc, sizeof(cx_t<T>) * (size_t)M, hipMemcpyDeviceToHost));
         return ier;
-    } catch (const std::bad_alloc &) {
-        return CG_ERR_ALLOC;
-    }
+    });
 }
 
 // ---- allocation-free 2-D NUFFT

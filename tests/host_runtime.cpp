@@ -33,10 +33,10 @@ std::mutex mtx;
 std::map<char *, Alloc> live;
 std::map<const void *, std::string> kernels;
 std::vector<std::string> launches;
-size_t used = 0, total = (size_t)1 << 40;
+size_t used = 0, peak = 0, total = (size_t)1 << 40;
 uint32_t next_id = 1;
 int bad_frees = 0, bad_copies = 0, allocs = 0;
-// hipMalloc of exactly this size fails, fail_times times
+// hipMalloc of exactly this size fails fail_times times
 size_t fail_size = 0;
 int fail_times = 0;
 bool fail_new = false;  // operator new throws
@@ -66,6 +66,7 @@ hipError_t take(void **p, size_t bytes, bool host)
     if (!q) return hipErrorOutOfMemory;
     live[q] = Alloc{bytes, next_id++, host};
     if (!host) used += bytes;
+    peak = used > peak ? used : peak;
     *p = q;
     return hipSuccess;
 }
@@ -216,6 +217,13 @@ struct Lib {
             "ms2dirty_1");
         return f(nrow, nx, ny, 1.0, 1e9, uvw.data(), vis.data(), img.data(), eps, 2.0, -1);
     }
+    int nufft(int M, int n) const
+    {
+        std::vector<double> x(M), c(2 * (size_t)M), k(2 * (size_t)n * n);
+        auto f = sym<int (*)(int, const double *, const double *, const double *, int, int, double *, double, double)>(
+            "nufft2d1");
+        return f(M, x.data(), x.data(), c.data(), n, n, k.data(), 1e-5, 2.0);
+    }
     int imagef(int nrow, int nx, int ny, float eps = 1e-5f) const
     {
         std::vector<float> uvw(3 * (size_t)nrow), vis(2 * (size_t)nrow), img(2 * (size_t)nx * ny);
@@ -245,8 +253,8 @@ void twiddle_tags(const Lib &L)
 {
     tables(L, 64, 64, false, "first");
     tables(L, 64, 64, false, "again");
-    fail_size = 3200;  // the row table of the larger call (and the retry after a release)
-    fail_times = 1;
+    fail_size = 3200;  // the row table of the larger call, also when it is tried again
+    fail_times = 100;
     tables(L, 64, 100, false, "failed");
     fail_times = 0;
     tables(L, 64, 64, false, "after_row");
@@ -254,10 +262,67 @@ void twiddle_tags(const Lib &L)
     // complex64 tables of 960 points take 7680 bytes
     tables(L, 480, 64, true, "single");
     fail_size = 15360;
-    fail_times = 1;
+    fail_times = 100;
     tables(L, 480, 64, false, "failed_column");
     fail_times = 0;
     tables(L, 480, 64, true, "single_again");
+}
+
+// the same in a context, whose buffers outlive a failed call
+void context_tags(const Lib &L)
+{
+    const auto create = L.sym<int (*)(void **, void *)>("cg_ctx_create");
+    const auto fft = L.sym<int (*)(void *, int, void *, int, int, int, int)>("cg_fft2d_dev");
+    void *ctx = nullptr, *data = nullptr;
+    show("ier", create(&ctx, nullptr));
+    (void)take(&data, 1 << 20, false);
+    auto run = [&](const char *name, int prec, int n2, int n1) {
+        launches.clear();
+        show((std::string(name) + "_ier").c_str(), fft(ctx, prec, data, 1, n2, n1, 1));
+        show((std::string(name) + "_tables").c_str(), launched("twiddles"));
+    };
+    run("first", 1, 128, 128);
+    run("again", 1, 128, 128);
+    fail_size = 3200;
+    fail_times = 100;
+    run("failed", 1, 128, 200);
+    run("after_row", 1, 128, 128);
+    run("single", 0, 240, 128);
+    fail_size = 3840;
+    run("failed_column", 1, 240, 128);
+    run("single_again", 0, 240, 128);
+    fail_times = 0;
+    L.sym<int (*)(void *)>("cg_ctx_destroy")(ctx);
+    (void)give(data);
+    show("left", (long long)used);
+}
+
+// What an earlier call left must not take the room of a later one: with a
+// device that just holds the later call, it runs as on an idle device.
+void surplus(const Lib &L)
+{
+    const auto release = L.sym<int (*)()>("cg_host_release");
+    show("alone_ier", L.nufft(2000, 256));
+    release();
+    const size_t need = peak;
+    show("before_ier", L.image(10, 16, 16));
+    show("kept", used > 0);
+    total = need;  // not a byte to spare
+    show("after_ier", L.nufft(2000, 256));
+    release();
+    // the least device memory that holds a call's whole grid
+    int whole = 0;
+    for (total = (size_t)256 << 20; !whole; total += (size_t)1 << 20) {
+        launches.clear();
+        const int ier = L.image(10, 512, 512);
+        whole = ier == 0 && launched("k_grid_sparse") == 1;
+        release();
+    }
+    show("many_ier", L.nufft(200000, 64));
+    show("many_kept", used > ((size_t)8 << 20));
+    launches.clear();
+    show("whole_ier", L.image(10, 512, 512));
+    show("slabs", launched("k_grid_sparse"));
 }
 
 // the release itself needs no host memory
@@ -287,6 +352,8 @@ int main(int argc, char **argv)
     const std::string what = argv[2];
     if (what == "twiddle_tags") twiddle_tags(L);
     else if (what == "release_without_heap") release_without_heap(L);
+    else if (what == "context_tags") context_tags(L);
+    else if (what == "surplus") surplus(L);
     else return 2;
     show("bad_frees", bad_frees);
     show("bad_copies", bad_copies);

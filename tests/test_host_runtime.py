@@ -32,17 +32,19 @@ def scenario(tmp_path_factory):
     return run
 
 
-def test_twiddle_tables_do_not_outlive_their_memory(scenario):
+@pytest.mark.parametrize("where", ["twiddle_tags", "context_tags"])
+def test_twiddle_tables_do_not_outlive_their_memory(scenario, where):
     """A call whose table cannot be allocated, or which ends between the two
     tables of a new precision, must not leave a later call a table that is
     gone or of the other precision."""
-    r = scenario("twiddle_tags")
+    r = scenario(where)
     assert r["first_tables"] == 2 and r["again_tables"] == 0
     assert r["failed_ier"] == 5
     assert r["after_row_ier"] == 0 and r["after_row_tables"] >= 1
     assert r["single_tables"] == 2
     assert r["failed_column_ier"] == 5
     assert r["single_again_ier"] == 0 and r["single_again_tables"] == 2
+    assert r.get("left", 0) == 0
 
 
 def test_release_without_host_memory(scenario):
@@ -51,3 +53,14 @@ def test_release_without_host_memory(scenario):
     r = scenario("release_without_heap")
     assert r["ier"] == 0 and r["kept"] == 1
     assert r["release_ier"] == 0 and r["left"] == 0 and r["allocations_left"] == 0
+
+
+def test_kept_memory_makes_room(scenario):
+    """Memory kept from one call is given up when the next one needs the room,
+    also by the call that leased it: neither is a call refused nor a grid cut
+    into slabs that would run whole without the earlier call."""
+    r = scenario("surplus")
+    assert r["alone_ier"] == 0 and r["before_ier"] == 0 and r["kept"] == 1
+    assert r["after_ier"] == 0
+    assert r["many_ier"] == 0 and r["many_kept"] == 1
+    assert r["whole_ier"] == 0 and r["slabs"] == 1
