@@ -168,7 +168,10 @@ inline size_t arena_round(size_t bytes) { return (bytes + kArenaAlign - 1) / kAr
 // fit beside them; so is the set a call leased, which may hold more than it
 // needs.  Every host call runs on the default stream and returns with
 // it idle.  Sets are plain values in fixed arrays: giving one back or freeing it
-// allocates nothing and cannot fail.
+// allocates nothing and cannot fail.  hipDeviceReset frees the memory of a kept
+// set and its addresses may be another's by the next call: a set remembers the
+// runtime's number of one of its allocations, and is forgotten when that
+// address has another number or none.
 constexpr int kHostInputs = 4;
 struct HostPool {
     struct Set {
@@ -176,6 +179,21 @@ struct HostPool {
         size_t bytes = 0;
         DevBuf bufs[Ctx::kBufs + kHostInputs];
         double *pinned = nullptr;
+        uint64_t id = 0;
+        // the number of its first allocation, 0: none
+        uint64_t allocation() const
+        {
+            uint64_t v = 0;
+            for (const DevBuf &b : bufs) {
+                if (!b.p) continue;
+                if (hipPointerGetAttribute(&v, HIP_POINTER_ATTRIBUTE_BUFFER_ID, (hipDeviceptr_t)b.p) ==
+                    hipSuccess)
+                    return v;
+                (void)hipGetLastError();
+                break;
+            }
+            return 0;
+        }
     };
     static constexpr int kMostSets = 8;
     std::mutex m;
@@ -191,6 +209,10 @@ struct HostPool {
     }
     static void free_set(Set &s)
     {
+        if (s.id && s.allocation() != s.id) {
+            s = Set();  // gone with a device reset
+            return;
+        }
         for (DevBuf &b : s.bufs)
             if (b.p) (void)hipFree(b.p);
         if (s.pinned) (void)hipHostFree(s.pinned);
@@ -200,7 +222,10 @@ struct HostPool {
     {
         std::lock_guard<std::mutex> lock(m);
         for (int i = n; i-- > 0;)
-            if (idle[i].device == device) return take(i);
+            if (idle[i].device == device) {
+                const Set s = take(i);
+                if (s.allocation() == s.id) return s;
+            }
         Set s;
         s.device = device;
         return s;
@@ -212,7 +237,8 @@ struct HostPool {
             size_t held = s.bytes;
             for (int i = 0; i < n; i++)
                 if (idle[i].device == s.device) held += idle[i].bytes;
-            if (held <= most && n < kMostSets) {
+            s.id = s.allocation();
+            if (s.id && held <= most && n < kMostSets) {
                 idle[n++] = s;
                 return;
             }

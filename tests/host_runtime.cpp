@@ -181,6 +181,15 @@ hipError_t hipPointerGetAttribute(void *data, hipPointer_attribute what, hipDevi
     *(uint32_t *)data = it->second.id;
     return hipSuccess;
 }
+// every allocation is gone; the next one of the size may get its address
+hipError_t hipDeviceReset(void)
+{
+    std::lock_guard<std::mutex> lock(mtx);
+    for (auto &a : live) std::free(a.first);
+    live.clear();
+    used = 0;
+    return hipSuccess;
+}
 hipError_t hipGetDevice(int *d)
 {
     *d = 0;
@@ -325,6 +334,35 @@ void surplus(const Lib &L)
     show("slabs", launched("k_grid_sparse"));
 }
 
+// After a device reset the kept buffers are gone: nothing may write to them,
+// free them or take their addresses, now another's, for its own.
+void device_reset(const Lib &L)
+{
+    show("before_ier", L.image(1000, 64, 64));
+    show("kept", used > 0);
+    (void)hipDeviceReset();
+    std::vector<void *> others;
+    for (const size_t bytes : {(size_t)1 << 12, (size_t)24000, (size_t)16000, (size_t)1 << 20}) {
+        others.push_back(nullptr);
+        (void)take(&others.back(), bytes, false);
+    }
+    const size_t held = used;
+    show("after_ier", L.image(1000, 64, 64));
+    (void)hipDeviceReset();
+    const int ier = L.sym<int (*)()>("cg_host_release")();
+    show("release_ier", ier);
+    show("left", (long long)used);
+    // a reset with another's memory at every kept address
+    show("again_ier", L.image(1000, 64, 64));
+    std::vector<std::pair<char *, Alloc>> was(live.begin(), live.end());
+    for (auto &a : was) live[a.first].id = next_id++;
+    show("moved_ier", L.image(1000, 64, 64));
+    int lost = 0;
+    for (auto &a : was) lost += !live.count(a.first);
+    show("others_freed", lost);
+    show("held", held > 0);
+}
+
 // the release itself needs no host memory
 void release_without_heap(const Lib &L)
 {
@@ -353,6 +391,7 @@ int main(int argc, char **argv)
     if (what == "twiddle_tags") twiddle_tags(L);
     else if (what == "release_without_heap") release_without_heap(L);
     else if (what == "context_tags") context_tags(L);
+    else if (what == "device_reset") device_reset(L);
     else if (what == "surplus") surplus(L);
     else return 2;
     show("bad_frees", bad_frees);

@@ -64,3 +64,14 @@ def test_kept_memory_makes_room(scenario):
     assert r["after_ier"] == 0
     assert r["many_ier"] == 0 and r["many_kept"] == 1
     assert r["whole_ier"] == 0 and r["slabs"] == 1
+
+
+def test_device_reset_between_host_calls(scenario):
+    """After hipDeviceReset a host call works as the first one did, and what the
+    earlier calls kept is neither used nor freed, whoever has the addresses
+    now."""
+    r = scenario("device_reset")
+    assert r["before_ier"] == 0 and r["kept"] == 1
+    assert r["after_ier"] == 0
+    assert r["release_ier"] == 0 and r["left"] == 0
+    assert r["again_ier"] == 0 and r["moved_ier"] == 0 and r["others_freed"] == 0
