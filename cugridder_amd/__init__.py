@@ -8,10 +8,11 @@ __init__.py:1-3); ``vis2dirty`` / ``dirty2vis`` the plain complex ones; and
 from .cursl import dirty2ms, ms2dirty
 from .curagridder import (dirty2vis, dirty2vis_mixed, nufft2d1, nufft2d2, vis2dirty,
                           vis2dirty_mixed)
-from ._lib import LIB_PATH, lib
+from ._lib import LIB_PATH, lib, release_host_memory
 
 __all__ = ["ms2dirty", "dirty2ms", "vis2dirty", "dirty2vis", "vis2dirty_mixed",
-           "dirty2vis_mixed", "nufft2d1", "nufft2d2", "Context", "lib", "LIB_PATH"]
+           "dirty2vis_mixed", "nufft2d1", "nufft2d2", "Context", "lib", "release_host_memory",
+           "LIB_PATH"]
 
 
 def __getattr__(name):

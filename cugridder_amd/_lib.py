@@ -45,6 +45,15 @@ BATCH_AUTOTUNE = 1
 BATCH_GRAPH = 2
 
 
+def release_host_memory():
+    """Frees the device memory the numpy entry points keep between their calls.
+
+    The library does so itself when it runs out of memory; another allocator
+    in the process (torch) cannot ask for it.  CG_HOST_KEEP_MB in the
+    environment bounds what is kept (0: nothing)."""
+    check(lib().cg_host_release(), "release_host_memory")
+
+
 def lib():
     """The loaded libcurafft.so with argtypes declared."""
     global _lib

@@ -163,7 +163,8 @@ inline size_t arena_round(size_t bytes) { return (bytes + kArenaAlign - 1) / kAr
 // freed memory at some 30 GB/s, which a program that calls back to back ends up
 // waiting for: 8 ms a call, then 68 ms).  A call leases an idle set of buffers of
 // its device, or starts an empty one, so that threads never share a set.  Returned
-// sets are kept while they hold at most a twelfth of the device's memory together;
+// sets are kept while they hold at most a twelfth of the device's memory together
+// (or CG_HOST_KEEP_MB in the environment, if that is less: 0 keeps nothing);
 // they are freed by cg_host_release, and when an allocation or a grid does not
 // fit beside them; so is the set a call leased, which may hold more than it
 // needs.  Every host call runs on the default stream and returns with
@@ -1527,9 +1528,12 @@ struct HostCall {
             *b++ = d;
             d = DevBuf();
         });
-        size_t total = 0;
-        if (!idle || hipDeviceTotalMem(&total, set.device) != hipSuccess) total = 0;
-        HostPool::get().give_back(set, total / 12);
+        size_t most = 0;
+        if (idle && hipDeviceTotalMem(&most, set.device) == hipSuccess) most /= 12;
+        else most = 0;
+        if (const char *e = std::getenv("CG_HOST_KEEP_MB"))
+            most = std::min(most, (size_t)std::max(0, std::atoi(e)) << 20);
+        HostPool::get().give_back(set, most);
     }
 
 private:

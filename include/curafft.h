@@ -316,7 +316,10 @@ int cg_sort_pairs_dev(void *ctx, void *d_keys, void *d_vals, int m,
                       int key_bits);
 
 /* Frees the device memory that the host-pointer entry points keep between
- * their calls (at most a twelfth of each GPU's memory). */
+ * their calls: at most a twelfth of each GPU's memory, or CG_HOST_KEEP_MB MiB
+ * when that environment variable is set to less (0: nothing is kept).  The
+ * library gives it up by itself when one of its own allocations fails; a
+ * program that allocates device memory by other means calls this first. */
 int cg_host_release(void);
 
 /* Device-to-device copy of bytes on a HIP stream (test hook). */

@@ -334,6 +334,15 @@ void surplus(const Lib &L)
     show("slabs", launched("k_grid_sparse"));
 }
 
+// what two calls leave allocated
+void kept_bytes(const Lib &L)
+{
+    show("ier", L.image(1000, 64, 64));
+    show("kept", (long long)used);
+    show("second_ier", L.image(1000, 100, 64));
+    show("second_kept", (long long)used);
+}
+
 // After a device reset the kept buffers are gone: nothing may write to them,
 // free them or take their addresses, now another's, for its own.
 void device_reset(const Lib &L)
@@ -392,6 +401,7 @@ int main(int argc, char **argv)
     else if (what == "release_without_heap") release_without_heap(L);
     else if (what == "context_tags") context_tags(L);
     else if (what == "device_reset") device_reset(L);
+    else if (what == "kept_bytes") kept_bytes(L);
     else if (what == "surplus") surplus(L);
     else return 2;
     show("bad_frees", bad_frees);

@@ -75,3 +75,21 @@ def test_device_reset_between_host_calls(scenario):
     assert r["after_ier"] == 0
     assert r["release_ier"] == 0 and r["left"] == 0
     assert r["again_ier"] == 0 and r["moved_ier"] == 0 and r["others_freed"] == 0
+
+
+def test_kept_memory_is_bounded(scenario):
+    """CG_HOST_KEEP_MB bounds what host calls keep, down to nothing."""
+    whole = scenario("kept_bytes")
+    assert whole["ier"] == 0 and whole["second_ier"] == 0
+    assert 3 << 20 < whole["kept"] <= whole["second_kept"]
+    for mb in (0, 2, 1000):
+        r = scenario("kept_bytes", CG_HOST_KEEP_MB=str(mb))
+        assert r["ier"] == 0 and r["second_ier"] == 0
+        for k in ("kept", "second_kept"):
+            assert r[k] == (whole[k] if whole[k] <= mb << 20 else 0)
+
+
+def test_release_from_python():
+    import cugridder_amd
+    cugridder_amd.release_host_memory()
+    assert "release_host_memory" in cugridder_amd.__all__
