@@ -721,8 +721,15 @@ static int plan_ms2dirty(Ctx &C, CallPlan &cp, int64_t nrow, int nchan, const do
     cp.M = nrow * nchan;
     CG_TRY(plan_slab(C, P, eb, cp.M, cp.slab));
     // gridding accumulates in FP64 (16 bytes per cell) whatever the precision
-    cp.t = choose_tiling(P.nf1, P.nf2, cp.slab ? cp.slab : P.nf3, P.conv.kw, 16, tn.grid_lds,
-                         tn.tile_grid, 0);
+    const int planes = cp.slab ? cp.slab : P.nf3;
+    cp.t = choose_tiling(P.nf1, P.nf2, planes, P.conv.kw, 16, tn.grid_lds, tn.tile_grid, 0);
+    if (P.wstack && std::min(cp.t.tx, cp.t.ty) < 2) {
+        // a tile_grid of 1, or one that leaves 1 after halving: with too many bins
+        // around a cell refused as in the 2-D gridder, else tiles of 2, the
+        // least launch_grid_sparse takes (an axis has an even number of cells)
+        if (cp.t.sbx * cp.t.sby > kMaxBins) return CG_ERR_SIZE;
+        cp.t = choose_tiling(P.nf1, P.nf2, planes, P.conv.kw, 16, tn.grid_lds, tn.tile_grid, 0, 2);
+    }
     cp.a = make_coord_args(P, cp.t);
     set_key_rect(cp.a, P, cp.t, C.compact_keys != 0);
     CG_TRY(channel_scales(C, nchan, freq, cp.a));

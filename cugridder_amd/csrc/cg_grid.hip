@@ -64,9 +64,6 @@ __device__ __forceinline__ Span tile_span(int r, int t, int n)
     return sp;
 }
 
-// most source bins feeding one tile: (1 + ceil(15/2))^2 for tiles >= 2
-constexpr int kMaxBins = 81;
-
 template <typename T, int KW>
 __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
                                                const cx_t<T> *__restrict__ val,

@@ -183,6 +183,8 @@ struct GridArgs {
     // the output instead of storing it.
     int zb, zn, accumulate;
 };
+// most source bins feeding one tile: (1 + ceil(15/2))^2 for tiles >= 2
+constexpr int kMaxBins = 81;
 // planes held by the grid buffer
 __host__ __device__ inline int slab_planes(const GridArgs &g) { return g.zn > 0 ? g.zn : g.nf3; }
 bool grid2d_mfma_supported(const GridArgs &g, int kw);

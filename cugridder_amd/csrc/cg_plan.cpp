@@ -217,7 +217,7 @@ void plan_bands(WPlan &p, double ulo, double uhi, double vlo, double vhi)
 }
 
 Tiling choose_tiling(int nf1, int nf2, int nplanes, int kw, int elem_bytes,
-                     int lds_budget, int tile_pref, int halo)
+                     int lds_budget, int tile_pref, int halo, int least)
 {
     // Tiles must divide the grid (so no tile is partial); pick the largest
     // power of two <= tile_pref that divides each axis.
@@ -239,6 +239,8 @@ Tiling choose_tiling(int nf1, int nf2, int nplanes, int kw, int elem_bytes,
         if (T.tx >= T.ty && T.tx > 2) T.tx >>= 1;
         else T.ty >>= 1;
     }
+    T.tx = std::max(T.tx, least);
+    T.ty = std::max(T.ty, least);
     T.ntx = nf1 / T.tx;
     T.nty = nf2 / T.ty;
     // a point whose footprint starts in bin b touches tiles b .. b+sb-1

@@ -114,8 +114,8 @@ int make_wplan(WPlan &p, int64_t nrow, int nxdirty, int nydirty, double fov,
 // Chooses tile extents and plane chunking for an LDS budget (bytes) and
 // complex element size; `nplanes` is the grid depth and `halo` the extra
 // cells per axis a workgroup keeps in LDS (kw-1 when degridding, 0 when
-// gridding).
+// gridding).  No edge is shorter than `least` (1 or 2: the axes are even).
 Tiling choose_tiling(int nf1, int nf2, int nplanes, int kw, int elem_bytes,
-                     int lds_budget, int tile_pref, int halo);
+                     int lds_budget, int tile_pref, int halo, int least = 1);
 
 }  // namespace cg

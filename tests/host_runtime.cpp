@@ -10,6 +10,7 @@
 // prints one "name value" pair per line for the test to check.
 #include <dlfcn.h>
 
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -334,6 +335,29 @@ void surplus(const Lib &L)
     show("slabs", launched("k_grid_sparse"));
 }
 
+// ms2dirty on a context with gridding tiles of a given edge, 40 x 36 pixels
+void tile_edges(const Lib &L)
+{
+    const auto create = L.sym<int (*)(void **, void *)>("cg_ctx_create");
+    const auto option = L.sym<int (*)(void *, const char *, int)>("cg_ctx_set_option");
+    const auto run = L.sym<int (*)(void *, int, int, int, int, double, double, const void *, int, const void *,
+                                   const void *, int, void *, double, double, int)>("cg_ms2dirty_dev");
+    void *uvw = nullptr, *vis = nullptr, *img = nullptr;
+    (void)take(&uvw, 24 * 50, false);
+    (void)take(&vis, 16 * 50, false);
+    (void)take(&img, 16 * 40 * 36, false);
+    for (const int tile : {0, 1, 2, 3, 5, 8, 12})
+        for (const int kw : {4, 9, 10, 13}) {
+            void *ctx = nullptr;
+            (void)create(&ctx, nullptr);
+            option(ctx, "tile_grid", tile);
+            launches.clear();
+            const int ier = run(ctx, 1, 50, 40, 36, 5.0, 1e9, uvw, 1, vis, nullptr, 1, img, std::pow(10.0, 1 - kw) * 1.01, 2.0, -1);
+            show(("tile" + std::to_string(tile) + "_kw" + std::to_string(kw)).c_str(), ier);
+            L.sym<int (*)(void *)>("cg_ctx_destroy")(ctx);
+        }
+}
+
 // what two calls leave allocated
 void kept_bytes(const Lib &L)
 {
@@ -402,6 +426,7 @@ int main(int argc, char **argv)
     else if (what == "context_tags") context_tags(L);
     else if (what == "device_reset") device_reset(L);
     else if (what == "kept_bytes") kept_bytes(L);
+    else if (what == "tile_edges") tile_edges(L);
     else if (what == "surplus") surplus(L);
     else return 2;
     show("bad_frees", bad_frees);

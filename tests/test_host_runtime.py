@@ -93,3 +93,13 @@ def test_release_from_python():
     import cugridder_amd
     cugridder_amd.release_host_memory()
     assert "release_host_memory" in cugridder_amd.__all__
+
+
+def test_tile_edges_stay_accepted(scenario):
+    """Gridding tiles of one cell, asked for or left after halving (3 and 12 on
+    80 x 72 cells), are accepted up to kernel width 9, where the bins around a
+    tile are at most 81, and refused by size above."""
+    r = scenario("tile_edges")
+    for tile in (0, 1, 2, 3, 5, 8, 12):
+        for kw in (4, 9, 10, 13):
+            assert r[f"tile{tile}_kw{kw}"] == (3 if tile < 2 and kw > 9 else 0)
