@@ -78,7 +78,7 @@ struct Ctx {
     int last_cshift = 0;
     // workspace (grow-only)
     DevBuf keys, keys2, vals, vals2, hist, scan, tstart, geo, val, grid, zq, phi3, phi1, phi2,
-        part, tw1, tw2, fftmp, dlist, rmask, chans, tlist;
+        part, tw1, tw2, fftmp, dlist, rmask, chans, tlist, clist;
     // 6 doubles of pinned memory for the coordinate ranges, in contexts that
     // outlive a call (keep_pinned)
     double *pinned = nullptr;
@@ -112,13 +112,13 @@ struct Ctx {
     Arena arena;
     bool arena_mode = false;
 
-    static constexpr int kBufs = 22;
+    static constexpr int kBufs = 23;
     template <typename F>
     void each_buf(F f)
     {
         DevBuf *bufs[] = {&keys, &keys2, &vals, &vals2, &hist, &scan, &tstart, &geo, &val,
                           &grid, &zq, &phi3, &phi1, &phi2, &part, &tw1, &tw2, &fftmp, &dlist,
-                          &rmask, &chans, &tlist};
+                          &rmask, &chans, &tlist, &clist};
         static_assert(sizeof(bufs) / sizeof(bufs[0]) == kBufs, "");
         for (DevBuf *b : bufs) f(*b);
     }
@@ -404,6 +404,45 @@ static int grid_masks(Ctx &C, GridArgs &g, const uint8_t *mask, int nf1, int nf2
         CG_TRY(ensure(C.tlist, sizeof(int32_t) * (size_t)(n + 1)));
         g.rowmask = mask;
         g.colmask = mask + nf2;
+        g.tile_list = as<int32_t>(C.tlist);
+    }
+    return CG_OK;
+}
+
+// W-stacking: the points that reach a crowded part of the grid go to k_grid, whose
+// workgroups share them; a block of k_grid_sparse takes its points on one wave for
+// every window of 16 planes, 0.14 us a point.  k_grid takes about 0.27 + 0.0018
+// taps inside a tile of that for a point (measured for kw 2 .. 9 and tiles of 2, 4
+// and 8; from kw 10 on its registers spill, from 12 on it is never the faster);
+// its chunks of planes run side by side as the windows do.  Below some hundred
+// points its fixed cost per tile is the larger part, and a few crowded regions
+// leave the rim's chains to k_grid_sparse, which run before it.  complex128, ms per call on k_grid_sparse alone and so: 1024^2
+// cells, 10^6 rows spread over 1 / 20 / 60 cells, kw 2 102 / 2.8 / 1.28,
+// 9.9 / 1.08 / 0.45; kw 6 134 / 5.9 / 2.39, 66 / 5.1 / 1.74; kw 7 136 / 7.3 / 2.76,
+// 94 / 7.4 / 2.30; kw 8, where it does not (with it from 1024 points on),
+// 137 / 8.2 / 3.0, (125 / 10.2 / 3.3).  1250^2 cells, tiles of 2, kw 8, spread over
+// 5 / 20 / 60: 74 / 8.0 / 3.3, 23 / 5.1 / 3.5.
+static int crowd_min(const WPlan &P, const GridArgs &g, int planes)
+{
+    const int kw = P.conv.kw, windows = (planes + 15) / 16;
+    if (!P.wstack || kw > 11 || !sparse_crowdable(g)) return 0;
+    const double share = windows == 1 ? 1.0 : (kw + 15) / (16.0 * windows);
+    const int taps = std::min(kw, g.tx) * std::min(kw, g.ty) * kw;
+    const double cost = (0.27 + 0.0018 * taps) * (kw > 9 ? 1.4 : 1.0);
+    if (cost >= share * g.nchunk) return 0;
+    const int least = (int)((256 << (kw > 7 ? kw - 4 : std::max(0, kw - 5))) / share);
+    // (the dense path's bins do not count)
+    return g.m < least || (g.dense_min > 0 && g.dense_min <= least) ? 0 : least;
+}
+
+static int grid_crowded(Ctx &C, const WPlan &P, const Tiling &t, GridArgs &g, int planes)
+{
+    g.crowd_min = crowd_min(P, g, planes);
+    if (!g.crowd_min) return CG_OK;
+    CG_TRY(ensure(C.clist, sizeof(int32_t) * (size_t)(t.ntiles() + 1)));
+    g.crowd_list = as<int32_t>(C.clist);
+    if (!g.tile_list) {
+        CG_TRY(ensure(C.tlist, sizeof(int32_t) * (size_t)(sparse_blocks(P.nf1, P.nf2) + 1)));
         g.tile_list = as<int32_t>(C.tlist);
     }
     return CG_OK;
@@ -767,9 +806,11 @@ static int exec_ms2dirty(Ctx &C, const CallPlan &cp, const TU *uvw, const cx_t<T
     g.kr = key_rect(a);
     g.dense_min = cp.dense_min;
     CG_TRY(grid_masks<T>(C, g, rm, P.nf1, P.nf2));
+    CG_TRY(grid_crowded(C, P, t, g, cp.slab ? cp.slab : P.nf3));
     WArgs w = make_wargs(P);
     CG_TRY(image_tables(C, P));
     CallClear clr{rm, rm ? P.nf1 + P.nf2 : 0, {g.tile_list}};
+    clr.counter[3] = g.crowd_list;
     if (cp.dense_min > 0) {
         CG_TRY(ensure(C.dlist, sizeof(int32_t) * dense_list_ints(t.ntiles(), g.m)));
         clr.counter[1] = as<int32_t>(C.dlist);
@@ -823,10 +864,16 @@ static int exec_ms2dirty(Ctx &C, const CallPlan &cp, const TU *uvw, const cx_t<T
             g.zn = zn;
             g.nchunk = (zn + t.pc - 1) / t.pc;
         }
-        if (P.wstack)
+        if (P.wstack) {
             CG_TRY(launch_grid_sparse<T>(as<geo_t<T>>(C.geo), as<cx_t<T>>(C.val), as<int32_t>(C.tstart),
                                          as<cx_t<T>>(C.grid), g, P.conv.kw, C.stream));
-        else
+            if (g.crowd_min > 0) {
+                GridArgs c = g;
+                c.tile_list = g.crowd_list;
+                CG_TRY(launch_grid<T>(as<geo_t<T>>(C.geo), as<cx_t<T>>(C.val), as<int32_t>(C.tstart),
+                                      as<cx_t<T>>(C.grid), c, P.conv.kw, C.stream));
+            }
+        } else
             CG_TRY(launch_grid<T>(as<geo_t<T>>(C.geo), as<cx_t<T>>(C.val), as<int32_t>(C.tstart),
                                   as<cx_t<T>>(C.grid), g, P.conv.kw, C.stream));
         if (cp.dense_min > 0) {

@@ -7,8 +7,9 @@
 // |d| < kw/2 (conv.cu:32-36, unnormalised as in the reference).
 //
 // W-stacking grids: cg_sparse.hip, and for dense bins k_grid_dense2 below.
-// 2-D grids (one plane): one workgroup owns a tx*ty tile of grid cells and
-// accumulates it in LDS (real parts, then imaginary parts, so
+// 2-D grids (one plane), and crowded tiles of W-stacking grids (crowd_min in
+// cg_api.hip): one workgroup owns a tx*ty tile of grid cells, of W-stacking
+// grids for a chunk of planes, and accumulates it in LDS (real parts, then imaginary parts, so
 // the lanes' random cells spread over twice as many banks as interleaved
 // pairs would) with FP64 ds_add atomics (on gfx950 the
 // FP32 LDS atomic add runs ~20x slower than the FP64 one, and FP64 also makes
@@ -40,7 +41,7 @@ int degrid_lds_bytes(const GridArgs &g, int kw, int elem)
 
 // ------------------------------------------------------------ gridding
 
-// Footprint of a point relative to a tile [0, t) of an axis
+// Footprint of a point relative to a tile (or plane chunk) [0, t) of an axis
 // of length n, given its start r relative to the tile origin (in [0, n)):
 // first tap position s (negative when the footprint starts in an earlier
 // tile) and the taps [lo, hi) that land inside the tile.  With one tile
@@ -68,19 +69,25 @@ template <typename T, int KW>
 __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
                                                const cx_t<T> *__restrict__ val,
                                                const int32_t *__restrict__ tile_start,
-                                               cx_t<T> *__restrict__ fw, GridArgs g)
+                                               cx_t<T> *__restrict__ fw, GridArgs g, int is2d)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     double *acc = reinterpret_cast<double *>(smem_raw);
     __shared__ int s_beg[kMaxBins], s_cnt[kMaxBins], s_ox[kMaxBins], s_oy[kMaxBins];
     __shared__ int s_total;
-    // work item = a tile: one per workgroup, or, with a tile list (the tiles
-    // some FFT pass reads), the workgroups walk the list
-    const int nwork = g.tile_list ? g.tile_list[0] : (int)gridDim.x;
+    // work item = (tile, plane chunk): one per workgroup, or, with a tile
+    // list (the tiles some FFT pass reads, or the crowded ones), the
+    // workgroups walk the list
+    const int nwork = g.tile_list ? g.tile_list[0] * g.nchunk : (int)gridDim.x;
     for (int wi = blockIdx.x; wi < nwork; wi += gridDim.x) {
-    const int tile = g.tile_list ? g.tile_list[1 + wi] : wi;
+    const int chunk = wi % g.nchunk;
+    const int tile = g.tile_list ? g.tile_list[1 + wi / g.nchunk] : wi / g.nchunk;
     const int bx = tile % g.ntx, by = tile / g.ntx;
-    const int cells = g.ty * g.tx;
+    // planes [p0, p0 + np) of the slab [zb, zb + zn) held by the buffer
+    const int zn = slab_planes(g);
+    const int p0 = g.zb + chunk * g.pc;
+    const int np = min(g.pc, g.zb + zn - p0);
+    const int cells = np * g.ty * g.tx;
     for (int k = threadIdx.x; k < 2 * cells; k += blockDim.x) acc[k] = 0.0;
     // source bins whose footprints can reach this tile: bin (bx - sx, by - sy)
     const int nbins = g.sbx * g.sby;
@@ -97,6 +104,8 @@ __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
             const int sidx = sby_ * g.ntx + sbx_;
             s_beg[b] = tile_start[sidx];
             s_cnt[b] = tile_start[sidx + 1] - s_beg[b];
+            // dense bins are added afterwards by k_grid_dense2
+            if (g.dense_min > 0 && s_cnt[b] >= g.dense_min) s_cnt[b] = 0;
             s_ox[b] = ox;
             s_oy[b] = oy;
             tot += s_cnt[b];
@@ -126,6 +135,13 @@ __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
         const Span X = tile_span<KW>(rx, g.tx, g.nf1);
         const Span Y = tile_span<KW>(ry, g.ty, g.nf2);
         if (X.lo >= X.hi || Y.lo >= Y.hi) continue;
+        Span Z{0, 0, 1};
+        if (!is2d) {
+            int rz = (int)(pk >> 16) - p0;
+            if (rz < 0) rz += g.nf3;
+            Z = tile_span<KW>(rz, np, g.nf3);
+            if (Z.lo >= Z.hi) continue;
+        }
         const cx_t<T> v = val[idx];
         T kx[KW], ky[KW];
 #pragma unroll
@@ -133,27 +149,36 @@ __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
             kx[t] = ker(G.x, t);
             ky[t] = ker(G.y, t);
         }
+        for (int tz = Z.lo; tz < Z.hi; tz++) {
+            int zz = Z.s + tz;
+            if (zz >= np) zz -= np;  // wraps only when one chunk holds every plane
+            const T kz = is2d ? (T)1 : ker(G.z, tz);
+            const T vzr = v.x * kz, vzi = v.y * kz;
 #pragma unroll
-        for (int t2 = 0; t2 < KW; t2++) {
-            if (t2 < Y.lo || t2 >= Y.hi) continue;
-            int yy = Y.s + t2;
-            if (yy >= g.nf2) yy -= g.nf2;  // wraps only with one tile along nf2
-            const T vyr = v.x * ky[t2], vyi = v.y * ky[t2];
-            double *row = acc + yy * g.tx;
+            for (int t2 = 0; t2 < KW; t2++) {
+                if (t2 < Y.lo || t2 >= Y.hi) continue;
+                int yy = Y.s + t2;
+                if (yy >= g.nf2) yy -= g.nf2;  // wraps only with one tile along nf2
+                const T vyr = vzr * ky[t2], vyi = vzi * ky[t2];
+                double *row = acc + (zz * g.ty + yy) * g.tx;
 #pragma unroll
-            for (int t1 = 0; t1 < KW; t1++) {
-                if (t1 < X.lo || t1 >= X.hi) continue;
-                int xx = X.s + t1;
-                if (xx >= g.nf1) xx -= g.nf1;
-                atomicAdd(row + xx, (double)(vyr * kx[t1]));
-                atomicAdd(row + cells + xx, (double)(vyi * kx[t1]));
+                for (int t1 = 0; t1 < KW; t1++) {
+                    if (t1 < X.lo || t1 >= X.hi) continue;
+                    int xx = X.s + t1;
+                    if (xx >= g.nf1) xx -= g.nf1;
+                    atomicAdd(row + xx, (double)(vyr * kx[t1]));
+                    atomicAdd(row + cells + xx, (double)(vyi * kx[t1]));
+                }
             }
         }
     }
     __syncthreads();
+    const int plane_cells = g.ty * g.tx;
     for (int k = threadIdx.x; k < cells; k += blockDim.x) {
-        const int y = k / g.tx, x = k - y * g.tx;
-        const size_t gi = (size_t)(by * g.ty + y) * g.nf1 + bx * g.tx + x;
+        int lz = k / plane_cells;
+        int rem = k - lz * plane_cells;
+        int y = rem / g.tx, x = rem - y * g.tx;
+        size_t gi = ((size_t)(p0 - g.zb + lz) * g.nf2 + (size_t)(by * g.ty + y)) * g.nf1 + bx * g.tx + x;
         fw[gi] = mkc((T)acc[k], (T)acc[cells + k]);
     }
     __syncthreads();  // acc and the bin table are reused by the next item
@@ -369,19 +394,21 @@ template <typename T, int KW>
 static int grid_kw(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *ts, cx_t<T> *fw,
                    const GridArgs &g, hipStream_t s)
 {
-    if (g.sbx * g.sby > kMaxBins || g.nf3 != 1 || g.nchunk != 1) return CG_ERR_SIZE;
+    const int is2d = g.nf3 == 1 ? 1 : 0;
+    if (g.sbx * g.sby > kMaxBins || (!is2d && !g.tile_list)) return CG_ERR_SIZE;
     size_t lds = (size_t)grid_lds_bytes(g, (int)sizeof(cx_t<T>));
     const int64_t ntiles = (int64_t)g.ntx * g.nty;
     unsigned nblk = (unsigned)ntiles;
     if (g.tile_list) {
-        // build the list of tiles to write; workgroups then walk it
-        hipLaunchKernelGGL(k_need_tiles, dim3((unsigned)ceil_div(ntiles, 256)), dim3(256), 0, s,
-                           g.rowmask, g.colmask, g.ntx, ntiles, g.tx, g.ty,
-                           const_cast<int32_t *>(g.tile_list));
+        // build the list of tiles to write (that of crowded ones is there);
+        // workgroups then walk it
+        if (is2d)
+            hipLaunchKernelGGL(k_need_tiles, dim3((unsigned)ceil_div(ntiles, 256)), dim3(256), 0, s,
+                               g.rowmask, g.colmask, g.ntx, ntiles, g.tx, g.ty, g.tile_list);
         const int threads = grid_threads(lds);
         const int per_cu = std::max(1, std::min((int)(163840 / std::max<size_t>(lds, 1)),
                                                 2048 / threads));
-        nblk = (unsigned)std::min<int64_t>(ntiles, (int64_t)256 * per_cu);
+        nblk = (unsigned)std::min<int64_t>(ntiles * g.nchunk, (int64_t)256 * per_cu);
     }
     if constexpr (sizeof(T) == 4 && KW <= kQ2) {
         if (grid2d_mfma_supported(g, KW)) {
@@ -399,7 +426,7 @@ static int grid_kw(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *ts, c
         CG_HIP(hipFuncSetAttribute((const void *)k_grid<T, KW>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL((k_grid<T, KW>), dim3(nblk), dim3(grid_threads(lds)), lds, s, geo, val, ts,
-                       fw, g);
+                       fw, g, is2d);
     CG_HIP(hipGetLastError());
     return CG_OK;
 }

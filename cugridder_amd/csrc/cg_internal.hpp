@@ -158,6 +158,12 @@ struct GridArgs {
     // first 0)
     const uint8_t *rowmask, *colmask;
     int32_t *tile_list;
+    // W-stacking with crowd_min > 0: parts of the grid that at least so many
+    // points reach are left to launch_grid, as tiles in crowd_list (ntiles + 1
+    // ints, the first 0); the sparse gridder builds it beside tile_list, which
+    // is then always there
+    int crowd_min;
+    int32_t *crowd_list;
     // learned kernel (learned != 0): the value at offset d is
     // exp(beta sqrt(1 - es_c d^2) + sum_k kq[k] s^k), s = 2 es_c d^2 - 1,
     // instead of the ES kernel's exp(beta sqrt(1 - es_c d^2))
@@ -193,9 +199,11 @@ bool grid2d_mfma_supported(const GridArgs &g, int kw);
 // needs sparse_blocks + 1 ints, the first of them 0 on entry of the call whose
 // slab starts at plane 0; it builds the list, the other slabs' calls use it.
 int64_t sparse_blocks(int nf1, int nf2);
+bool sparse_crowdable(const GridArgs &g);
 template <typename T>
 int launch_grid_sparse(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *tile_start,
                        cx_t<T> *fw, const GridArgs &g, int kw, hipStream_t s);
+// a 2-D grid, or with nf3 > 1 the tiles of tile_list
 template <typename T>
 int launch_grid(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *tile_start,
                 cx_t<T> *fw, const GridArgs &g, int kw, hipStream_t s);

@@ -21,7 +21,9 @@
 // thread per point adding its 13^3 taps to an LDS tile with atomics: 274 ms,
 // the 34 points of a tile on 512 threads); 2500 x 3000 x 10 complex64 cells
 // with 196608 points 0.18 ms (0.52 ms).  Around crowded blocks by the chain of
-// one wave: about 512 cycles of matrix instructions per four points.
+// one wave: 0.14 us per point, 0.55 us per four (their 512 cycles of matrix
+// instructions, and the latency of evaluating their kernel values); where k_grid is
+// faster such regions are left to it.
 #include <type_traits>
 
 #include "cg_kernel.hpp"
@@ -303,24 +305,61 @@ __global__ __launch_bounds__(64 * kSpWaves, 3) void k_grid_sparse(const geo_t<T>
 }
 
 // list[0] = number of 8 x 8 blocks with a masked-in row and a masked-in
-// column, list[1..] = those blocks (any order; each is gridded independently)
-__global__ __launch_bounds__(256) void k_need_blocks(const uint8_t *__restrict__ rowmask,
-                                                     const uint8_t *__restrict__ colmask, int nbx,
-                                                     int nblocks, int nf1, int nf2,
+// column (all without masks), list[1..] = those blocks (any order; each is
+// gridded independently).  With crowd_min > 0 the blocks of a crowded region go
+// to crowd_list as its sort tiles instead.  A region is a block, or the sort tile
+// if that is larger (edges along an axis divide one another), and the points of
+// all bins that can reach it count, those of the dense path aside.
+__global__ __launch_bounds__(256) void k_need_blocks(const int32_t *__restrict__ tile_start, int nbx,
+                                                     int nblocks, GridArgs g, int kw,
                                                      int32_t *__restrict__ list)
 {
     const int t = blockIdx.x * 256 + threadIdx.x;
     if (t >= nblocks) return;
     const int by = t / nbx, bx = t - by * nbx;
-    bool need_r = false, need_c = false;
-    for (int y = by * kBlk; y < min(by * kBlk + kBlk, nf2) && !need_r; y++) need_r = rowmask[y] != 0;
-    for (int x = bx * kBlk; x < min(bx * kBlk + kBlk, nf1) && !need_c; x++) need_c = colmask[x] != 0;
-    if (need_r && need_c) list[1 + atomicAdd(list, 1)] = t;
+    const int x0 = bx * kBlk, x1 = min(x0 + kBlk, g.nf1), y0 = by * kBlk, y1 = min(y0 + kBlk, g.nf2);
+    auto wanted = [&](int xa, int xb, int ya, int yb) -> bool {
+        bool row = !g.rowmask, col = !g.rowmask;
+        for (int y = ya; y < yb && !row; y++) row = g.rowmask[y] != 0;
+        for (int x = xa; x < xb && !col; x++) col = g.colmask[x] != 0;
+        return row && col;
+    };
+    if (g.crowd_min > 0) {
+        const int ex = max(kBlk, g.tx), ey = max(kBlk, g.ty), rx = x0 / ex * ex, ry = y0 / ey * ey;
+        const int nx = min(ex, g.nf1 - rx), ny = min(ey, g.nf2 - ry);
+        if (!wanted(rx, rx + nx, ry, ry + ny)) return;
+        const AxisBins X = axis_bins(rx - (kw - 1), nx + kw - 1, g.nf1, g.tx, g.ntx);
+        const AxisBins Y = axis_bins(ry - (kw - 1), ny + kw - 1, g.nf2, g.ty, g.nty);
+        int64_t n = 0;
+        for (int j = 0; j < Y.nb; j++)
+            for (int i = 0; i < X.nb; i++) {
+                int ty = Y.b0 + j, tx = X.b0 + i;
+                if (ty >= g.nty) ty -= g.nty;
+                if (tx >= g.ntx) tx -= g.ntx;
+                const int bin = ty * g.ntx + tx, c = tile_start[bin + 1] - tile_start[bin];
+                if (g.dense_min <= 0 || c < g.dense_min) n += c;
+            }
+        if (n >= g.crowd_min) {
+            // the tiles that begin in this block
+            for (int ty = (y0 + g.ty - 1) / g.ty; ty * g.ty < y1; ty++)
+                for (int tx = (x0 + g.tx - 1) / g.tx; tx * g.tx < x1; tx++)
+                    g.crowd_list[1 + atomicAdd(g.crowd_list, 1)] = ty * g.ntx + tx;
+            return;
+        }
+    }
+    if (wanted(x0, x1, y0, y1)) list[1 + atomicAdd(list, 1)] = t;
 }
 
 int64_t sparse_blocks(int nf1, int nf2)
 {
     return ceil_div(nf1, kBlk) * ceil_div(nf2, kBlk);
+}
+
+// the blocks and the sort tiles of a crowded region cover the same cells
+bool sparse_crowdable(const GridArgs &g)
+{
+    auto fits = [](int t) { return t % kBlk == 0 || kBlk % t == 0; };
+    return fits(g.tx) && fits(g.ty);
 }
 
 template <typename T>
@@ -333,9 +372,10 @@ int launch_grid_sparse(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *t
     const int nbx = (int)ceil_div(g.nf1, kBlk);
     const int64_t nblocks = sparse_blocks(g.nf1, g.nf2);
     const int nwin = (int)ceil_div(slab_planes(g), kWin);
+    if (g.crowd_min > 0 && (!g.tile_list || !g.crowd_list || !sparse_crowdable(g))) return CG_ERR_ARG;
     if (g.tile_list && g.zb == 0) {
-        hipLaunchKernelGGL(k_need_blocks, dim3((unsigned)ceil_div(nblocks, 256)), dim3(256), 0, s,
-                           g.rowmask, g.colmask, nbx, (int)nblocks, g.nf1, g.nf2, g.tile_list);
+        hipLaunchKernelGGL(k_need_blocks, dim3((unsigned)ceil_div(nblocks, 256)), dim3(256), 0, s, ts, nbx,
+                           (int)nblocks, g, kw, g.tile_list);
         CG_HIP(hipGetLastError());
     }
     // (a short list, split by row pairs, has four times as many items)

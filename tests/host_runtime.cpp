@@ -358,6 +358,40 @@ void tile_edges(const Lib &L)
         }
 }
 
+// ms2dirty calls by whether crowded regions may go to k_grid
+void crowded_rule(const Lib &L)
+{
+    const auto create = L.sym<int (*)(void **, void *)>("cg_ctx_create");
+    const auto option = L.sym<int (*)(void *, const char *, int)>("cg_ctx_set_option");
+    const auto run = L.sym<int (*)(void *, int, int, int, int, double, double, const void *, int, const void *,
+                                   const void *, int, void *, double, double, int)>("cg_ms2dirty_dev");
+    const int most = 50000;
+    void *uvw = nullptr, *vis = nullptr, *img = nullptr;
+    (void)take(&uvw, (size_t)24 * most, false);
+    (void)take(&vis, (size_t)16 * most, false);
+    (void)take(&img, (size_t)16 * 64 * 64, false);
+    auto call = [&](const char *name, int prec, int rows, int nx, int kw, int tile, int dense) {
+        void *ctx = nullptr;
+        (void)create(&ctx, nullptr);
+        option(ctx, "tile_grid", tile);
+        option(ctx, "dense_min", dense);
+        launches.clear();
+        const int ier = run(ctx, prec, rows, nx, nx, 5.0, 1e9, uvw, 1, vis, nullptr, prec, img,
+                            std::pow(10.0, 1 - kw) * 1.01, 2.0, -1);
+        show(name, ier ? -ier : launched("6k_gridI"));
+        L.sym<int (*)(void *)>("cg_ctx_destroy")(ctx);
+    };
+    call("narrow", 1, 1000, 64, 4, 8, 64);
+    call("few_rows", 1, 200, 64, 4, 8, 64);
+    call("width8_tile8", 1, most, 64, 8, 8, 64);
+    call("width8_tile2", 1, most, 25, 8, 8, 64);
+    call("width13", 1, most, 25, 13, 8, 64);
+    call("odd_tile", 1, 1000, 60, 4, 12, 64);
+    call("dense", 0, most, 64, 4, 8, 64);
+    call("no_dense", 0, most, 64, 4, 8, 0);
+    call("late_dense", 0, most, 64, 4, 8, 100000);
+}
+
 // what two calls leave allocated
 void kept_bytes(const Lib &L)
 {
@@ -427,6 +461,7 @@ int main(int argc, char **argv)
     else if (what == "device_reset") device_reset(L);
     else if (what == "kept_bytes") kept_bytes(L);
     else if (what == "tile_edges") tile_edges(L);
+    else if (what == "crowded_rule") crowded_rule(L);
     else if (what == "surplus") surplus(L);
     else return 2;
     show("bad_frees", bad_frees);

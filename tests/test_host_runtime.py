@@ -103,3 +103,14 @@ def test_tile_edges_stay_accepted(scenario):
     for tile in (0, 1, 2, 3, 5, 8, 12):
         for kw in (4, 9, 10, 13):
             assert r[f"tile{tile}_kw{kw}"] == (3 if tile < 2 and kw > 9 else 0)
+
+
+def test_crowded_rule(scenario):
+    """k_grid takes crowded regions where it is the faster one and nothing else
+    does: narrow kernels or small tiles, enough rows for a region to be crowded,
+    no dense path below that, tiles and blocks that cover the same cells."""
+    r = scenario("crowded_rule")
+    for name in ("narrow", "width8_tile2", "no_dense", "late_dense"):
+        assert r[name] == 1, name
+    for name in ("few_rows", "width8_tile8", "width13", "odd_tile", "dense"):
+        assert r[name] == 0, name
