@@ -14,7 +14,7 @@
 // Columns: a short column (n2 <= 128, or a length with no usable split) is
 // transformed whole by a workgroup holding a block of adjacent columns.  A
 // long column uses the in-place four-step split n2 = na * nb on blocks of 64
-// adjacent columns: step A
+// (fp32) / 32 (fp64) adjacent columns, i.e. 512-byte row segments: step A
 // transforms the na-point sub-columns of stride nb and applies the twiddles
 // w^(b ka); step B transforms the nb-point contiguous sub-columns.  Without a
 // transposition the spectrum of a split column lands in "split order":
@@ -69,34 +69,46 @@ __device__ __forceinline__ TwTab<T> load_twtab(cx_t<T> *lds, const cx_t<T> *__re
     return TwTab<T>{lds + B, lds, sh};
 }
 
-// LDS position of element x of a row: one slot of padding per 32
-__device__ __forceinline__ int ct_pos(int x) { return x + (x >> 5); }
+template <int NB, bool BFAST, int N, bool PAD>
+__device__ __forceinline__ int ct_pos(int b, int e)
+{
+    if constexpr (BFAST) return b + e * NB;
+    const int x = b * N + e;
+    return PAD ? x + (x >> 5) : x;
+}
 
-// one Stockham pass of radix R over a row of length N held in LDS, NT threads
-template <typename T, int DIR, int N, int R, int P, int NT>
-__device__ __forceinline__ void ct_pass(cx_t<T> *buf, const TwTab<T> &tab)
+// one Stockham pass of radix R over NB transforms of length N held in LDS,
+// NT threads; twiddle w_N^t read as tab.get(t * ts) (tab may describe a
+// longer transform whose length is ts * N)
+template <typename T, int DIR, int N, int R, int P, int NB, bool BFAST, bool PAD, int NT>
+__device__ __forceinline__ void ct_pass(cx_t<T> *buf, const TwTab<T> &tab, int ts)
 {
     constexpr int TN = N / R;
-    constexpr int K = (TN + NT - 1) / NT;
+    constexpr int NBF = NB * TN;
+    constexpr int K = (NBF + NT - 1) / NT;
     constexpr int TWS = N / (P * R);
     cx_t<T> u[K][R];
 #pragma unroll
     for (int k = 0; k < K; k++) {
-        const int i = threadIdx.x + k * NT;
-        if (TN % NT == 0 || i < TN) {
+        const int q = threadIdx.x + k * NT;
+        if (NBF % NT == 0 || q < NBF) {
+            const int b = BFAST ? q % NB : q / TN;
+            const int i = BFAST ? q / NB : q % TN;
 #pragma unroll
-            for (int r = 0; r < R; r++) u[k][r] = buf[ct_pos(i + r * TN)];
+            for (int r = 0; r < R; r++) u[k][r] = buf[ct_pos<NB, BFAST, N, PAD>(b, i + r * TN)];
         }
     }
     lds_barrier();
 #pragma unroll
     for (int k = 0; k < K; k++) {
-        const int i = threadIdx.x + k * NT;
-        if (TN % NT == 0 || i < TN) {
+        const int q = threadIdx.x + k * NT;
+        if (NBF % NT == 0 || q < NBF) {
+            const int b = BFAST ? q % NB : q / TN;
+            const int i = BFAST ? q / NB : q % TN;
             const int kk = i % P;
             if constexpr (P > 1) {
                 // W^r for r = 4 r1 + r2 as (W^4)^r1 W^r2: two table lookups
-                cx_t<T> w1 = tab.get(kk * TWS);
+                cx_t<T> w1 = tab.get(kk * TWS * ts);
                 if (DIR < 0) w1.y = -w1.y;
                 const cx_t<T> w2 = cmul<T>(w1, w1);
                 const cx_t<T> pw[4] = {mkc((T)1, (T)0), w1, w2, cmul<T>(w2, w1)};
@@ -104,7 +116,7 @@ __device__ __forceinline__ void ct_pass(cx_t<T> *buf, const TwTab<T> &tab)
 #pragma unroll
                     for (int r = 1; r < R; r++) u[k][r] = cmul<T>(u[k][r], pw[r]);
                 } else {
-                    cx_t<T> w4 = tab.get(4 * kk * TWS);
+                    cx_t<T> w4 = tab.get(4 * kk * TWS * ts);
                     if (DIR < 0) w4.y = -w4.y;
                     const cx_t<T> w8 = cmul<T>(w4, w4);
                     const cx_t<T> qw[4] = {mkc((T)1, (T)0), w4, w8, cmul<T>(w8, w4)};
@@ -120,16 +132,27 @@ __device__ __forceinline__ void ct_pass(cx_t<T> *buf, const TwTab<T> &tab)
             dft_small<T, R, DIR>(u[k]);
             const int j = (i - kk) * R + kk;
 #pragma unroll
-            for (int r = 0; r < R; r++) buf[ct_pos(j + r * P)] = u[k][r];
+            for (int r = 0; r < R; r++) buf[ct_pos<NB, BFAST, N, PAD>(b, j + r * P)] = u[k][r];
         }
     }
     lds_barrier();
 }
 
+// all passes: radix RMAX while possible, then the remainder
+template <typename T, int DIR, int N, int P, int NB, bool BFAST, bool PAD, int NT, int RMAX>
+__device__ __forceinline__ void ct_fft(cx_t<T> *buf, const TwTab<T> &tab, int ts)
+{
+    if constexpr (P < N) {
+        constexpr int R = (N / P) >= RMAX ? RMAX : (N / P);
+        ct_pass<T, DIR, N, R, P, NB, BFAST, PAD, NT>(buf, tab, ts);
+        ct_fft<T, DIR, N, P * R, NB, BFAST, PAD, NT, RMAX>(buf, tab, ts);
+    }
+}
+
 template <typename T>
 constexpr int ct_rmax() { return sizeof(T) == 4 ? 16 : 8; }
 
-// one row of N held in padded LDS: every pass but the last, then
+// one row of N held in padded LDS (NB = 1): every pass but the last, then
 // the last pass from LDS into registers, its outputs x = i + r P handed to
 // out(x, value) instead of written back (P = N / R is a multiple of NT, so
 // the thread's outputs are its own columns x = threadIdx.x + u NT)
@@ -138,7 +161,7 @@ __device__ __forceinline__ void ct_fft_row_out(cx_t<T> *buf, const TwTab<T> &tab
 {
     constexpr int R = (N / P) >= RMAX ? RMAX : (N / P);
     if constexpr (P * R < N) {
-        ct_pass<T, DIR, N, R, P, NT>(buf, tab);
+        ct_pass<T, DIR, N, R, P, 1, false, true, NT>(buf, tab, 1);
         ct_fft_row_out<T, DIR, N, P * R, NT, RMAX>(buf, tab, out);
     } else {
         static_assert(P > 1 && P % NT == 0, "last pass layout");
@@ -289,15 +312,105 @@ __global__ __launch_bounds__((1 << LOGN) / fft_ept<T>()) void k_fft_rows_ct(cx_t
     }
 }
 
+// One step of the split column FFT with sub-transform length L = 2^LOGL on
+// CB adjacent live columns, complex128 (see k_fft_cols_mix for the arguments; tw2
+// is the length-n2 table) as a persistent kernel: a workgroup walks tiles (column
+// block x fastest, then sub-transform j, then plane) and loads the next
+// tile into registers while the current one is transformed in LDS and
+// stored, so the loads in flight are not limited to what fits in LDS.  Steps on
+// less than 1 GiB and long ones take it (cols_pf_faster).
+template <int DIR, int LOGL, int CB>
+__global__ __launch_bounds__(CB * (1 << LOGL) / fft_ept<double>()) void k_fft_cols_step_pf(
+    double2 *data, int n2, int n1, int se, int sj, int nsub, int batch, int twmode,
+    const double2 *__restrict__ tw2, Live live, const uint8_t *__restrict__ rowmask, int mode_in,
+    int mode_out, int spec_a, int spec_b)
+{
+    using T = double;
+    constexpr int L = 1 << LOGL;
+    constexpr int EPT = fft_ept<T>();
+    constexpr int E = CB * L;
+    constexpr int NT = E / EPT;
+    constexpr int SH2 = 7;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    cx_t<T> *buf = reinterpret_cast<cx_t<T> *>(smem_raw);
+    const TwTab<T> tab = load_twtab<T>(buf + E, tw2, n2, SH2);
+    lds_barrier();
+    const int nlive = live.count(n1);
+    const int nx = (nlive + CB - 1) / CB;
+    const int64_t ntile = (int64_t)nx * nsub * batch;
+    const int tstride = n2 >> LOGL;
+    auto dead = [&](int j, size_t row, int e) -> bool {
+        if (sj == 1) return rowmask && !rowmask[row];
+        const int k = j + nsub * e;
+        return k >= spec_a && k < spec_b;
+    };
+    cx_t<T> pre[EPT];
+    auto load = [&](int64_t t) {
+        const int x = (int)(t % nx);
+        const int64_t r = t / nx;
+        const int j = (int)(r % nsub);
+        const cx_t<T> *pl = data + (size_t)(r / nsub) * n2 * n1;
+        const size_t row0 = (size_t)j * sj;
+#pragma unroll
+        for (int u = 0; u < EPT; u++) {
+            const int k = threadIdx.x + u * NT;
+            const int e = k / CB, b = k % CB;
+            const int c = x * CB + b;
+            const size_t row = row0 + (size_t)e * se;
+            const bool rd = c < nlive && !(mode_in && dead(j, row, e));
+            pre[u] = rd ? pl[row * n1 + live.at(c)] : mkc((T)0, (T)0);
+        }
+    };
+    int64_t t = blockIdx.x;
+    if (t < ntile) load(t);
+    for (; t < ntile; t += gridDim.x) {
+        const int x = (int)(t % nx);
+        const int64_t r = t / nx;
+        const int j = (int)(r % nsub);
+        cx_t<T> *pl = data + (size_t)(r / nsub) * n2 * n1;
+        const size_t row0 = (size_t)j * sj;
+#pragma unroll
+        for (int u = 0; u < EPT; u++) {
+            const int k = threadIdx.x + u * NT;
+            cx_t<T> v = pre[u];
+            if (twmode == 2) {
+                cx_t<T> w = tab.get(j * (k / CB));
+                if (DIR < 0) w.y = -w.y;
+                v = cmul<T>(v, w);
+            }
+            buf[k] = v;
+        }
+        if (t + gridDim.x < ntile) load(t + gridDim.x);
+        lds_barrier();
+        ct_fft<T, DIR, L, 1, CB, true, false, NT, ct_rmax<T>()>(buf, tab, tstride);
+#pragma unroll
+        for (int u = 0; u < EPT; u++) {
+            const int k = threadIdx.x + u * NT;
+            const int e = k / CB, b = k % CB;
+            const int c = x * CB + b;
+            if (c >= nlive) continue;
+            const size_t row = row0 + (size_t)e * se;
+            if (mode_out && dead(j, row, e)) continue;
+            cx_t<T> v = buf[k];
+            if (twmode == 1) {
+                cx_t<T> w = tab.get(j * e);
+                if (DIR < 0) w.y = -w.y;
+                v = cmul<T>(v, w);
+            }
+            pl[row * n1 + live.at(c)] = v;
+        }
+        lds_barrier();
+    }
+}
+
 // One step of the split column FFT with sub-transform length L = 2^LOGL on CB
 // adjacent live columns (see k_fft_cols_mix for the arguments; tw2 is the
 // length-n2 table), fp32 and L = 16 R2 (R2 = 2..16), as a persistent kernel: a
 // workgroup walks tiles (column block x fastest, then sub-transform j, then
 // plane) and loads the next tile into registers while the current one is
 // transformed and stored.  It is a little faster than k_fft_cols_mix
-// there (2-D transforms of 2^25 points on an 8192^2 grid: 7.14 against 7.20 ms); fp64
-// and shorter lengths take that one (complex128 4096^2 x 194 inverse: 50.1 ms
-// the call with a prefetching fp64 form of this kernel, 45.0 ms).
+// there (2-D transforms of 2^25 points on an 8192^2 grid: 7.14 against 7.20 ms);
+// shorter lengths take that one.
 // Two passes:
 // thread t holds column b = t % CB at rows e0 + (L/16) u, u < 16
 // (e0 = t / CB), which are exactly the inputs of the first radix-16
@@ -893,6 +1006,38 @@ static int cols_step_ct(float2 *data, int batch, int n2, int n1, int se, int sj,
     return CG_OK;
 }
 
+// complex128: k_fft_cols_mix is the faster one where HBM bounds the step and a
+// block of its 64 columns leaves two workgroups on a CU; else the twice as many
+// tiles of k_fft_cols_step_pf are.  Column stage of dirty2ms, pf / mix: 1024^2
+// cells x 16 planes 0.091 / 0.127 ms, 2048^2 x 26 (0.9 GB) 0.48 / 0.59, 4096^2 x 8
+// (1.07 GB) 0.74 / 0.68, 4096^2 x 26 2.4 / 2.0, 8192^2 x 16 (L = 128, blocks of 32
+// columns) 5.5 / 6.1.
+static bool cols_pf_faster(int batch, int n2, int nlive, int L)
+{
+    return (64 * L * 16 > 81920) || (int64_t)batch * n2 * nlive * 16 < (int64_t)1 << 30;
+}
+
+template <int DIR, int LOGL>
+static int cols_step_pf(double2 *data, int batch, int n2, int n1, int se, int sj, int nsub, int twmode,
+                        const double2 *tw2, Live live, const DeadRows &dr, hipStream_t s)
+{
+    constexpr int L = 1 << LOGL;
+    constexpr int CB = 32 * L * 16 <= 65536 ? 32 : 65536 / (L * 16);
+    constexpr int NT = CB * L / fft_ept<double>();
+    const size_t lds = (size_t)(CB * L + 128 + (n2 + 127) / 128) * sizeof(double2);
+    if (lds > 65536)
+        CG_HIP(hipFuncSetAttribute((const void *)k_fft_cols_step_pf<DIR, LOGL, CB>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const int64_t ntile = (int64_t)((live.count(n1) + CB - 1) / CB) * nsub * batch;
+    const int per_cu = std::max(1, std::min((int)(kLdsMax / lds), 2048 / NT));
+    const int64_t grid = std::min<int64_t>(ntile, (int64_t)256 * per_cu);
+    hipLaunchKernelGGL((k_fft_cols_step_pf<DIR, LOGL, CB>), dim3((unsigned)grid), dim3(NT), lds, s, data, n2,
+                       n1, se, sj, nsub, batch, twmode, tw2, live, dr.rowmask, dr.mode_in, dr.mode_out,
+                       dr.spec_a, dr.spec_b);
+    CG_HIP(hipGetLastError());
+    return CG_OK;
+}
+
 template <typename T, int DIR>
 static int cols_step_ct_dispatch(cx_t<T> *data, int batch, int n2, int n1, int L, int se, int sj,
                                  int nsub, int twmode, const cx_t<T> *tw2, Live live,
@@ -904,6 +1049,14 @@ static int cols_step_ct_dispatch(cx_t<T> *data, int batch, int n2, int n1, int L
         case 6: return cols_step_ct<DIR, 6>(data, batch, n2, n1, se, sj, nsub, twmode, tw2, live, d, s);
         case 7: return cols_step_ct<DIR, 7>(data, batch, n2, n1, se, sj, nsub, twmode, tw2, live, d, s);
         case 8: return cols_step_ct<DIR, 8>(data, batch, n2, n1, se, sj, nsub, twmode, tw2, live, d, s);
+        default: break;
+        }
+    } else if (cols_pf_faster(batch, n2, live.count(n1), L)) {
+        switch (log2_exact(L)) {
+        case 4: return cols_step_pf<DIR, 4>(data, batch, n2, n1, se, sj, nsub, twmode, tw2, live, d, s);
+        case 5: return cols_step_pf<DIR, 5>(data, batch, n2, n1, se, sj, nsub, twmode, tw2, live, d, s);
+        case 6: return cols_step_pf<DIR, 6>(data, batch, n2, n1, se, sj, nsub, twmode, tw2, live, d, s);
+        case 7: return cols_step_pf<DIR, 7>(data, batch, n2, n1, se, sj, nsub, twmode, tw2, live, d, s);
         default: break;
         }
     }

@@ -392,6 +392,26 @@ void crowded_rule(const Lib &L)
     call("late_dense", 0, most, 64, 4, 8, 100000);
 }
 
+// the column steps of complex128 transforms: steps on the prefetching kernel
+void column_rule(const Lib &L)
+{
+    const auto create = L.sym<int (*)(void **, void *)>("cg_ctx_create");
+    const auto fft = L.sym<int (*)(void *, int, void *, int, int, int, int)>("cg_fft2d_dev");
+    void *ctx = nullptr, *data = nullptr;
+    (void)create(&ctx, nullptr);
+    (void)take(&data, (size_t)4 << 30, false);
+    const int shapes[][4] = {{1, 1, 1024, 1024}, {1, 16, 2048, 1024}, {1, 16, 2048, 2048}, {1, 17, 4096, 2048},
+                             {1, 16, 8192, 2048}, {1, 1, 1000, 1024}, {0, 1, 1024, 1024}};
+    for (const auto &s : shapes) {
+        launches.clear();
+        const int ier = fft(ctx, s[0], data, s[1], s[2], s[3], 1);
+        char name[64];
+        std::snprintf(name, sizeof name, "p%d_%dx%dx%d", s[0], s[1], s[2], s[3]);
+        show(name, ier ? -ier : launched("k_fft_cols_step_pf"));
+    }
+    L.sym<int (*)(void *)>("cg_ctx_destroy")(ctx);
+}
+
 // what two calls leave allocated
 void kept_bytes(const Lib &L)
 {
@@ -462,6 +482,7 @@ int main(int argc, char **argv)
     else if (what == "kept_bytes") kept_bytes(L);
     else if (what == "tile_edges") tile_edges(L);
     else if (what == "crowded_rule") crowded_rule(L);
+    else if (what == "column_rule") column_rule(L);
     else if (what == "surplus") surplus(L);
     else return 2;
     show("bad_frees", bad_frees);

@@ -114,3 +114,14 @@ def test_crowded_rule(scenario):
         assert r[name] == 1, name
     for name in ("few_rows", "width8_tile8", "width13", "odd_tile", "dense"):
         assert r[name] == 0, name
+
+
+def test_column_rule(scenario):
+    """complex128 column steps of powers of two take the prefetching kernel
+    below a gibibyte and at lengths whose mixed-radix blocks are narrow."""
+    r = scenario("column_rule")
+    for name in ("p1_1x1024x1024", "p1_16x2048x1024"):
+        assert r[name] == 2, name
+    assert r["p1_16x8192x2048"] == 1  # of its steps of 64 and 128 points
+    for name in ("p1_16x2048x2048", "p1_17x4096x2048", "p1_1x1000x1024", "p0_1x1024x1024"):
+        assert r[name] == 0, name
