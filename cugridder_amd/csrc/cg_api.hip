@@ -425,7 +425,7 @@ static int grid_masks(Ctx &C, GridArgs &g, const uint8_t *mask, int nf1, int nf2
 static int crowd_min(const WPlan &P, const GridArgs &g, int planes)
 {
     const int kw = P.conv.kw, windows = (planes + 15) / 16;
-    if (!P.wstack || kw > 11 || !sparse_crowdable(g)) return 0;
+    if (!P.wstack || kw > kCrowdKW || !sparse_crowdable(g)) return 0;
     const double share = windows == 1 ? 1.0 : (kw + 15) / (16.0 * windows);
     const int taps = std::min(kw, g.tx) * std::min(kw, g.ty) * kw;
     const double cost = (0.27 + 0.0018 * taps) * (kw > 9 ? 1.4 : 1.0);

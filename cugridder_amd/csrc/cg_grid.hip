@@ -65,11 +65,17 @@ __device__ __forceinline__ Span tile_span(int r, int t, int n)
     return sp;
 }
 
-template <typename T, int KW>
+// PLANES: W-stacking (the 2-D form is free of the plane loop's registers).  WRAP:
+// one tile along an axis, whose footprints wrap inside it; without, a tap is an
+// immediate offset from the footprint's first cell.  With the x masks besides,
+// complex128 type 1, 3e5 clustered points on 1024^2 cells, kw 8 / 13: 6.8 / 12.9 ms,
+// with wrap positions and masks per tap in a 2-D form 7.9 / 16.6, as the plane
+// loop of one form for both 7.0 / 29.
+template <typename T, int KW, bool PLANES, bool WRAP>
 __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
                                                const cx_t<T> *__restrict__ val,
                                                const int32_t *__restrict__ tile_start,
-                                               cx_t<T> *__restrict__ fw, GridArgs g, int is2d)
+                                               cx_t<T> *__restrict__ fw, GridArgs g)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     double *acc = reinterpret_cast<double *>(smem_raw);
@@ -78,15 +84,15 @@ __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
     // work item = (tile, plane chunk): one per workgroup, or, with a tile
     // list (the tiles some FFT pass reads, or the crowded ones), the
     // workgroups walk the list
-    const int nwork = g.tile_list ? g.tile_list[0] * g.nchunk : (int)gridDim.x;
+    const int nchunk = PLANES ? g.nchunk : 1;
+    const int nwork = g.tile_list ? g.tile_list[0] * nchunk : (int)gridDim.x;
     for (int wi = blockIdx.x; wi < nwork; wi += gridDim.x) {
-    const int chunk = wi % g.nchunk;
-    const int tile = g.tile_list ? g.tile_list[1 + wi / g.nchunk] : wi / g.nchunk;
+    const int chunk = PLANES ? wi % nchunk : 0;
+    const int tile = g.tile_list ? g.tile_list[1 + wi / nchunk] : wi / nchunk;
     const int bx = tile % g.ntx, by = tile / g.ntx;
     // planes [p0, p0 + np) of the slab [zb, zb + zn) held by the buffer
-    const int zn = slab_planes(g);
-    const int p0 = g.zb + chunk * g.pc;
-    const int np = min(g.pc, g.zb + zn - p0);
+    const int p0 = PLANES ? g.zb + chunk * g.pc : 0;
+    const int np = PLANES ? min(g.pc, g.zb + slab_planes(g) - p0) : 1;
     const int cells = np * g.ty * g.tx;
     for (int k = threadIdx.x; k < 2 * cells; k += blockDim.x) acc[k] = 0.0;
     // source bins whose footprints can reach this tile: bin (bx - sx, by - sy)
@@ -105,7 +111,7 @@ __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
             s_beg[b] = tile_start[sidx];
             s_cnt[b] = tile_start[sidx + 1] - s_beg[b];
             // dense bins are added afterwards by k_grid_dense2
-            if (g.dense_min > 0 && s_cnt[b] >= g.dense_min) s_cnt[b] = 0;
+            if (PLANES && g.dense_min > 0 && s_cnt[b] >= g.dense_min) s_cnt[b] = 0;
             s_ox[b] = ox;
             s_oy[b] = oy;
             tot += s_cnt[b];
@@ -136,7 +142,7 @@ __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
         const Span Y = tile_span<KW>(ry, g.ty, g.nf2);
         if (X.lo >= X.hi || Y.lo >= Y.hi) continue;
         Span Z{0, 0, 1};
-        if (!is2d) {
+        if constexpr (PLANES) {
             int rz = (int)(pk >> 16) - p0;
             if (rz < 0) rz += g.nf3;
             Z = tile_span<KW>(rz, np, g.nf3);
@@ -149,23 +155,28 @@ __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
             kx[t] = ker(G.x, t);
             ky[t] = ker(G.y, t);
         }
+        // the lanes whose tap t lands inside the tile along x, as scalar masks
+        uint64_t mx[KW];
+#pragma unroll
+        for (int t = 0; t < KW; t++) mx[t] = __ballot(t >= X.lo && t < X.hi);
         for (int tz = Z.lo; tz < Z.hi; tz++) {
             int zz = Z.s + tz;
             if (zz >= np) zz -= np;  // wraps only when one chunk holds every plane
-            const T kz = is2d ? (T)1 : ker(G.z, tz);
+            if (!PLANES) zz = 0;
+            const T kz = PLANES ? ker(G.z, tz) : (T)1;
             const T vzr = v.x * kz, vzi = v.y * kz;
 #pragma unroll
             for (int t2 = 0; t2 < KW; t2++) {
                 if (t2 < Y.lo || t2 >= Y.hi) continue;
                 int yy = Y.s + t2;
-                if (yy >= g.nf2) yy -= g.nf2;  // wraps only with one tile along nf2
+                if (WRAP && yy >= g.nf2) yy -= g.nf2;
                 const T vyr = vzr * ky[t2], vyi = vzi * ky[t2];
                 double *row = acc + (zz * g.ty + yy) * g.tx;
 #pragma unroll
                 for (int t1 = 0; t1 < KW; t1++) {
-                    if (t1 < X.lo || t1 >= X.hi) continue;
+                    if (!__builtin_amdgcn_inverse_ballot_w64(mx[t1])) continue;
                     int xx = X.s + t1;
-                    if (xx >= g.nf1) xx -= g.nf1;
+                    if (WRAP && xx >= g.nf1) xx -= g.nf1;
                     atomicAdd(row + xx, (double)(vyr * kx[t1]));
                     atomicAdd(row + cells + xx, (double)(vyi * kx[t1]));
                 }
@@ -175,10 +186,10 @@ __global__ __launch_bounds__(1024) void k_grid(const geo_t<T> *__restrict__ geo,
     __syncthreads();
     const int plane_cells = g.ty * g.tx;
     for (int k = threadIdx.x; k < cells; k += blockDim.x) {
-        int lz = k / plane_cells;
+        const int lz = PLANES ? k / plane_cells : 0;
         int rem = k - lz * plane_cells;
         int y = rem / g.tx, x = rem - y * g.tx;
-        size_t gi = ((size_t)(p0 - g.zb + lz) * g.nf2 + (size_t)(by * g.ty + y)) * g.nf1 + bx * g.tx + x;
+        size_t gi = ((size_t)(PLANES ? p0 - g.zb + lz : 0) * g.nf2 + (size_t)(by * g.ty + y)) * g.nf1 + bx * g.tx + x;
         fw[gi] = mkc((T)acc[k], (T)acc[cells + k]);
     }
     __syncthreads();  // acc and the bin table are reused by the next item
@@ -422,13 +433,19 @@ static int grid_kw(const geo_t<T> *geo, const cx_t<T> *val, const int32_t *ts, c
             return CG_OK;
         }
     }
-    if (lds > 65536)
-        CG_HIP(hipFuncSetAttribute((const void *)k_grid<T, KW>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((k_grid<T, KW>), dim3(nblk), dim3(grid_threads(lds)), lds, s, geo, val, ts,
-                       fw, g, is2d);
-    CG_HIP(hipGetLastError());
-    return CG_OK;
+    auto go = [&](auto kern) -> int {
+        if (lds > 65536)
+            CG_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)lds));
+        hipLaunchKernelGGL(kern, dim3(nblk), dim3(grid_threads(lds)), lds, s, geo, val, ts, fw, g);
+        CG_HIP(hipGetLastError());
+        return CG_OK;
+    };
+    const bool wrap = g.tx == g.nf1 || g.ty == g.nf2;
+    if (is2d) return wrap ? go(k_grid<T, KW, false, true>) : go(k_grid<T, KW, false, false>);
+    if constexpr (KW <= kCrowdKW)
+        return wrap ? go(k_grid<T, KW, true, true>) : go(k_grid<T, KW, true, false>);
+    return CG_ERR_SIZE;
 }
 
 // ------------------------------------------------------------ dense bins

@@ -191,6 +191,8 @@ struct GridArgs {
 };
 // most source bins feeding one tile: (1 + ceil(15/2))^2 for tiles >= 2
 constexpr int kMaxBins = 81;
+// widest kernel of launch_grid's W-stacking form
+constexpr int kCrowdKW = 11;
 // planes held by the grid buffer
 __host__ __device__ inline int slab_planes(const GridArgs &g) { return g.zn > 0 ? g.zn : g.nf3; }
 bool grid2d_mfma_supported(const GridArgs &g, int kw);
