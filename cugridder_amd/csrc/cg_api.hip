@@ -411,33 +411,47 @@ static int grid_masks(Ctx &C, GridArgs &g, const uint8_t *mask, int nf1, int nf2
 
 // W-stacking: the points that reach a crowded part of the grid go to k_grid, whose
 // workgroups share them; a block of k_grid_sparse takes its points on one wave for
-// every window of 16 planes, 0.14 us a point.  k_grid takes about 0.27 + 0.0018
-// taps inside a tile of that for a point (measured for kw 2 .. 9 and tiles of 2, 4
-// and 8; from kw 10 on its registers spill, from 12 on it is never the faster);
-// its chunks of planes run side by side as the windows do.  Below some hundred
-// points its fixed cost per tile is the larger part, and a few crowded regions
-// leave the rim's chains to k_grid_sparse, which run before it.  complex128, ms per call on k_grid_sparse alone and so: 1024^2
-// cells, 10^6 rows spread over 1 / 20 / 60 cells, kw 2 102 / 2.8 / 1.28,
-// 9.9 / 1.08 / 0.45; kw 6 134 / 5.9 / 2.39, 66 / 5.1 / 1.74; kw 7 136 / 7.3 / 2.76,
-// 94 / 7.4 / 2.30; kw 8, where it does not (with it from 1024 points on),
-// 137 / 8.2 / 3.0, (125 / 10.2 / 3.3).  1250^2 cells, tiles of 2, kw 8, spread over
-// 5 / 20 / 60: 74 / 8.0 / 3.3, 23 / 5.1 / 3.5.
+// every window of 16 planes, 0.14 us a point (complex64 0.08).  cost is about what a
+// point of a tile takes in k_grid, in units of that, by its taps inside the tile
+// (above kw 9 its registers spill, above kCrowdKW it is never the faster); the
+// windows run side by side, but a point reaches only some of them and its taps meet
+// fewer others' the more planes there are, hence the power.  ms per call on 512^2
+// cells, 200000 rows, k_grid_sparse alone and k_grid, the points within 1 / within
+// about 8 cells (tiles of 8; kw: windows 1, 4, 16):
+//   complex128 kw 4: 26.4, 6.0 / 4.0, 2.0   10.5, 5.0 / 2.1, 1.5   4.4, 3.0 / 2.2, 1.9
+//              kw 5: 27.1, 8.5 / 4.8, 3.0   11.5, 7.4 / 2.5, 2.4   4.6, 4.2 / 2.3, 2.6
+//              kw 6: 27.1, 12.0 / 5.6, 4.5  12.2, 10.5 / 3.0, 3.7  4.8, 5.8 / 2.5, 3.3
+//              kw 7: 27.0, 16.9 / 6.5, 6.4  12.9, 15.0 / 3.4, 5.5
+//              kw 8: 27.2, 23.8 / 7.4, 8.9
+//   complex64  kw 3: 4 windows 5.8, 2.8 / 1.4, 0.8   16 windows 3.2, 1.5 / 1.4, 1.0
+//              kw 5: 4 windows 7.0, 7.3 / 1.8, 2.4
+// and with the cluster at the middle of a tile instead of a corner (600^2 cells),
+// complex128, 1 window: kw 6 27.0, 23.4, kw 7 26.8, 39.6 (within 1 cell).  1250^2
+// cells, tiles of 2, kw 8, 10^6 rows within 5 / 20 / 60: 74, 23 / 8.0, 5.1 / 3.3, 3.5.
+// Below some hundred points k_grid's fixed cost per tile is the larger part.
+template <typename T>
 static int crowd_min(const WPlan &P, const GridArgs &g, int planes)
 {
     const int kw = P.conv.kw, windows = (planes + 15) / 16;
     if (!P.wstack || kw > kCrowdKW || !sparse_crowdable(g)) return 0;
-    const double share = windows == 1 ? 1.0 : (kw + 15) / (16.0 * windows);
     const int taps = std::min(kw, g.tx) * std::min(kw, g.ty) * kw;
-    const double cost = (0.27 + 0.0018 * taps) * (kw > 9 ? 1.4 : 1.0);
-    if (cost >= share * g.nchunk) return 0;
-    const int least = (int)((256 << (kw > 7 ? kw - 4 : std::max(0, kw - 5))) / share);
+    const bool dbl = sizeof(T) == 8;
+    const double cost = (dbl ? 0.29 + 0.0020 * taps : 0.284 + 0.0037 * taps) * (kw > 9 ? 1.5 : 1.0);
+    if (cost >= std::pow((double)windows, dbl ? -0.30 : -0.23)) return 0;
+    const double share = windows == 1 ? 1.0 : (kw + 15) / (16.0 * windows) + 0.06;
+    // the chain the other blocks do not hide: short on a GPU full of blocks.  90 x 54
+    // cells, kw 7, 240 points a block: 0.375 ms the call, crowded from 128 points on 0.24
+    const int64_t rows = P.band_len > 0 ? P.band_len : P.nf2, cols = P.cband_len > 0 ? P.cband_len : P.nf1;
+    const bool few = rows * cols * windows <= 64 * 1024;
+    const int least = (int)((few ? (kw > 7 ? 512 : 128) : 256 << (kw > 7 ? kw - 4 : std::max(0, kw - 5))) / share);
     // (the dense path's bins do not count)
     return g.m < least || (g.dense_min > 0 && g.dense_min <= least) ? 0 : least;
 }
 
+template <typename T>
 static int grid_crowded(Ctx &C, const WPlan &P, const Tiling &t, GridArgs &g, int planes)
 {
-    g.crowd_min = crowd_min(P, g, planes);
+    g.crowd_min = crowd_min<T>(P, g, planes);
     if (!g.crowd_min) return CG_OK;
     CG_TRY(ensure(C.clist, sizeof(int32_t) * (size_t)(t.ntiles() + 1)));
     g.crowd_list = as<int32_t>(C.clist);
@@ -806,7 +820,7 @@ static int exec_ms2dirty(Ctx &C, const CallPlan &cp, const TU *uvw, const cx_t<T
     g.kr = key_rect(a);
     g.dense_min = cp.dense_min;
     CG_TRY(grid_masks<T>(C, g, rm, P.nf1, P.nf2));
-    CG_TRY(grid_crowded(C, P, t, g, cp.slab ? cp.slab : P.nf3));
+    CG_TRY(grid_crowded<T>(C, P, t, g, cp.slab ? cp.slab : P.nf3));
     WArgs w = make_wargs(P);
     CG_TRY(image_tables(C, P));
     CallClear clr{rm, rm ? P.nf1 + P.nf2 : 0, {g.tile_list}};

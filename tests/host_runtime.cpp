@@ -2,8 +2,9 @@
 // GPU: the program defines the runtime calls libcurafft.so makes (they take
 // precedence over libamdhip64's), counts and checks allocations, logs kernel
 // launches by name and runs no kernel.  With every kernel skipped the
-// coordinate ranges read back as zero, so a W-stacking call plans the fewest
-// planes of its kernel.
+// coordinate ranges read back as range6 was when the context's memory for them
+// was allocated: zero, for which a W-stacking call plans the fewest planes of its
+// kernel, unless a scenario sets it.
 //
 //   host_runtime LIB SCENARIO
 //
@@ -41,6 +42,7 @@ int bad_frees = 0, bad_copies = 0, allocs = 0;
 size_t fail_size = 0;
 int fail_times = 0;
 bool fail_new = false;  // operator new throws
+double range6[6];       // w, u and v: least and largest
 
 // p lies in a live allocation with `bytes` to go
 bool holds(const void *p, size_t bytes)
@@ -159,7 +161,12 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream
 
 hipError_t hipMalloc(void **p, size_t n) { return take(p, n, false); }
 hipError_t hipFree(void *p) { return give(p); }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return take(p, n, true); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned)
+{
+    const hipError_t e = take(p, n, true);
+    if (e == hipSuccess && n == sizeof range6) std::memcpy(*p, range6, n);
+    return e;
+}
 hipError_t hipHostFree(void *p) { return give(p); }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { return copy(d, s, n, k); }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) { return copy(d, s, n, k); }
@@ -382,14 +389,27 @@ void crowded_rule(const Lib &L)
         L.sym<int (*)(void *)>("cg_ctx_destroy")(ctx);
     };
     call("narrow", 1, 1000, 64, 4, 8, 64);
-    call("few_rows", 1, 200, 64, 4, 8, 64);
+    call("few_rows", 1, 50, 64, 4, 8, 64);
     call("width8_tile8", 1, most, 64, 8, 8, 64);
     call("width8_tile2", 1, most, 25, 8, 8, 64);
     call("width13", 1, most, 25, 13, 8, 64);
+    call("few_rows_wide", 1, 400, 25, 8, 8, 64);
     call("odd_tile", 1, 1000, 60, 4, 12, 64);
     call("dense", 0, most, 64, 4, 8, 64);
     call("no_dense", 0, most, 64, 4, 8, 0);
     call("late_dense", 0, most, 64, 4, 8, 100000);
+    // some 22 and 56 planes (w, u and v in metres)
+    for (int windows : {2, 4})
+        for (int kw : {3, 4, 5, 6, 7}) {
+            const double w = windows == 2 ? 620 : 2000, uv = 95;
+            const double r[6] = {-w, w, -uv, uv, -uv, uv};
+            std::memcpy(range6, r, sizeof r);
+            for (int prec : {0, 1}) {
+                const std::string name = "p" + std::to_string(prec) + "_windows" + std::to_string(windows) + "_kw" +
+                                         std::to_string(kw);
+                call(name.c_str(), prec, most, 64, kw, 8, 0);
+            }
+        }
 }
 
 // the column steps of complex128 transforms: steps on the prefetching kernel

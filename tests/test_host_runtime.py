@@ -112,8 +112,12 @@ def test_crowded_rule(scenario):
     r = scenario("crowded_rule")
     for name in ("narrow", "width8_tile2", "no_dense", "late_dense"):
         assert r[name] == 1, name
-    for name in ("few_rows", "width8_tile8", "width13", "odd_tile", "dense"):
+    for name in ("few_rows", "few_rows_wide", "width8_tile8", "width13", "odd_tile", "dense"):
         assert r[name] == 0, name
+    # several windows of planes: narrower kernels only, complex64's narrower still
+    for prec, windows, widest in ((1, 2, 6), (1, 4, 5), (0, 2, 5), (0, 4, 4)):
+        for kw in (3, 4, 5, 6, 7):
+            assert r[f"p{prec}_windows{windows}_kw{kw}"] == (kw <= widest), (prec, windows, kw)
 
 
 def test_column_rule(scenario):
