@@ -971,22 +971,28 @@ static int plan_dirty2ms(Ctx &C, CallPlan &cp, int64_t nrow, int nchan, const do
     return cp.ier;
 }
 
-// Degridding tiles with fewer points than this are read straight from the
-// planes instead of staged in LDS.  With uniform points, 120 per 16 x 16 tile:
-// 2.86 against 3.49 ms per complex64 call (1024^2, eps 1e-5), 32 per tile 0.34
-// against 0.40 ms; 488 per tile 3.47 against 2.68 ms.  complex128 at eps 1e-12
-// with 15 per tile 50 against 165 ms, no difference at 256 to 512.  When the
-// tiles the points reach hold kDegridStagedFrom points on average, the few
-// sparse ones at the rim are not worth a launch (131072 Gaussian points, 360
-// per tile: 365 against 360 us).
-constexpr int kDegridDirectBelow = 256, kDegridStagedFrom = 128;
-
+// Degridding tiles with fewer points than the result are read straight from the
+// planes instead of staged in LDS: twice the mean count per tile the points reach
+// from which staging is the faster one, or 1 when the mean is above that (the few
+// sparse tiles at the rim are then not worth a launch: 131072 Gaussian points, 360
+// per tile: 365 against 360 us).  Staging reads a tile's whole halo, so that the
+// mean falls with the tile: with uniform points the calls are even at 57 (kw 6),
+// 65 (8), 60 (9), 48 (10) and 62 (11) points per tile of 4 x 4 cells, 115 at kw 12,
+// whose staged form spills; at 30 (9), 60 (11, 12) and 115 (13) of 2 x 2; at 108 (6),
+// 80 (9) and 108 (10) of 8 x 8.  Tiles of 16 x 16: 120 per tile 2.86 against 3.49 ms
+// per complex64 call (1024^2, eps 1e-5), 488 per tile 3.47 against 2.68 ms;
+// complex128 at eps 1e-12 with 15 per tile 50 against 165 ms, no difference at 256
+// to 512.
 static int degrid_direct_below(const WPlan &P, const Tiling &t, int64_t M)
 {
     if (!P.wstack) return 1;
     const int64_t rows = P.band_len > 0 ? P.band_len : P.nf2, cols = P.cband_len > 0 ? P.cband_len : P.nf1;
     const int64_t tiles = ceil_div(rows, t.ty) * ceil_div(cols, t.tx);
-    return M < tiles * kDegridStagedFrom ? kDegridDirectBelow : 1;
+    const int kw = P.conv.kw;
+    const double edge = std::sqrt((double)t.tx * t.ty);
+    const int staged_from =
+        (int)std::min(128.0, (16.0 + 8.0 * edge) * 8.0 / std::min(kw, 8) * (1 << std::max(0, kw - 11)));
+    return M < tiles * staged_from ? 2 * staged_from : 1;
 }
 
 template <typename T, typename TU, typename TW>

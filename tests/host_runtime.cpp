@@ -412,6 +412,35 @@ void crowded_rule(const Lib &L)
         }
 }
 
+// dirty2ms calls by whether tiles with few points are read straight from the planes
+void degrid_rule(const Lib &L)
+{
+    const auto create = L.sym<int (*)(void **, void *)>("cg_ctx_create");
+    const auto option = L.sym<int (*)(void *, const char *, int)>("cg_ctx_set_option");
+    const auto run = L.sym<int (*)(void *, int, int, int, int, double, double, const void *, int, void *,
+                                   const void *, int, const void *, double, double, int)>("cg_dirty2ms_dev");
+    const int most = 130 * 4096;
+    void *uvw = nullptr, *vis = nullptr, *img = nullptr;
+    (void)take(&uvw, (size_t)24 * most, false);
+    (void)take(&vis, (size_t)16 * most, false);
+    (void)take(&img, (size_t)16 * 64 * 64, false);
+    const double r[6] = {-10, 10, -108, 108, -108, 108};  // u and v reach the whole grid
+    std::memcpy(range6, r, sizeof r);
+    for (int tile : {2, 4, 8, 16})
+        for (int kw : {4, 6, 9, 11, 13})
+            for (int per : {10, 25, 40, 70, 90, 120, 130}) {
+                void *ctx = nullptr;
+                (void)create(&ctx, nullptr);
+                option(ctx, "tile_degrid", tile);
+                launches.clear();
+                const int ier = run(ctx, 1, per * (128 / tile) * (128 / tile), 64, 64, 5.0, 1e9, uvw, 1, vis,
+                                    nullptr, 1, img, std::pow(10.0, 1 - kw) * 1.01, 2.0, -1);
+                show(("tile" + std::to_string(tile) + "_kw" + std::to_string(kw) + "_" + std::to_string(per)).c_str(),
+                     ier ? -ier : launched("k_degrid_direct"));
+                L.sym<int (*)(void *)>("cg_ctx_destroy")(ctx);
+            }
+}
+
 // the column steps of complex128 transforms: steps on the prefetching kernel
 void column_rule(const Lib &L)
 {
@@ -502,6 +531,7 @@ int main(int argc, char **argv)
     else if (what == "kept_bytes") kept_bytes(L);
     else if (what == "tile_edges") tile_edges(L);
     else if (what == "crowded_rule") crowded_rule(L);
+    else if (what == "degrid_rule") degrid_rule(L);
     else if (what == "column_rule") column_rule(L);
     else if (what == "surplus") surplus(L);
     else return 2;

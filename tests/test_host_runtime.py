@@ -120,6 +120,21 @@ def test_crowded_rule(scenario):
             assert r[f"p{prec}_windows{windows}_kw{kw}"] == (kw <= widest), (prec, windows, kw)
 
 
+def test_degrid_rule(scenario):
+    """Tiles are read straight from the planes up to the mean number of points per
+    tile from which staging them is the faster: fewer the smaller the tile and the
+    wider the kernel, as the halo read for them grows, and more from width 12 on,
+    where the staged kernel spills."""
+    r = scenario("degrid_rule")
+    until = {(2, 4): 40, (2, 6): 40, (2, 9): 25, (2, 11): 25, (2, 13): 120,
+             (4, 4): 90, (4, 6): 40, (4, 9): 40, (4, 11): 40, (4, 13): 120,
+             (8, 4): 120, (8, 6): 90, (8, 9): 70, (8, 11): 70, (8, 13): 120,
+             (16, 4): 120, (16, 6): 120, (16, 9): 120, (16, 11): 120, (16, 13): 120}
+    for (tile, kw), most in until.items():
+        for per in (10, 25, 40, 70, 90, 120, 130):
+            assert r[f"tile{tile}_kw{kw}_{per}"] == (per <= most), (tile, kw, per)
+
+
 def test_column_rule(scenario):
     """complex128 column steps of powers of two take the prefetching kernel
     below a gibibyte and at lengths whose mixed-radix blocks are narrow."""
