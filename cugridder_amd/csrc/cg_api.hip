@@ -413,8 +413,8 @@ static int grid_masks(Ctx &C, GridArgs &g, const uint8_t *mask, int nf1, int nf2
 // workgroups share them; a block of k_grid_sparse takes its points on one wave for
 // every window of 16 planes, 0.14 us a point (complex64 0.08).  cost is about what a
 // point of a tile takes in k_grid, in units of that, by its taps inside the tile
-// (above kw 9 its registers spill, above kCrowdKW it is never the faster); the
-// windows run side by side, but a point reaches only some of them and its taps meet
+// (above kw 9 its registers spill; complex64 above kw 5 and complex128 above
+// kCrowdKW stay on k_grid_sparse, mostly the faster there); the windows run side by side, but a point reaches only some of them and its taps meet
 // fewer others' the more planes there are, hence the power.  ms per call on 512^2
 // cells, 200000 rows, k_grid_sparse alone and k_grid, the points within 1 / within
 // about 8 cells (tiles of 8; kw: windows 1, 4, 16):
@@ -425,6 +425,7 @@ static int grid_masks(Ctx &C, GridArgs &g, const uint8_t *mask, int nf1, int nf2
 //              kw 8: 27.2, 23.8 / 7.4, 8.9
 //   complex64  kw 3: 4 windows 5.8, 2.8 / 1.4, 0.8   16 windows 3.2, 1.5 / 1.4, 1.0
 //              kw 5: 4 windows 7.0, 7.3 / 1.8, 2.4
+//              kw 7: 50 x 1500 cells, 11 windows, tiles of 2 x 4 20.6, 44
 // and with the cluster at the middle of a tile instead of a corner (600^2 cells),
 // complex128, 1 window: kw 6 27.0, 23.4, kw 7 26.8, 39.6 (within 1 cell).  1250^2
 // cells, tiles of 2, kw 8, 10^6 rows within 5 / 20 / 60: 74, 23 / 8.0, 5.1 / 3.3, 3.5.
@@ -437,13 +438,25 @@ static int crowd_min(const WPlan &P, const GridArgs &g, int planes)
     const int taps = std::min(kw, g.tx) * std::min(kw, g.ty) * kw;
     const bool dbl = sizeof(T) == 8;
     const double cost = (dbl ? 0.29 + 0.0020 * taps : 0.284 + 0.0037 * taps) * (kw > 9 ? 1.5 : 1.0);
+    if (!dbl && kw > 5) return 0;
     if (cost >= std::pow((double)windows, dbl ? -0.30 : -0.23)) return 0;
     const double share = windows == 1 ? 1.0 : (kw + 15) / (16.0 * windows) + 0.06;
     // the chain the other blocks do not hide: short on a GPU full of blocks.  90 x 54
     // cells, kw 7, 240 points a block: 0.375 ms the call, crowded from 128 points on 0.24
     const int64_t rows = P.band_len > 0 ? P.band_len : P.nf2, cols = P.cband_len > 0 ? P.cband_len : P.nf1;
     const bool few = rows * cols * windows <= 64 * 1024;
-    const int least = (int)((few ? (kw > 7 ? 512 : 128) : 256 << (kw > 7 ? kw - 4 : std::max(0, kw - 5))) / share);
+    int least = (int)((few ? (kw > 7 ? 512 : 128) : 256 << (kw > 7 ? kw - 4 : std::max(0, kw - 5))) / share);
+    // Where k_grid is the slower one on a full GPU (about 2 cost, for every tile
+    // against every block a footprint reaches), only regions whose chain is longer
+    // than all chains over the waves that run at once.  512^2 pixels, 8.2e6 uniform
+    // complex128 rows, 2000 a region: kw 5 3.4 ms the call, with k_grid 3.7, kw 6
+    // 3.8, 5.6, kw 7 4.3, 8.4; kw 4 3.0, 2.4.
+    const double blocks = (kBlk + kw - 1.0) * (kBlk + kw - 1.0) / (kBlk * kBlk);
+    const double ntile = (g.tx + kw - 1.0) * (g.ty + kw - 1.0) / (g.tx * g.ty);
+    if (2 * cost * ntile > blocks * (windows == 1 ? 1.0 : (kw + 15) / 16.0)) {
+        const double waves = std::clamp(rows * cols * windows * 0.35 / (kBlk * kBlk), 400.0, 800.0);
+        least = std::max(least, (int)(g.m * blocks / waves));
+    }
     // (the dense path's bins do not count)
     return g.m < least || (g.dense_min > 0 && g.dense_min <= least) ? 0 : least;
 }

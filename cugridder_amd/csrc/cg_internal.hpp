@@ -193,6 +193,8 @@ struct GridArgs {
 constexpr int kMaxBins = 81;
 // widest kernel of launch_grid's W-stacking form
 constexpr int kCrowdKW = 11;
+
+constexpr int kBlk = 8;  // edge (cells) of the blocks of k_grid_sparse
 // planes held by the grid buffer
 __host__ __device__ inline int slab_planes(const GridArgs &g) { return g.zn > 0 ? g.zn : g.nf3; }
 bool grid2d_mfma_supported(const GridArgs &g, int kw);

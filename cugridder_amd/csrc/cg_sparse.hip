@@ -30,7 +30,6 @@
 
 namespace cg {
 
-constexpr int kBlk = 8;      // block edge (cells)
 constexpr int kWin = 16;     // planes per window
 constexpr int kSpWaves = 4;  // independent waves per workgroup
 // bins that reach a block: along an axis at most ceil((kBlk + kw - 2) / tile)
