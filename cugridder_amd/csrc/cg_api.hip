@@ -988,12 +988,15 @@ static int plan_dirty2ms(Ctx &C, CallPlan &cp, int64_t nrow, int nchan, const do
 // planes instead of staged in LDS: twice the mean count per tile the points reach
 // from which staging is the faster one, or 1 when the mean is above that (the few
 // sparse tiles at the rim are then not worth a launch: 131072 Gaussian points, 360
-// per tile: 365 against 360 us).  Staging reads a tile's whole halo, so that the
-// mean falls with the tile: with uniform points the calls are even at 57 (kw 6),
-// 65 (8), 60 (9), 48 (10) and 62 (11) points per tile of 4 x 4 cells, 115 at kw 12,
-// whose staged form spills; at 30 (9), 60 (11, 12) and 115 (13) of 2 x 2; at 108 (6),
-// 80 (9) and 108 (10) of 8 x 8.  Tiles of 16 x 16: 120 per tile 2.86 against 3.49 ms
-// per complex64 call (1024^2, eps 1e-5), 488 per tile 3.47 against 2.68 ms;
+// per tile: 365 against 360 us).  Staging reads a tile's whole halo in every plane,
+// a point only kw planes, so that the mean falls with the tile and grows with the
+// planes.  With uniform complex128 points the calls are even at about 56 points per
+// tile of 2 x 2 cells (kw 6 and 9, 24 planes) and 110 (60 planes); of 4 x 4 at 100
+// (kw 6, 24 planes), 80 (kw 9), 145 (kw 9, 60 planes); of 8 x 8 at 108 (kw 6, 12
+// planes), 80 (kw 9, 18); twice that from kw 12 on, whose staged form spills.  2 x 2,
+// kw 9, 60 points per tile, staged / not: 24 planes 0.77 / 0.80 ms the call, 60 planes
+// 1.32 / 0.87, 300 planes 4.5 / 1.6.  Tiles of 16 x 16: 120 per tile 2.86 against
+// 3.49 ms per complex64 call (1024^2, eps 1e-5), 488 per tile 3.47 against 2.68 ms;
 // complex128 at eps 1e-12 with 15 per tile 50 against 165 ms, no difference at 256
 // to 512.
 static int degrid_direct_below(const WPlan &P, const Tiling &t, int64_t M)
@@ -1003,8 +1006,9 @@ static int degrid_direct_below(const WPlan &P, const Tiling &t, int64_t M)
     const int64_t tiles = ceil_div(rows, t.ty) * ceil_div(cols, t.tx);
     const int kw = P.conv.kw;
     const double edge = std::sqrt((double)t.tx * t.ty);
-    const int staged_from =
-        (int)std::min(128.0, (16.0 + 8.0 * edge) * 8.0 / std::min(kw, 8) * (1 << std::max(0, kw - 11)));
+    const double planes = std::pow(std::max(1.0, P.nf3 / (2.0 * kw + 2)), 0.9);
+    const int staged_from = (int)std::min(
+        128.0, (16 + 8 * edge) * 8 / std::clamp(kw, 6, 8) * (1 << std::max(0, kw - 11)) * planes);
     return M < tiles * staged_from ? 2 * staged_from : 1;
 }
 

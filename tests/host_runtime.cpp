@@ -424,21 +424,24 @@ void degrid_rule(const Lib &L)
     (void)take(&uvw, (size_t)24 * most, false);
     (void)take(&vis, (size_t)16 * most, false);
     (void)take(&img, (size_t)16 * 64 * 64, false);
-    const double r[6] = {-10, 10, -108, 108, -108, 108};  // u and v reach the whole grid
-    std::memcpy(range6, r, sizeof r);
-    for (int tile : {2, 4, 8, 16})
-        for (int kw : {4, 6, 9, 11, 13})
-            for (int per : {10, 25, 40, 70, 90, 120, 130}) {
-                void *ctx = nullptr;
-                (void)create(&ctx, nullptr);
-                option(ctx, "tile_degrid", tile);
-                launches.clear();
-                const int ier = run(ctx, 1, per * (128 / tile) * (128 / tile), 64, 64, 5.0, 1e9, uvw, 1, vis,
-                                    nullptr, 1, img, std::pow(10.0, 1 - kw) * 1.01, 2.0, -1);
-                show(("tile" + std::to_string(tile) + "_kw" + std::to_string(kw) + "_" + std::to_string(per)).c_str(),
-                     ier ? -ier : launched("k_degrid_direct"));
-                L.sym<int (*)(void *)>("cg_ctx_destroy")(ctx);
-            }
+    auto call = [&](int tile, int kw, double w, int per) {
+        const double r[6] = {-w, w, -108, 108, -108, 108};  // u and v reach the whole grid
+        std::memcpy(range6, r, sizeof r);
+        void *ctx = nullptr;
+        (void)create(&ctx, nullptr);
+        option(ctx, "tile_degrid", tile);
+        launches.clear();
+        const int ier = run(ctx, 1, per * (128 / tile) * (128 / tile), 64, 64, 5.0, 1e9, uvw, 1, vis, nullptr, 1,
+                            img, std::pow(10.0, 1 - kw) * 1.01, 2.0, -1);
+        show(("tile" + std::to_string(tile) + "_kw" + std::to_string(kw) + "_w" + std::to_string((int)w) + "_" +
+              std::to_string(per)).c_str(), ier ? -ier : launched("k_degrid_direct"));
+        L.sym<int (*)(void *)>("cg_ctx_destroy")(ctx);
+    };
+    // the fewest planes, about 30 and about 110
+    for (double w : {10., 620., 4000.})
+        for (int tile : {2, 4, 8, 16})
+            for (int kw : {4, 6, 9, 13})
+                for (int per : {10, 25, 40, 70, 90, 120, 130}) call(tile, kw, w, per);
 }
 
 // the column steps of complex128 transforms: steps on the prefetching kernel

@@ -123,16 +123,20 @@ def test_crowded_rule(scenario):
 def test_degrid_rule(scenario):
     """Tiles are read straight from the planes up to the mean number of points per
     tile from which staging them is the faster: fewer the smaller the tile and the
-    wider the kernel, as the halo read for them grows, and more from width 12 on,
-    where the staged kernel spills."""
+    wider the kernel, as the halo read for them grows; more the more planes there
+    are, which staging reads whole; more from width 12 on, where the staged kernel
+    spills."""
     r = scenario("degrid_rule")
-    until = {(2, 4): 40, (2, 6): 40, (2, 9): 25, (2, 11): 25, (2, 13): 120,
-             (4, 4): 90, (4, 6): 40, (4, 9): 40, (4, 11): 40, (4, 13): 120,
-             (8, 4): 120, (8, 6): 90, (8, 9): 70, (8, 11): 70, (8, 13): 120,
-             (16, 4): 120, (16, 6): 120, (16, 9): 120, (16, 11): 120, (16, 13): 120}
-    for (tile, kw), most in until.items():
-        for per in (10, 25, 40, 70, 90, 120, 130):
-            assert r[f"tile{tile}_kw{kw}_{per}"] == (per <= most), (tile, kw, per)
+    until = {(2, 4, 10): 40, (2, 6, 10): 40, (2, 9, 10): 25, (4, 4, 10): 40, (4, 6, 10): 40, (4, 9, 10): 40,
+             (8, 4, 10): 90, (8, 6, 10): 90, (8, 9, 10): 70,
+             (2, 4, 620): 70, (2, 6, 620): 40, (2, 9, 620): 25, (4, 4, 620): 90, (4, 6, 620): 90,
+             (4, 9, 620): 40, (8, 9, 620): 90}
+    for w in (10, 620, 4000):
+        for tile in (2, 4, 8, 16):
+            for kw in (4, 6, 9, 13):
+                for per in (10, 25, 40, 70, 90, 120, 130):
+                    most = until.get((tile, kw, w), 120)
+                    assert r[f"tile{tile}_kw{kw}_w{w}_{per}"] == (per <= most), (tile, kw, w, per)
 
 
 def test_column_rule(scenario):
