@@ -10,6 +10,7 @@
 // nor written.
 #include <algorithm>
 #include <mutex>
+#include <new>
 #include <unordered_map>
 
 #include "cg_fft.hpp"
@@ -109,16 +110,21 @@ MixPlan search_plan(int n, int nb, int ept, int rmax)
     return P;
 }
 
-// plans are searched once per length
-const MixPlan &cached_plan(int n, int nb, int ept, int rmax)
+// plans are searched once per length; without memory to keep one, on every call
+MixPlan cached_plan(int n, int nb, int ept, int rmax)
 {
     static std::mutex m;
     static std::unordered_map<uint64_t, MixPlan> plans;
     const uint64_t key = ((uint64_t)n << 32) | ((uint64_t)nb << 16) | ((uint64_t)ept << 8) | rmax;
     std::lock_guard<std::mutex> lock(m);
     auto it = plans.find(key);
-    if (it == plans.end()) it = plans.emplace(key, search_plan(n, nb, ept, rmax)).first;
-    return it->second;  // references into an unordered_map stay valid
+    if (it != plans.end()) return it->second;
+    const MixPlan P = search_plan(n, nb, ept, rmax);
+    try {
+        plans.emplace(key, P);
+    } catch (const std::bad_alloc &) {
+    }
+    return P;
 }
 
 // rows per workgroup: short rows are transformed together, about 4096
@@ -126,7 +132,7 @@ const MixPlan &cached_plan(int n, int nb, int ept, int rmax)
 int rows_per_group(int n) { return std::min(32, std::max(1, 4096 / n)); }
 
 template <typename T>
-const MixPlan &row_plan(int n)
+MixPlan row_plan(int n)
 {
     return cached_plan(n, rows_per_group(n), sizeof(T) == 4 ? kRowEpt32 : kRowEpt64, mix_max_radix<T>());
 }
@@ -449,7 +455,7 @@ bool fft_rows_mix_supported(int n)
 {
     if (n == 1) return true;
     if (n < 1 || n > 16384) return false;
-    const MixPlan &P = row_plan<T>(n);
+    const MixPlan P = row_plan<T>(n);
     return P.ns > 0 && row_lds<T>(P) <= 163840;
 }
 
@@ -468,7 +474,7 @@ int launch_fft_rows_mix(cx_t<T> *data, int64_t nrows, int n, int dir, const cx_t
 {
     if (n <= 1 || nrows <= 0) return CG_OK;
     if (!fft_rows_mix_supported<T>(n)) return CG_ERR_SIZE;
-    const MixPlan &P = row_plan<T>(n);
+    const MixPlan P = row_plan<T>(n);
     const size_t lds = row_lds<T>(P);
     const void *fn = dir > 0 ? (const void *)k_fft_rows_mix<T, 1> : (const void *)k_fft_rows_mix<T, -1>;
     if (lds > 65536)
@@ -507,10 +513,10 @@ int launch_fft_cols_mix(cx_t<T> *data, int batch, int n2, int n1, int L, int dir
     int sh = 6;
     while (sh > 3 && ((int64_t)L * elem << sh) > 81920) sh--;
     while (sh > 3 && (1 << (sh - 1)) >= nlive) sh--;
-    const MixPlan *P = nullptr;
+    MixPlan P;
     for (;; sh--) {
-        P = &cached_plan(L, 1 << sh, kColEpt, mix_max_radix<T>());
-        if (P->ns > 0) break;
+        P = cached_plan(L, 1 << sh, kColEpt, mix_max_radix<T>());
+        if (P.ns > 0) break;
         if (sh == 0) return CG_ERR_SIZE;
     }
     const size_t lds = ((size_t)L << sh) * elem;
@@ -519,9 +525,9 @@ int launch_fft_cols_mix(cx_t<T> *data, int batch, int n2, int n1, int L, int dir
             CG_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)lds));
         const int64_t ntile = (int64_t)((nlive + (1 << sh) - 1) >> sh) * nsub * batch;
-        const int per_cu = std::max(1, std::min((int)(163840 / lds), 2048 / P->threads));
+        const int per_cu = std::max(1, std::min((int)(163840 / lds), 2048 / P.threads));
         const unsigned grid = (unsigned)std::min<int64_t>(ntile, (int64_t)256 * 4 * per_cu);
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(P->threads), lds, s, data, n2, n1, *P, sh, se, sj, nsub,
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(P.threads), lds, s, data, n2, n1, P, sh, se, sj, nsub,
                            batch, twmode, tw2, live, rowmask, rowmask || mode_in != 1 ? mode_in : 0,
                            rowmask || mode_out != 1 ? mode_out : 0, spec_a, spec_b);
         CG_HIP(hipGetLastError());

@@ -41,7 +41,12 @@ int bad_frees = 0, bad_copies = 0, allocs = 0;
 // hipMalloc of exactly this size fails fail_times times
 size_t fail_size = 0;
 int fail_times = 0;
-bool fail_new = false;  // operator new throws
+bool fail_new = false;  // operator new throws, but for what this program itself needs
+struct OwnMemory {
+    bool was = fail_new;
+    OwnMemory() { fail_new = false; }
+    ~OwnMemory() { fail_new = was; }
+};
 double range6[6];       // w, u and v: least and largest
 
 // p lies in a live allocation with `bytes` to go
@@ -56,6 +61,7 @@ bool holds(const void *p, size_t bytes)
 hipError_t take(void **p, size_t bytes, bool host)
 {
     std::lock_guard<std::mutex> lock(mtx);
+    OwnMemory own;
     if (!host) {
         if (bytes == fail_size && fail_times > 0) {
             fail_times--;
@@ -155,6 +161,7 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t 
 }
 hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t)
 {
+    OwnMemory own;
     launches.push_back(kernels[f]);
     return hipSuccess;
 }
@@ -516,6 +523,27 @@ void release_without_heap(const Lib &L)
     show("allocations_left", (long long)live.size());
 }
 
+// transforms of lengths seen for the first time, without host memory to keep
+// their plans, then with it
+void plans_without_heap(const Lib &L)
+{
+    void *ctx = nullptr, *data = nullptr;
+    L.sym<int (*)(void **, void *)>("cg_ctx_create")(&ctx, nullptr);
+    (void)take(&data, (size_t)16 * 1000 * 900, false);
+    const auto fft = L.sym<int (*)(void *, int, void *, int, int, int, int)>("cg_fft2d_dev");
+    for (const bool none : {true, false})
+        for (int prec : {0, 1}) {
+            launches.clear();
+            fail_new = none;
+            const int ier = fft(ctx, prec, data, 1, 900, 1000, 1);
+            fail_new = false;
+            const std::string name = std::string(none ? "none" : "some") + std::to_string(prec);
+            show((name + "_ier").c_str(), ier);
+            show((name + "_rows").c_str(), launched("k_fft_rows_mix"));
+            show((name + "_cols").c_str(), launched("k_fft_cols_mix"));
+        }
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -535,6 +563,7 @@ int main(int argc, char **argv)
     else if (what == "tile_edges") tile_edges(L);
     else if (what == "crowded_rule") crowded_rule(L);
     else if (what == "degrid_rule") degrid_rule(L);
+    else if (what == "plans_without_heap") plans_without_heap(L);
     else if (what == "column_rule") column_rule(L);
     else if (what == "surplus") surplus(L);
     else return 2;

@@ -148,3 +148,13 @@ def test_column_rule(scenario):
     assert r["p1_16x8192x2048"] == 1  # of its steps of 64 and 128 points
     for name in ("p1_16x2048x2048", "p1_17x4096x2048", "p1_1x1000x1024", "p0_1x1024x1024"):
         assert r[name] == 0, name
+
+
+def test_plans_without_heap(scenario):
+    """A transform whose plan cannot be kept runs all the same: no exception
+    leaves a C entry."""
+    r = scenario("plans_without_heap")
+    for prec in (0, 1):
+        assert r[f"none{prec}_ier"] == 0
+        for what in ("rows", "cols"):
+            assert r[f"none{prec}_{what}"] == r[f"some{prec}_{what}"] > 0
