@@ -397,10 +397,17 @@ static int grid_masks(Ctx &C, GridArgs &g, const uint8_t *mask, int nf1, int nf2
         // W-stacking grids are gridded in 8 x 8 blocks, 2-D ones in sort tiles
         const int64_t n = g.nf3 > 1 ? sparse_blocks(nf1, nf2) : (int64_t)g.ntx * g.nty;
         if (n < kListedTiles) return CG_OK;
-        // 2-D grids of other sides keep the tiles' order: with every tile reached
-        // a list costs more than it saves (5400 x 5000 cells, 3.9e6 uniform
-        // points: 2.14 ms the call, listed 2.81)
-        if (g.nf3 == 1 && ((nf1 & (nf1 - 1)) || (nf2 & (nf2 - 1)))) return CG_OK;
+        // A list loses the tiles' order.  2-D tiles whose rows are shorter than a
+        // cache line (128 bytes) then write parts of lines: 5400^2 cells, complex64,
+        // tiles of 8, 30000 / 10^6 uniform points 1.04 / 1.89 ms whole, 1.28 / 2.48
+        // listed.  Wider ones pay up to a tenth where every tile is reached (3000^2,
+        // complex128, tiles of 8, 4e6 uniform points 1.55, 1.69) and gain where many
+        // are not (5400^2, 30000 points in four clusters 1.20, 0.49); complex64
+        // gains as much in clusters as it pays (6000^2, tiles of 16, 30000 points 0.66,
+        // 0.62; uniform 0.55, 0.59).  Tiles of 32 pay up to 5 % (8192^2, 10^6 uniform
+        // points complex64 0.78, 0.80; in clusters 0.78, 0.70).
+        const bool wide = sizeof(T) == 8 && g.tx >= 8;
+        if (g.nf3 == 1 && !(g.tx >= 32 || (wide && g.m <= 2 * n))) return CG_OK;
         CG_TRY(ensure(C.tlist, sizeof(int32_t) * (size_t)(n + 1)));
         g.rowmask = mask;
         g.colmask = mask + nf2;

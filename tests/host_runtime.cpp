@@ -523,6 +523,28 @@ void release_without_heap(const Lib &L)
     show("allocations_left", (long long)live.size());
 }
 
+// nufft2d1 calls by whether the gridder takes the tiles from a list
+void list_rule(const Lib &L)
+{
+    const auto create = L.sym<int (*)(void **, void *)>("cg_ctx_create");
+    const auto run = L.sym<int (*)(void *, int, int, int, const void *, const void *, void *, int, int, void *, double,
+                                   double)>("cg_nufft2d_dev");
+    void *x = nullptr, *f = nullptr;
+    (void)take(&x, (size_t)16 * 2000000, false);
+    (void)take(&f, (size_t)16 * 2700 * 2700, false);
+    for (int prec : {0, 1})
+        for (int n : {256, 1024, 1500, 2048, 2700})
+            for (int m : {30000, 1000000}) {
+                void *ctx = nullptr;
+                (void)create(&ctx, nullptr);
+                launches.clear();
+                const int ier = run(ctx, 1, prec, m, x, x, x, n, n, f, 1e-5, 2.0);
+                show(("p" + std::to_string(prec) + "_" + std::to_string(n) + "_" + std::to_string(m)).c_str(),
+                     ier ? -ier : launched("k_need_tiles"));
+                L.sym<int (*)(void *)>("cg_ctx_destroy")(ctx);
+            }
+}
+
 // transforms of lengths seen for the first time, without host memory to keep
 // their plans, then with it
 void plans_without_heap(const Lib &L)
@@ -563,6 +585,7 @@ int main(int argc, char **argv)
     else if (what == "tile_edges") tile_edges(L);
     else if (what == "crowded_rule") crowded_rule(L);
     else if (what == "degrid_rule") degrid_rule(L);
+    else if (what == "list_rule") list_rule(L);
     else if (what == "plans_without_heap") plans_without_heap(L);
     else if (what == "column_rule") column_rule(L);
     else if (what == "surplus") surplus(L);

@@ -158,3 +158,17 @@ def test_plans_without_heap(scenario):
         assert r[f"none{prec}_ier"] == 0
         for what in ("rows", "cols"):
             assert r[f"none{prec}_{what}"] == r[f"some{prec}_{what}"] > 0
+
+
+def test_list_rule(scenario):
+    """2-D gridding takes the tiles that are read from a list, which loses their
+    order, on tiles of 32 cells and, where few are reached, on tiles whose rows fill
+    cache lines: 3000^2 and 5400^2 cells have tiles of 8."""
+    r = scenario("list_rule")
+    for prec in (0, 1):
+        for m in (30000, 1000000):
+            assert r[f"p{prec}_256_{m}"] == 0        # 256 tiles
+            for n in (1024, 2048):
+                assert r[f"p{prec}_{n}_{m}"] == 1
+            for n in (1500, 2700):
+                assert r[f"p{prec}_{n}_{m}"] == (prec == 1 and m == 30000)
