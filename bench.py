@@ -257,15 +257,17 @@ def kernel_table(W, plan, fw, bw, stage_ms):
     Md = fw["dense_points"]
     Rm, Cm = fw["rows"], fw["cols"]
     sm, sb = stage_ms["ms2dirty"], stage_ms["dirty2ms"]
-    col_kernel = "k_fft_cols_step_r2" if (nf2 > 128 and nf2 & (nf2 - 1) == 0) else "k_fft_cols_step"
+    col_kernel = "k_fft_cols_step_r2" if (nf2 > 128 and nf2 & (nf2 - 1) == 0) else "k_fft_cols_mix"
+    row_kernel = "k_fft_rows_mix" if nf1 & (nf1 - 1) else "k_fft_rows_ct"
     cells_w = P * fw["tiles_written"] * fw["tile"]
     rows = []
-    # the sparse kernel writes every kept cell once; the dense kernel adds
-    # the dense bins' points onto those cells
-    rows.append(("k_grid", "ms2dirty", 1, sm["grid"] - sm["grid_dense"], 36 * (M - Md) + 8 * cells_w))
+    # the sparse kernel writes every kept cell once (with k_grid, which takes
+    # crowded regions where there is no dense path); the dense kernel adds the
+    # dense bins' points onto those cells
+    rows.append(("k_grid_sparse", "ms2dirty", 1, sm["grid"] - sm["grid_dense"], 36 * (M - Md) + 8 * cells_w))
     if Md:
         rows.append(("k_grid_dense", "ms2dirty", 1, sm["grid_dense"], 36 * Md))
-    rows.append(("k_fft_rows_ct", "ms2dirty", 1, sm["fft_rows"], 8 * P * Rm * (Cm + N1)))
+    rows.append((row_kernel, "ms2dirty", 1, sm["fft_rows"], 8 * P * Rm * (Cm + N1)))
     if band_kernel(nf2, fw["band"]):
         # one pass: the masked rows of the band in, the live spectrum out
         rows.append(("k_fft_cols_band", "ms2dirty", 1, sm["fft_cols"], 8 * P * Rm * N1 + 8 * P * N2 * N1))
@@ -281,8 +283,10 @@ def kernel_table(W, plan, fw, bw, stage_ms):
     else:
         rows.append((col_kernel, "dirty2ms", 2, sb["fft_cols"],
                      (8 * P * (N2 * N1 + nf2 * N1) + 8 * P * (nf2 * N1 + Rb * N1)) // 2))
-    rows.append(("k_fft_rows_ct", "dirty2ms", 1, sb["fft_rows"], 8 * P * Rb * (N1 + Cb)))
-    # the degridders read each point once and each cell of their tiles once
+    rows.append((row_kernel, "dirty2ms", 1, sb["fft_rows"], 8 * P * Rb * (N1 + Cb)))
+    # the degridders read each point once and each cell of their tiles once;
+    # the k_degrid row is the staged tiles and those k_degrid_direct reads
+    # straight from the planes
     Mb, Tb = bw["dense_points"], bw["dense_tiles"]
     rows.append(("k_degrid", "dirty2ms", 1, sb["grid"] - sb["grid_dense"],
                  36 * (M - Mb) + 8 * P * max(bw["tiles_written"] - Tb, 0) * bw["tile"]))
@@ -591,11 +595,11 @@ def main():
                 "launches_per_call": launches}
         if traffic:
             roof["traffic_GBs"] = round(traffic / (t_launch * 1e-3) / 1e9, 1)
-        if name in ("k_grid_dense", "k_grid", "k_degrid", "k_degrid_dense"):
+        if name in ("k_grid_dense", "k_grid_sparse", "k_degrid", "k_degrid_dense"):
             # useful arithmetic: kw^3 taps per point, a complex value times a
             # real kernel product (4 flop) per tap
             pts = {"k_grid_dense": fw_stats["dense_points"],
-                   "k_grid": W["M"] - fw_stats["dense_points"],
+                   "k_grid_sparse": W["M"] - fw_stats["dense_points"],
                    "k_degrid_dense": bw_stats["dense_points"],
                    "k_degrid": W["M"] - bw_stats["dense_points"]}[name]
             kw = plan["kw"]

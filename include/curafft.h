@@ -143,7 +143,8 @@ int dirty2ms_px(int prec, int nrow, int nchan, int nxdirty, int nydirty,
 int cg_ctx_create(void **ctx, void *stream);
 int cg_ctx_destroy(void *ctx);
 /* options: "timing" (0/1, per-stage HIP events), "lds_budget" (degridding
- * staging bytes), "grid_lds_budget" (gridding accumulator bytes),
+ * staging bytes), "grid_lds_budget" (LDS bytes of a gridding tile: one plane
+ * of a 2-D grid; W-stacking, as many planes as fit, for crowded regions),
  * "tile_grid", "tile_degrid" (preferred tile edge, power of two <= 32),
  * "tile_grid2d" (the same for 2-D NUFFT type 1, <= 64; default 32),
  * "tile_degrid2d" (the same for 2-D NUFFT type 2; default 32),
