@@ -103,3 +103,31 @@ def test_crowded_call_is_not_serial(gpu):
             best.append(time.perf_counter() - t0)
         ms.append(min(best) * 1e3)
     assert ms[0] < 12 * ms[1], ms
+
+
+def test_crowded_batch_replays(gpu):
+    """Channels with crowded regions captured as one graph (complex64, several windows
+    of planes, so no dense path): every replay gives the single call's image, with
+    eager calls between the replays."""
+    torch = gpu
+    from cugridder_amd import Context
+    ctx = Context()
+    items, ref = [], []
+    for nx, ny, n in ((64, 64, 20000), (30, 36, 6000)):
+        k = crowded_case(n, nx, ny, 40.0, 2000.0, (1, -2))
+        it = dict(uvw=torch.tensor(k["uvw"], device="cuda"),
+                  vis=torch.tensor(k["ms"], dtype=torch.complex64, device="cuda"),
+                  wgt=torch.tensor(k["wgt"], dtype=torch.float32, device="cuda"), fov=40.0, freq=k["f0"],
+                  dirty=torch.zeros(nx, ny, dtype=torch.complex64, device="cuda"))
+        items.append(it)
+        ref.append(ctx.ms2dirty(it["uvw"], it["vis"], it["wgt"], nx, ny, 40.0, k["f0"], 1e-2).cpu().numpy())
+        assert ctx.last_plan()["nf3"] > 32
+    batch = ctx.batch("ms2dirty", items, 1e-2, graph=True)
+    for _ in range(4):
+        for it in items:
+            it["dirty"].fill_(5.0)
+        batch.run()
+        torch.cuda.synchronize()
+        for it, r in zip(items, ref):
+            assert rel_l2(it["dirty"].cpu().numpy(), r) < 2e-6
+        ctx.ms2dirty(items[0]["uvw"], items[0]["vis"], None, 64, 64, 40.0, items[0]["freq"], 1e-2)
